@@ -336,9 +336,9 @@ int ukv_paged_prefill(const void* q, const void* k_cache, const void* v_cache, c
  * stats_seq_stride counts (value, flag) pairs and is at least num_q_heads * obs_len; obs_stats is
  * 8-byte aligned. For the layout ukv_snapkv_scores_from_stats reads ([seqs][layers][num_q_heads]
  * [obs_len] pairs) pass obs_stats + 2 * layer * num_q_heads * obs_len and stats_seq_stride =
- * layers * num_q_heads * obs_len. The rows come from the tiled kernel (head_dim 128, n_rep
- * 1/2/4/8/16, 16-byte aligned rows); on the scalar path every row is written flagged (0, 1), so the
- * scores recompute them. C_b >= obs_len for the rows to exist.
+ * layers * num_q_heads * obs_len. The rows come from the tiled kernel's fp16-weight instances
+ * (head_dim 128, n_rep 1/2/4/8/16, 16-byte aligned rows); elsewhere every row is written flagged
+ * (0, 1), so the scores recompute them. C_b >= obs_len for the rows to exist.
  * The reference captures the window's queries in its q_proj hook (core/scheduler.py:269-341)
  * and normalises their softmax over K_mid at selection time (core/scheduler.py:565-592,
  * core/compress.py:116-130); here that normaliser comes from the prefill's own softmax
@@ -355,6 +355,28 @@ int ukv_paged_prefill_obs_stats(const void* q, const void* k_cache, const void* 
                                 const int64_t* k_strides, const int64_t* v_strides, float softmax_scale, int dtype,
                                 int sink_len, int obs_len, float* obs_stats, int64_t stats_seq_stride,
                                 ukv_stream_t stream);
+
+/*
+ * Bytes of device scratch with which ukv_paged_prefill_parts cuts the keys of this shape into parts,
+ * or 0 where whole query blocks already fill the device (the call then needs no workspace).
+ */
+size_t ukv_paged_prefill_workspace_bytes(int batch, int total_q, int max_chunk, int num_q_heads, int num_kv_heads,
+                                         int head_dim, int n_rep, int max_blocks);
+
+/*
+ * ukv_paged_prefill (obs_stats NULL) or ukv_paged_prefill_obs_stats (otherwise), with the query
+ * blocks of a launch too small to fill the device also cut along the keys: the parts' partial
+ * results go through the workspace, ukv_paged_prefill_workspace_bytes() bytes aligned to 16. It
+ * needs no initialisation and may be reused once the stream has passed the call. With a NULL or
+ * smaller workspace the keys are not cut.
+ */
+int ukv_paged_prefill_parts(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
+                            const int32_t* cu_seqlens_q, const int32_t* kv_lens, void* out, int batch, int total_q,
+                            int max_chunk, int num_q_heads, int num_kv_heads, int head_dim, int n_rep,
+                            int max_blocks, int num_pages, const int64_t* q_strides, const int64_t* k_strides,
+                            const int64_t* v_strides, float softmax_scale, int dtype, int sink_len, int obs_len,
+                            float* obs_stats, int64_t stats_seq_stride, void* workspace, size_t workspace_bytes,
+                            ukv_stream_t stream);
 
 /*
  * SnapKV observation-window block scores (the importance scores ukv_select_topk ranks).

@@ -1,0 +1,141 @@
+"""Tiled prefill beyond head_dim 128 with n_rep a divisor of 16, and key parts (GPU).
+
+Head shapes whose q heads straddle the 16-column blocks, 64-dim heads, and launches small enough
+that a query block's keys are cut into parts and merged, against the fp64 closed form. Outputs are
+rounded to the pool's type once from fp32 sums of fp32-grade weights (two 16-bit parts, relative
+error at most 2^-16 in bf16 and 2^-21 in fp16), so a row is off by its own rounding (2^-9 / 2^-12 of
+each value) plus 2^-15 of the largest |V|: what FINE_TOL states. Shapes with fp16 weights (relative
+error 2^-12 each) get 2^-11 of the largest |V|.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from test_prefill import check, expected, make_case, run_gpu, to_dev
+from unifiedkv_amd import _ext, workloads
+
+ROUND = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}  # one unit in the last place, relative
+
+
+def _close(got, exp, v_max, dtype, weights, what):
+    bound = ROUND[dtype] * np.abs(exp) + weights * v_max
+    err = np.abs(got - exp)
+    assert np.isfinite(got).all() and (err <= bound).all(), f"{what}: worst excess {np.max(err - bound):.3e}"
+
+
+def _v_max(case):
+    f = lambda a: oracle.bits_to_f32(a, workloads.DTYPE_CODES[case["dtype"]])
+    return max(float(np.abs(f(case["v_cache"])).max()), float(np.abs(f(case["v_new"])).max()))
+
+
+def _parts_bytes(case):
+    Hq, Hkv, D = case["q"].shape[1], case["k_cache"].shape[2], case["q"].shape[2]
+    return int(_ext.load().ukv_paged_prefill_workspace_bytes(
+        len(case["kv_lens"]), len(case["q"]), max(case["chunk"]), Hq, Hkv, D, case["n_rep"],
+        case["block_table"].shape[1]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("n_rep,Hkv,D,prefix,chunk", [
+    (7, 2, 128, [0], [1]), (7, 4, 128, [45, 0, 200], [37, 16, 110]), (3, 2, 128, [31, 64], [85, 1]),
+    (5, 1, 128, [15], [52]), (6, 2, 128, [0], [43]), (9, 1, 128, [100], [29]), (20, 1, 128, [7], [13]),
+    (64, 1, 128, [33], [5]),
+    (4, 8, 64, [0, 0, 0], [16, 129, 97]), (1, 2, 64, [63], [385]), (7, 2, 64, [64, 5], [55, 64]), (16, 1, 64, [127], [25]),
+])
+def test_fine_instances_match_the_closed_form(cuda, n_rep, Hkv, D, prefix, chunk, dtype):
+    case = make_case(n_rep * 100 + D + sum(chunk), prefix, chunk, Hq=n_rep * Hkv, Hkv=Hkv, D=D, dtype=dtype)
+    out, _ = run_gpu(case, cuda)
+    _close(out.float().cpu().numpy(), expected(case), _v_max(case), dtype, 2.0 ** -15,
+           f"n_rep={n_rep} Hkv={Hkv} D={D} prefix={prefix} chunk={chunk} {dtype}")
+
+
+# Launches of few query blocks over many keys. (The second sequence of a batch is short: fewer parts.)
+PARTS = [(4, 2, 128, [1531], [37]), (4, 1, 128, [3000, 90], [70, 3]), (16, 1, 128, [2047], [1]),
+         (7, 2, 128, [1600], [41]), (5, 1, 128, [4001, 0], [33, 20]), (4, 2, 64, [3100], [64]), (7, 1, 64, [5000, 1], [9, 60])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("n_rep,Hkv,D,prefix,chunk", PARTS)
+def test_key_parts_match_the_closed_form(cuda, n_rep, Hkv, D, prefix, chunk, dtype):
+    case = make_case(n_rep * 10 + D + sum(prefix), prefix, chunk, Hq=n_rep * Hkv, Hkv=Hkv, D=D, dtype=dtype)
+    assert _parts_bytes(case) > 0  # the shape is cut into parts
+    out, _ = run_gpu(case, cuda)
+    fine = D != 128 or 16 % n_rep
+    _close(out.float().cpu().numpy(), expected(case), _v_max(case), dtype, 2.0 ** -15 if fine else 2.0 ** -11,
+           f"parts n_rep={n_rep} Hkv={Hkv} D={D} prefix={prefix} chunk={chunk} {dtype}")
+
+
+@pytest.mark.gpu
+def test_parts_with_an_invalid_page_and_a_last_group_short_of_heads(cuda):
+    """A masked page empties one part of the keys; 10 q heads in groups of 4 leave the last group two."""
+    import torch
+
+    from unifiedkv_amd import prefill
+
+    case = make_case(5, [1500], [30], Hq=10, Hkv=3, D=128, dtype="bf16")
+    bad = case["block_table"].copy()
+    bad[0, 20:44] = [-1, 1 << 20] * 12  # keys 320 .. 703: masked
+    t = to_dev(case, cuda)
+    prefill.write_chunk_kv(t["k_cache"], t["v_cache"], t["k_new"], t["v_new"], t["block_table"], t["cu"], t["kv_lens"], 30)
+    t["block_table"] = torch.from_numpy(bad).to(cuda)
+    out = prefill.paged_prefill_attention(t["q"], t["k_cache"], t["v_cache"], t["block_table"], t["cu"], t["kv_lens"],
+                                          softmax_scale=case["scale"], n_rep=4, max_chunk=30).float().cpu().numpy()
+    keep = [p for p in range(bad.shape[1]) if not 20 <= p < 44]  # the same keys without the masked pages
+    small = dict(case, block_table=case["block_table"][:, keep], kv_lens=case["kv_lens"] - 24 * 16, n_rep=4)
+    _close(out, expected(small), _v_max(case), "bf16", 2.0 ** -11, "masked pages")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_rep,Hkv,D,dtype,big", [(4, 2, 128, "bf16", 3.0e38), (7, 2, 128, "bf16", np.inf),
+                                                   (7, 2, 128, "bf16", 3.0e38), (7, 1, 64, "fp16", np.inf)])
+@pytest.mark.parametrize("prefix,chunk", [([200], [30]), ([4000], [12])])
+def test_wide_and_infinite_v(cuda, n_rep, Hkv, D, dtype, big, prefix, chunk):
+    """Values the 16-bit P.V cannot carry take the fp32 fallback, in whole blocks and in parts; an
+    infinite V gives an infinite output in its dimension and leaves the others alone."""
+    case = make_case(9, prefix, chunk, Hq=n_rep * Hkv, Hkv=Hkv, D=D, dtype=dtype)
+    case["v_cache"][case["block_table"][0][6], 5, 0, 7] = workloads._round_bits(np.array([big], np.float32), dtype)[0]
+    with np.errstate(invalid="ignore"):
+        exp = expected(case)
+    out, _ = run_gpu(case, cuda)
+    got = out.float().cpu().numpy()
+    fin = np.isfinite(exp)
+    np.testing.assert_array_equal(np.isfinite(got), fin)
+    np.testing.assert_array_equal(got[~fin], exp[~fin].astype(np.float32))
+    check(np.where(fin, got, 0.0), np.where(fin, exp, 0.0), f"n_rep={n_rep} D={D} |v|={big}")
+
+
+@pytest.mark.gpu
+def test_parts_replay_from_a_captured_graph(cuda):
+    import torch
+
+    from unifiedkv_amd import prefill
+
+    case = make_case(3, [1700], [40], Hq=14, Hkv=2, D=128, dtype="fp16")
+    t = to_dev(case, cuda)
+    args = (t["q"], t["k_cache"], t["v_cache"], t["block_table"], t["cu"], t["kv_lens"])
+    kw = dict(softmax_scale=case["scale"], n_rep=7, max_chunk=40)
+    want = prefill.paged_prefill_attention(*args, **kw)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        prefill.paged_prefill_attention(*args, **kw)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = prefill.paged_prefill_attention(*args, **kw)
+    for _ in range(3):
+        got.fill_(0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        prefill.paged_prefill_attention(*args, **kw)
+
+
+def test_parts_are_taken_only_by_launches_short_of_blocks():
+    """The plan on the CPU (no device: 256 CUs are not known, so nothing is cut)."""
+    lib = _ext.load()
+    assert lib.ukv_paged_prefill_workspace_bytes(0, 1, 1, 8, 2, 128, 4, 100) == 0
+    assert lib.ukv_paged_prefill_workspace_bytes(1, 64, 64, 8, 2, 96, 4, 1000) == 0  # no tiled instance
+    assert lib.ukv_paged_prefill_workspace_bytes(64, 64 * 2048, 2048, 32, 8, 128, 4, 1000) == 0

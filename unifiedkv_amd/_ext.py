@@ -162,6 +162,19 @@ SIGNATURES = {
             _c_int, _c_int, _c_void_p, ctypes.c_int64, _c_void_p,  # sink obs stats stats_seq_stride stream
         ],
     ),
+    "ukv_paged_prefill_workspace_bytes": (
+        ctypes.c_size_t, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),
+    "ukv_paged_prefill_parts": (
+        _c_int,
+        [
+            _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,  # q k v bt cu kv_lens out
+            _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,  # batch total_q max_chunk Hq Hkv D n_rep
+            _c_int, _c_int, _c_i64p, _c_i64p, _c_i64p,  # max_blocks num_pages strides
+            ctypes.c_float, _c_int,  # scale dtype
+            _c_int, _c_int, _c_void_p, ctypes.c_int64,  # sink obs stats (nullable) stats_seq_stride
+            _c_void_p, ctypes.c_size_t, _c_void_p,  # workspace, bytes, stream
+        ],
+    ),
     "ukv_snapkv_block_count": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
     "ukv_snapkv_workspace_bytes": (
         ctypes.c_size_t, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),

@@ -41,6 +41,14 @@
 //     operands come from ds_read_b64_tr_b16 transpose reads; the softmax
 //     denominators come from one more MFMA against a ones operand, so they sum
 //     exactly the rounded P;
+//   * shapes whose n_rep does not divide 16, and 64-dim heads, run FINE instances: columns are
+//     (query, head) pairs laid end to end, so every column of the matrix cores is used, V keeps its
+//     type and P goes in as two 16-bit parts (fp32-grade weights, as the scalar kernel they ran on
+//     before had): 28 q heads on 4 KV heads, 4 x 512 queries over 0.5-8K keys in 0.33 ms against
+//     72.7 ms; twelve 64-dim prompts of 16-700 tokens in 0.10 ms against 6.4 ms;
+//   * key parts: a launch of few query blocks leaves CUs idle however long its prefix. Its keys are
+//     then cut into equal parts, each (block, part) a workgroup, and a merge kernel adds the parts
+//     up: one 389-query chunk behind 32256 keys (40 blocks) in 0.23 ms against 0.86 ms;
 //   * SnapKV row statistics: the blocks holding each sequence's last obs queries
 //     also write those rows' running max and denominator; obs_rows_finish_kernel
 //     then sums the sink and window keys' weights again from the same scores and
@@ -77,6 +85,14 @@ struct PrefillArgs {
   // partial or empty (chunks shorter than the longest). The three-column blocks of every pair are
   // dispatched in a first pass, the two-column ones in a second.
   int n3, n2;
+  // Key split (n_parts > 1): the key tiles of a sequence are cut into part_count() <= n_parts equal
+  // parts of about part_tiles tiles, each (query block, part) is a work item of its own, and
+  // prefill_combine_kernel merges the parts' (m, l, O) from part_o / part_ml, rows
+  // [part][query row][q head] of D floats / one float2.
+  int n_parts, part_tiles;
+  int total_q;
+  float* part_o;
+  float2* part_ml;
   // The longest chunk the caller declared: the block plan covers that many queries. A chunk
   // longer than it gets NaN in every row of its output (its K/V were not all written either).
   int max_chunk;
@@ -145,43 +161,67 @@ constexpr int kRowPad = UKV_PREFILL_KPAD;
 constexpr int kVRowPad = UKV_PREFILL_VPAD;
 constexpr int kStages = 4;  // K/V ring slots: tiles are written two ahead, a barrier every second tile
 
-// Fallback for a workgroup whose key range holds a bf16 V value of magnitude
-// >= 65520 (or infinite), which fp16 cannot carry: every (query, head) pair
-// of the workgroup is recomputed in fp32 on the vector ALUs, one pair per
-// wave at a time, keys in page order (the reference's order), natural exp.
-// D = 128: lane l owns dims 2l and 2l + 1.
-template <int DT>
-__device__ void prefill_pairs_fp32(const PrefillArgs& a, int b, int g, int q_begin, int C, int P0, int Lk, int qa,
-                                   int qe, int wv, int nwaves, int lane) {
+// Parts the n_tiles key tiles of a sequence are cut into; part s holds tiles
+// [s * n_tiles / n, (s + 1) * n_tiles / n).
+__device__ __forceinline__ int part_count(const PrefillArgs& a, int n_tiles) {
+  return max(1, min(a.n_parts, (n_tiles + a.part_tiles - 1) / a.part_tiles));
+}
+
+// Fallback for a workgroup whose keys hold a V the matrix cores' P.V would get wrong (a bf16 V of
+// magnitude >= 65520, or infinite, which fp16 cannot carry; FINE: an infinite one, which a zero low
+// part turns into NaN, or one near the type's end): every column of the workgroup, c0 .. c0 + n_cols - 1,
+// is recomputed in fp32 on the vector ALUs, one column per wave at a time, keys in page order (the
+// reference's order), natural exp. Lane l owns dims l * D / 64 ... Keys [key_a, key_b) are taken; with
+// part >= 0 the column's partial is left for prefill_combine_kernel, its denominator's sign bit set:
+// the rows' statistics are then flagged.
+template <int DT, int D>
+__device__ void prefill_cols_fp32(const PrefillArgs& a, int b, int g, int q_begin, int C, int P0, int Lk, int c0,
+                                  int n_cols, int wv, int nwaves, int lane, int part, int key_a, int key_b) {
+  constexpr int W = D / 64;  // dims per lane
   const int32_t* btrow = a.bt + (int64_t)b * a.max_blocks;
-  const int npairs = (qe - qa) * a.n_rep;
-  for (int pi = wv; pi < npairs; pi += nwaves) {
-    const int qi = qa + pi / a.n_rep;
-    const int h = g * a.n_rep + pi % a.n_rep;
+  for (int c = c0 + wv; c < c0 + n_cols; c += nwaves) {
+    if (c < 0) continue;
+    const int qi = c / a.n_rep;
+    const int h = g * a.n_rep + c % a.n_rep;
     if (qi >= C || h >= a.Hq) continue;
-    const int L = max(0, min(Lk, P0 + qi + 1));
-    const uint16_t* qrow = a.q + (int64_t)(q_begin + qi) * a.q_st + (int64_t)h * a.q_sh + 2 * lane;
-    const float q0 = Elem<DT>::one(qrow[0]), q1 = Elem<DT>::one(qrow[1]);
-    float m = kNegFltMax, l = 0.f, acc0 = 0.f, acc1 = 0.f;
-    for (int key = 0; key < L; ++key) {
+    const int L = min(key_b, max(0, min(Lk, P0 + qi + 1)));
+    const uint16_t* qrow = a.q + (int64_t)(q_begin + qi) * a.q_st + (int64_t)h * a.q_sh + W * lane;
+    float q[W], acc[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      q[w] = Elem<DT>::one(qrow[w]);
+      acc[w] = 0.f;
+    }
+    float m = kNegFltMax, l = 0.f;
+    for (int key = key_a; key < L; ++key) {
       const int id = btrow[key >> 4];
       if ((unsigned)id >= (unsigned)a.num_pages) continue;
-      const uint16_t* kr = a.k + (int64_t)id * a.k_sp + (int64_t)(key & 15) * a.k_st + (int64_t)g * a.k_sh + 2 * lane;
-      const uint16_t* vr = a.v + (int64_t)id * a.v_sp + (int64_t)(key & 15) * a.v_st + (int64_t)g * a.v_sh + 2 * lane;
-      float part = q0 * Elem<DT>::one(kr[0]) + q1 * Elem<DT>::one(kr[1]);
+      const int64_t slot = key & 15;
+      const uint16_t* kr = a.k + (int64_t)id * a.k_sp + slot * a.k_st + (int64_t)g * a.k_sh + W * lane;
+      const uint16_t* vr = a.v + (int64_t)id * a.v_sp + slot * a.v_st + (int64_t)g * a.v_sh + W * lane;
+      float dot = 0.f;
 #pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off);
-      const float sc = part * a.scale;
+      for (int w = 0; w < W; ++w) dot += q[w] * Elem<DT>::one(kr[w]);
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
+      const float sc = dot * a.scale;
       const float mn = fmaxf(m, sc);
       const float alpha = expf(m - mn), pk = expf(sc - mn);
       l = l * alpha + pk;
-      acc0 = acc0 * alpha + pk * Elem<DT>::one(vr[0]);
-      acc1 = acc1 * alpha + pk * Elem<DT>::one(vr[1]);
+#pragma unroll
+      for (int w = 0; w < W; ++w) acc[w] = acc[w] * alpha + pk * Elem<DT>::one(vr[w]);
       m = mn;
     }
-    uint16_t* orow = a.out + ((int64_t)(q_begin + qi) * a.Hq + h) * 128 + 2 * lane;
-    orow[0] = Elem<DT>::from_float(acc0 / l);
-    orow[1] = Elem<DT>::from_float(acc1 / l);
+    if (part >= 0) {
+      const int64_t row = ((int64_t)part * a.total_q + q_begin + qi) * a.Hq + h;
+#pragma unroll
+      for (int w = 0; w < W; ++w) a.part_o[row * D + W * lane + w] = acc[w];
+      if (lane == 0) a.part_ml[row] = make_float2(m * kLog2e, -l);
+      continue;
+    }
+    uint16_t* orow = a.out + ((int64_t)(q_begin + qi) * a.Hq + h) * D + W * lane;
+#pragma unroll
+    for (int w = 0; w < W; ++w) orow[w] = Elem<DT>::from_float(acc[w] / l);
   }
 }
 
@@ -198,30 +238,68 @@ __device__ void flag_obs_rows(const PrefillArgs& a, int b, int g, int C, int lo,
   }
 }
 
-// LDS of one workgroup: kStages ring slots of K and V (fp16) tiles.
-struct PrefillLds {
-  __attribute__((aligned(16))) uint16_t k_s[kStages][kTileKeys][kRowPad];
-  __attribute__((aligned(16))) uint16_t v_s[kStages][kTileKeys][kVRowPad];
+// LDS of one workgroup: kStages ring slots of K and V (fp16, or the pool's type) tiles. At D = 64 a
+// tile is 64 keys, so that every thread still loads one 16-byte chunk of K and one of V per tile
+// or more; the row pitch D + 16 elements keeps the bank pattern (a multiple of 8 banks per row).
+template <int D> struct PrefillLds {
+  static constexpr int kKeys = kTileKeys * 128 / D;
+  __attribute__((aligned(16))) uint16_t k_s[kStages][kKeys][kRowPad - 128 + D];
+  __attribute__((aligned(16))) uint16_t v_s[kStages][kKeys][kVRowPad - 128 + D];
 };
 
-// The query block q0 .. q0 + QW - 1 (QW = WAVES * CB * 16 / n_rep; q0 may be negative) of
-// sequence b, KV group g, with CB 16-column blocks per wave. With statistics (obs > 0) it also
-// writes, for each of the sequence's last obs queries in the block and each q head h, the pair
-// (m, l) of the column's running max m (log2 units) and its softmax denominator l (the sum of the
-// fp16 weights 2^(s * scale * log2e - m) over every key the query sees) into
-// obs_stats[b * stats_seq_stride + h * obs + i], for obs_rows_finish_kernel.
-template <int DT, int WAVES, int CB>
-__device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, const int g, const int q0,
-                                             PrefillLds& lds) {
-  constexpr int D = 128;
+// Softmax weights for P.V on 16-bit MFMAs with fp32-grade precision: p ~= hi + lo, both in V's
+// type (relative error below 2^-16 in bf16, 2^-21 in fp16). fp16 weights are lifted by 2^7 so
+// that small ones stay normal; the tile's vote keeps them below 2^8 (2^15 lifted).
+template <int DT> struct PrefillSplit;
+template <> struct PrefillSplit<UKV_DTYPE_BF16> {
+  static constexpr float kLift = 0.f;
+  static constexpr unsigned short kMax = 0x437F;  // bf16 bit pattern just below 2^8
+  static constexpr uint32_t kOnes = 0x3F803F80u;
+  static __device__ __forceinline__ void split(float x0, float x1, uint32_t& hi, uint32_t& lo) {
+    hi = pack_bf16(x0, x1);
+    lo = pack_bf16(x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xffff0000u));
+  }
+};
+template <> struct PrefillSplit<UKV_DTYPE_F16> {
+  static constexpr float kLift = 7.f;
+  static constexpr unsigned short kMax = 0x77FF;  // fp16 bit pattern just below 2^15
+  static constexpr uint32_t kOnes = 0x3C003C00u;
+  static __device__ __forceinline__ void split(float x0, float x1, uint32_t& hi, uint32_t& lo) {
+    hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0 - Elem<UKV_DTYPE_F16>::lo(hi),
+                                                                 x1 - Elem<UKV_DTYPE_F16>::hi(hi)));
+  }
+};
+
+// The columns c0 .. c0 + WAVES * CB * 16 - 1 of sequence b, KV group g, with CB 16-column blocks per
+// wave. Column c is the pair (query c / n_rep, q head g * n_rep + c % n_rep); c0 may be negative.
+//   FINE   the weights keep fp32-grade precision (PrefillSplit) and V its own type: shapes whose
+//          n_rep does not divide 16 or whose D is 64. Otherwise n_rep divides 16 (a query's heads
+//          lie in one column block) and P and V are fp16.
+//   PARTS  part `part` of the sequence's keys (part_count() of them), left for
+//          prefill_combine_kernel. The running max moves to whole powers of two, so that the
+//          parts' rounded weights are the ones an undivided pass would have summed.
+// With statistics (obs > 0) it also writes, for each of the sequence's last obs queries in the
+// block and each q head h, the pair (m, l) of the column's running max m (log2 units) and its
+// softmax denominator l (the sum of the fp16 weights 2^(s * scale * log2e - m) over every key the
+// query sees) into obs_stats[b * stats_seq_stride + h * obs + i], for obs_rows_finish_kernel.
+template <int DT, int D, int WAVES, int CB, bool FINE, bool PARTS>
+__device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, const int g, const int c0,
+                                             const int part, PrefillLds<D>& lds) {
   constexpr int STEPS = D / 32;
+  constexpr int NE = D / 16;  // output tiles of 16 dims
   constexpr int NT = 64 * WAVES;
-  constexpr int ITEMS = kTileKeys * 16 / NT;  // 16-byte chunks per thread per tensor per tile
+  constexpr int TK = PrefillLds<D>::kKeys;  // keys per tile
+  constexpr int PPT = TK / 16;              // pages per tile
+  constexpr int CH = D / 8;                 // 16-byte chunks per key row
+  constexpr int ITEMS = TK * CH / NT;       // 16-byte chunks per thread per tensor per tile
+  constexpr int PVT = FINE ? DT : (int)UKV_DTYPE_F16;  // type of the P.V operands
   constexpr float kTau = 8.f;
-  constexpr bool kBf16 = DT == UKV_DTYPE_BF16;
-  static_assert(ITEMS * NT == kTileKeys * 16, "loader mapping");
+  constexpr float kLift = FINE ? PrefillSplit<DT>::kLift : 0.f;
+  constexpr bool kConvert = DT == UKV_DTYPE_BF16 && !FINE;  // the loader converts V to fp16
+  static_assert(ITEMS * NT == TK * CH, "loader mapping");
   auto& k_s = lds.k_s;
-  auto& v_s = lds.v_s;  // fp16
+  auto& v_s = lds.v_s;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -229,47 +307,76 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   const int i16 = lane & 15;
   const int kg = lane >> 4;
 
-  const int qpb = 16 / a.n_rep;  // queries per column block
-  const int qw = WAVES * CB * qpb;
+  const int qpb = 16 / a.n_rep;  // queries per column block (not FINE)
   const int q_begin = a.cu_q[b];
   const int C = a.cu_q[b + 1] - q_begin;
-  if (q0 >= C || q0 + qw <= 0) return;  // whole workgroup
-  const int Lk = kv_len_of(a, b);
-  const int P0 = Lk - C;  // keys before the chunk
-  const int kend = max(0, min(Lk, P0 + min(C, q0 + qw)));
-  const int n_tiles = (kend + kTileKeys - 1) / kTileKeys;
+  // The block's queries [q0, q1) and the columns' division by n_rep: columns c0 + x of FINE blocks
+  // start at remainder rem of query q0, so query and head follow from (rem + x) / n_rep, a
+  // multiplication exact below 2^16 / n_rep.
+  const int q0 = FINE ? (c0 >= 0 ? c0 / a.n_rep : -((a.n_rep - 1 - c0) / a.n_rep)) : c0 / a.n_rep;
+  const int rem = FINE ? c0 - q0 * a.n_rep : 0;
+  const uint32_t inv_rep = FINE ? (65535u + a.n_rep) / a.n_rep : 0u;
+  const int q1 = FINE ? q0 + (rem + WAVES * CB * 16 + a.n_rep - 1) / a.n_rep : q0 + WAVES * CB * qpb;
+  if (q0 >= C || q1 <= 0) return;  // whole workgroup
+  int Lk = kv_len_of(a, b);
+  int P0 = Lk - C;  // keys before the chunk
+  int kend = max(0, min(Lk, P0 + min(C, q1)));
+  int key_a = 0;  // PARTS: first key of this part; Lk, P0 and kend count from it below
+  if constexpr (PARTS) {
+    const int nt = (Lk + TK - 1) / TK, np = part_count(a, nt);
+    if (part >= np) return;  // whole workgroup
+    key_a = (int)((int64_t)part * nt / np) * TK;
+    if (key_a >= kend) return;  // no row of the block sees this part (prefill_combine_kernel skips it)
+    kend = min(kend, (int)((int64_t)(part + 1) * nt / np) * TK) - key_a;
+    Lk -= key_a;
+    P0 -= key_a;
+  }
+  const int n_tiles = (kend + TK - 1) / TK;
   const int n_pg = (kend + 15) >> 4;
 
-  // This wave's queries and this lane's columns.
-  const int wq0 = q0 + wv * CB * qpb;
-  const bool wave_live = wq0 < C && wq0 + CB * qpb > 0;
+  // This wave's queries [wq0, wq1) and this lane's columns.
+  const int wx0 = rem + wv * CB * 16;  // the wave's first column, counted from query q0's first
+  const int wq0 = FINE ? q0 + (int)(wx0 * inv_rep >> 16) : q0 + wv * CB * qpb;
+  const int wq1 = FINE ? q0 + (int)((wx0 + CB * 16 - 1) * inv_rep >> 16) + 1 : wq0 + CB * qpb;
+  const bool wave_live = wq0 < C && wq1 > 0;
   const int wpos_min = P0 + wq0;
-  const int head = g * a.n_rep + i16 % a.n_rep;
-  // the query of this lane's column in column block cb is qi0 + cb * qpb (unused if outside 0 .. C - 1)
+  // Column x of the wave (x < CB * 16): its query and q head.
+  auto col_query = [&](int x) -> int { return FINE ? q0 + (int)((wx0 + x) * inv_rep >> 16) : wq0 + x / a.n_rep; };
+  auto col_head = [&](int x) -> int {
+    return FINE ? g * a.n_rep + (wx0 + x) - (int)((wx0 + x) * inv_rep >> 16) * a.n_rep : g * a.n_rep + x % a.n_rep;
+  };
+  const int head = g * a.n_rep + i16 % a.n_rep;  // (not FINE: the same in every column block)
+  // the query of this lane's column in column block cb (unused if outside 0 .. C - 1)
   const int qi0 = wq0 + i16 / a.n_rep;
+  int qic[FINE ? CB : 1];
+  if constexpr (FINE)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) qic[cb] = col_head(cb * 16 + i16) < a.Hq ? col_query(cb * 16 + i16) : -1;
+  auto lane_query = [&](int cb) -> int { return FINE ? qic[FINE ? cb : 0] : qi0 + cb * qpb; };
   u32x4 qv[CB][STEPS];
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
-    const int qi = qi0 + cb * qpb;
-    const bool live = qi >= 0 && qi < C && head < a.Hq;
-    const uint16_t* qp = a.q + (int64_t)(q_begin + (live ? qi : 0)) * a.q_st + (int64_t)(live ? head : 0) * a.q_sh +
+    const int qi = lane_query(cb);
+    const int hh = FINE ? col_head(cb * 16 + i16) : head;
+    const bool live = qi >= 0 && qi < C && hh < a.Hq;
+    const uint16_t* qp = a.q + (int64_t)(q_begin + (live ? qi : 0)) * a.q_st + (int64_t)(live ? hh : 0) * a.q_sh +
                          8 * kg;
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) qv[cb][s] = live ? ld16(qp + 32 * s) : u32x4{0u, 0u, 0u, 0u};
   }
 
   float m_ref[CB];  // running max of the column (log2 units)
-  f32x4 o[CB][8];
+  f32x4 o[CB][NE];
   f32x4 lacc[CB];  // softmax denominators of columns 4*kg + r
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
     m_ref[cb] = kNegFltMax;
     lacc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[cb][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < NE; ++e) o[cb][e] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // ---- tile loader: chunk idx = tid + i * NT is 16-byte chunk idx % 16 of key row idx / 16.
+  // ---- tile loader: chunk idx = tid + i * NT is 16-byte chunk idx % CH of key row idx / CH.
   // Tile u is loaded into register set u & 1 four tiles ahead, written into
   // ring slot u % 4 two tiles ahead (zeroing rows past the sequence or on an
   // invalid page and converting a bf16 V to fp16), and computed at tile u.
@@ -277,7 +384,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   // never writes it, and this keeps the wave-uniform page-id loads on the
   // scalar unit (SMEM), apart from the vector-memory count the tile loads use.
   typedef const __attribute__((address_space(4))) int32_t cint32;
-  cint32* btrow = (cint32*)(a.bt + (int64_t)b * a.max_blocks);
+  cint32* btrow = (cint32*)(a.bt + (int64_t)b * a.max_blocks + (key_a >> 4));
   auto page_id = [&](int pg) -> int { return pg < n_pg ? btrow[pg] : -1; };
   auto page_ok = [&](int id) -> bool { return (unsigned)id < (unsigned)a.num_pages; };
   // Within a page, this thread's chunk sits at a fixed offset; the page base is wave-uniform.
@@ -286,19 +393,27 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const int idx = tid + i * NT;
-    const int tok = (idx >> 4) & 15, ch = idx & 15;
+    const int tok = (idx / CH) & 15, ch = idx % CH;
     koff[i] = (uint32_t)(tok * a.k_st + g * a.k_sh + 8 * ch);
     voff[i] = (uint32_t)(tok * a.v_st + g * a.v_sh + 8 * ch);
-    lds_row[i] = idx >> 4;
+    lds_row[i] = idx / CH;
     lds_ch[i] = ch;
   }
   u32x4 rk0[ITEMS], rv0[ITEMS], rk1[ITEMS], rv1[ITEMS];
-  auto issue = [&](int id0, int id1, u32x4 (&rk)[ITEMS], u32x4 (&rv)[ITEMS]) {
+  // the page of chunk i of this thread among a tile's PPT (rows 16 j .. 16 j + 15 are page j); wave-uniform
+  auto chunk_page = [&](int i, const int (&ids)[PPT]) -> int {
+    const int j = __builtin_amdgcn_readfirstlane((tid + i * NT) / (16 * CH));
+    if constexpr (PPT == 2) {
+      return j ? ids[1] : ids[0];
+    } else {
+      const int i0 = ids[0], i1 = ids[1], i2 = ids[2], i3 = ids[3];  // (values: the array stays in registers)
+      return j < 2 ? (j ? i1 : i0) : (j == 2 ? i2 : i3);
+    }
+  };
+  auto issue = [&](const int (&ids)[PPT], u32x4 (&rk)[ITEMS], u32x4 (&rv)[ITEMS]) {
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-      // rows 0-15 of a tile come from its first page, rows 16-31 from the second
-      const int second = __builtin_amdgcn_readfirstlane((tid + i * NT) >> 8);
-      const int id = second ? id1 : id0;
+      const int id = chunk_page(i, ids);
       // page strides fit 32 bits (checked on the host): a 32 x 32 -> 64-bit scalar product
       const uint32_t pg = page_ok(id) ? (uint32_t)id : 0u;
       gload16(rk[i], a.k + (uint64_t)pg * (uint32_t)a.k_sp + koff[i]);
@@ -310,8 +425,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   // inf or NaN, i.e. a bf16 value fp16 cannot hold.
   typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
   hv2 vmax = {0, 0}, vmin = {0, 0};
-  auto store = [&](int u, int slot, int id0, int id1, u32x4 (&rk)[ITEMS], u32x4 (&rv)[ITEMS]) {
-    const bool full = page_ok(id0) && page_ok(id1) && kTileKeys * (u + 1) <= Lk;
+  auto store = [&](int u, int slot, const int (&ids)[PPT], u32x4 (&rk)[ITEMS], u32x4 (&rv)[ITEMS]) {
+    bool full = TK * (u + 1) <= Lk;
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) full = full && page_ok(ids[j]);
     // The other register set's 2 * ITEMS loads were issued after this set's.
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) vm_wait<2 * ITEMS>(rk[i], rv[i]);
@@ -321,13 +438,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
       // the zeroing then selects in place, with no copy of the loaded ones)
       u32x4 v;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) v[c] = kBf16 ? bf16x2_to_f16x2(rv[i][c]) : rv[i][c];
+      for (int c = 0; c < 4; ++c) v[c] = kConvert ? bf16x2_to_f16x2(rv[i][c]) : rv[i][c];
       if (!full) {  // (wave-uniform) rows past the sequence or on an invalid page hold junk
-        const bool ok = page_ok(lds_row[i] < 16 ? id0 : id1) && kTileKeys * u + lds_row[i] < Lk;
+        const bool ok = page_ok(chunk_page(i, ids)) && TK * u + lds_row[i] < Lk;
 #pragma unroll
         for (int c = 0; c < 4; ++c) v[c] = ok ? v[c] : 0u;
       }
-      if constexpr (kBf16) {
+      if constexpr (kConvert) {
         const uint32_t w0 = v[0], w1 = v[1], w2 = v[2], w3 = v[3];
         const hv2 c0 = __builtin_bit_cast(hv2, w0), c1 = __builtin_bit_cast(hv2, w1);
         const hv2 c2 = __builtin_bit_cast(hv2, w2), c3 = __builtin_bit_cast(hv2, w3);
@@ -341,38 +458,40 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     }
   };
 
-  // Page ids of tiles t .. t+3 (t_id[j] = tile t + j).
-  int t_id[4][2];
+  // Page ids of tiles t .. t+3 (t_id[j] = tile t + j) and of tile t+4.
+  int t_id[4][PPT], id_n[PPT];
+  auto tile_ids = [&](int t, int (&ids)[PPT]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    t_id[j][0] = page_id(2 * j);
-    t_id[j][1] = page_id(2 * j + 1);
-  }
+    for (int j = 0; j < PPT; ++j) ids[j] = page_id(PPT * t + j);
+  };
+#pragma unroll
+  for (int j = 0; j < 4; ++j) tile_ids(j, t_id[j]);
   // Prologue: tiles 0 and 1 into the ring, tiles 2 and 3 in flight. Loads are issued
   // unconditionally (tiles past the end read page 0 and are never used) so
   // that every wait is on loads of a fixed age: vmcnt(2) on the older set.
-  issue(t_id[0][0], t_id[0][1], rk0, rv0);
-  issue(t_id[1][0], t_id[1][1], rk1, rv1);
-  store(0, 0, t_id[0][0], t_id[0][1], rk0, rv0);
-  issue(t_id[2][0], t_id[2][1], rk0, rv0);
-  store(1, 1, t_id[1][0], t_id[1][1], rk1, rv1);
-  issue(t_id[3][0], t_id[3][1], rk1, rv1);
-  int id_n0 = page_id(8), id_n1 = page_id(9);  // page ids of tile t+4
+  issue(t_id[0], rk0, rv0);
+  issue(t_id[1], rk1, rv1);
+  store(0, 0, t_id[0], rk0, rv0);
+  issue(t_id[2], rk0, rv0);
+  store(1, 1, t_id[1], rk1, rv1);
+  issue(t_id[3], rk1, rv1);
+  tile_ids(4, id_n);
   // Retire every load issued so far (q columns, tiles 2 and 3) once, so that
   // no wait for them is left inside the loop.
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
 
-  // Tiles t < n_full end below the sequence end and below every column's diagonal (key
+  // 32-key runs t < n_full end below the sequence end and below every column's diagonal (key
   // 32t + 31 <= min(Lk - 1, wpos_min)).
   const int n_full = max(0, min(Lk, wpos_min + 1)) / kTileKeys;
   const float sl2 = a.scale_log2;
-  const uint32_t ones_f16 = 0x3C003C00u;
 
-  auto compute = [&](int t, int slot) {
-    const int key0 = t * kTileKeys;
-    const bool pg0 = page_ok(t_id[0][0]), pg1 = page_ok(t_id[0][1]);
-    const bool full = pg0 && pg1 && t < n_full;
+  // 32 keys at a time: run hf of tile t holds keys t * TK + 32 hf ..
+  auto compute_run = [&](int t, int slot, int hf) __attribute__((always_inline)) {
+    const int run = t * (TK / kTileKeys) + hf, row0 = hf * kTileKeys;
+    const int key0 = run * kTileKeys;
+    const bool pg0 = page_ok(t_id[0][2 * hf]), pg1 = page_ok(t_id[0][2 * hf + 1]);
+    const bool full = pg0 && pg1 && run < n_full;
     // S^T[key][column] for the tile's two 16-key blocks and every column block, masked. (As one
     // inlined function the register allocator keeps the three-column loop within 256 VGPRs with
     // no scratch under the iterative-ILP schedule this file is built with; written out in line,
@@ -384,7 +503,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
         for (int cb = 0; cb < CB; ++cb) sacc[kb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
-          const u32x4 ka = *reinterpret_cast<const u32x4*>(&k_s[slot][kb * 16 + i16][32 * s + 8 * kg]);
+          const u32x4 ka = *reinterpret_cast<const u32x4*>(&k_s[slot][row0 + kb * 16 + i16][32 * s + 8 * kg]);
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb) sacc[kb][cb] = mfma16x16x32<DT>(ka, qv[cb][s], sacc[kb][cb]);
         }
@@ -393,8 +512,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
         // key kb*16 + 4kg + r is visible to a column iff it is below lim[kb]
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
-          const int qi = qi0 + cb * qpb;
-          const bool live = qi >= 0 && qi < C && head < a.Hq;
+          const int qi = lane_query(cb);
+          const bool live = qi >= 0 && qi < C && (FINE || head < a.Hq);
           const int vis = live ? min(Lk, P0 + qi + 1) - key0 - 4 * kg : -1;  // an unused column sees no key
           const int lim0 = pg0 ? vis : 0, lim1 = pg1 ? vis - 16 : 0;
 #pragma unroll
@@ -411,15 +530,26 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     // 2^8: the packed fp16 P is checked (non-negative fp16 bit patterns order
     // like their values, and inf and NaN lie above), and a column block whose
     // max moved is rescaled and its P recomputed.
-    u32x4 pa[CB];
+    u32x4 pa[CB], pl[FINE ? CB : 1];  // pl: FINE's low parts
     auto exp_pack = [&](int cb) {
       float p[2][4];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[kb][r] = fast_exp2(__builtin_fmaf(sacc[kb][cb][r], sl2, -m_ref[cb]));
-      pa[cb] = u32x4{pack_f16(p[0][0], p[0][1]), pack_f16(p[0][2], p[0][3]), pack_f16(p[1][0], p[1][1]),
-                     pack_f16(p[1][2], p[1][3])};
+        for (int r = 0; r < 4; ++r)
+          p[kb][r] = fast_exp2(__builtin_fmaf(sacc[kb][cb][r], sl2, kLift != 0.f ? kLift - m_ref[cb] : -m_ref[cb]));
+      if constexpr (FINE) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t hi, lo;
+          PrefillSplit<DT>::split(p[i / 2][2 * (i & 1)], p[i / 2][2 * (i & 1) + 1], hi, lo);
+          pa[cb][i] = hi;
+          pl[cb][i] = lo;
+        }
+      } else {
+        pa[cb] = u32x4{pack_f16(p[0][0], p[0][1]), pack_f16(p[0][2], p[0][3]), pack_f16(p[1][0], p[1][1]),
+                       pack_f16(p[1][2], p[1][3])};
+      }
     };
     // Moves column block cb's max to the tile's where that lies more than kTau above it,
     // rescaling what was summed under the old one; returns whether it moved.
@@ -432,7 +562,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
       float mcol = fmaxf(mloc, __shfl_xor(mloc, 16));
       mcol = fmaxf(mcol, __shfl_xor(mcol, 32));
       if (!__any(mcol * sl2 > m_ref[cb] + kTau)) return false;
-      const float m_new = fmaxf(m_ref[cb], mcol * sl2);
+      const float m_new = fmaxf(m_ref[cb], PARTS ? __builtin_ceilf(mcol * sl2) : mcol * sl2);
       const float alpha = fast_exp2(m_ref[cb] - m_new);
       m_ref[cb] = m_new;
 #pragma unroll
@@ -440,7 +570,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
         const float ar = __shfl(alpha, 4 * kg + r);
         lacc[cb][r] *= ar;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[cb][e][r] *= ar;
+        for (int e = 0; e < NE; ++e) o[cb][e][r] *= ar;
       }
       return true;
     };
@@ -452,22 +582,38 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     {  // the tile's weights, then the vote on them
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) exp_pack(cb);
-      // The max of the packed weights with three-input fp16 maxima (v_pk_maximum3_f16): a NaN
-      // weight makes the maximum NaN, whose pattern, like inf's, lies above the threshold.
-      typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-      // (the element is copied out first: clang lowers __builtin_bit_cast of a vector element
-      // lvalue to a load of the vector's first element, whatever the index)
-      auto hv = [&](int i) {
-        const uint32_t w = pa[i / 4][i % 4];
-        return __builtin_bit_cast(h2, w);
-      };
-      h2 mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(hv(0), hv(1)), hv(2));
+      bool moved;
+      if constexpr (FINE) {
+        // (non-negative 16-bit float patterns order like their values; inf and NaN lie above)
+        u16x2 mx = {0, 0};
 #pragma unroll
-      for (int i = 3; i + 1 < 4 * CB; i += 2)
-        mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, hv(i)), hv(i + 1));
-      if constexpr ((4 * CB - 3) % 2) mx = __builtin_elementwise_maximum(mx, hv(4 * CB - 1));
-      const u16x2 pmax = __builtin_bit_cast(u16x2, mx);
-      if (__any(__builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(pmax, u16x2{0x5BFF, 0x5BFF})) != 0u)) {
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t w = pa[cb][i];
+            mx = __builtin_elementwise_max(mx, as_u16x2(w));
+          }
+        constexpr unsigned short kMax = PrefillSplit<DT>::kMax;
+        moved = __any(__builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(mx, u16x2{kMax, kMax})) != 0u);
+      } else {
+        // The max of the packed weights with three-input fp16 maxima (v_pk_maximum3_f16): a NaN
+        // weight makes the maximum NaN, whose pattern, like inf's, lies above the threshold.
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        // (the element is copied out first: clang lowers __builtin_bit_cast of a vector element
+        // lvalue to a load of the vector's first element, whatever the index)
+        auto hv = [&](int i) {
+          const uint32_t w = pa[i / 4][i % 4];
+          return __builtin_bit_cast(h2, w);
+        };
+        h2 mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(hv(0), hv(1)), hv(2));
+#pragma unroll
+        for (int i = 3; i + 1 < 4 * CB; i += 2)
+          mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, hv(i)), hv(i + 1));
+        if constexpr ((4 * CB - 3) % 2) mx = __builtin_elementwise_maximum(mx, hv(4 * CB - 1));
+        const u16x2 pmax = __builtin_bit_cast(u16x2, mx);
+        moved = __any(__builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(pmax, u16x2{0x5BFF, 0x5BFF})) != 0u);
+      }
+      if (moved) {
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb)
           if (settle(cb)) exp_pack(cb);
@@ -479,19 +625,29 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     // key order of P's A operand). ds_read_b64_tr_b16 builds it from row-major
     // V: within each 16-lane group, lane L names 4 dims 4(L%4).. of key row
     // L/4, and lane j receives dim j of the 4 rows.
-    const uint16_t* vlane = &v_s[slot][4 * kg + (i16 >> 2)][4 * (i16 & 3)];
+    const uint16_t* vlane = &v_s[slot][row0 + 4 * kg + (i16 >> 2)][4 * (i16 & 3)];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < NE; ++e) {
       const u32x2 lo = ds_read_tr16(vlane + 16 * e);
-      const u32x2 hi = ds_read_tr16(vlane + 16 * kVRowPad + 16 * e);
+      const u32x2 hi = ds_read_tr16(vlane + 16 * (kVRowPad - 128 + D) + 16 * e);
       const u32x4 bv = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) o[cb][e] = mfma16x16x32<UKV_DTYPE_F16>(pa[cb], bv, o[cb][e]);
+      for (int cb = 0; cb < CB; ++cb) o[cb][e] = mfma16x16x32<PVT>(pa[cb], bv, o[cb][e]);
+      if constexpr (FINE)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) o[cb][e] = mfma16x16x32<PVT>(pl[cb], bv, o[cb][e]);
     }
     // Denominators: the same P against a ones operand.
+    constexpr uint32_t kOnes = FINE ? PrefillSplit<DT>::kOnes : 0x3C003C00u;
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-      lacc[cb] = mfma16x16x32<UKV_DTYPE_F16>(pa[cb], u32x4{ones_f16, ones_f16, ones_f16, ones_f16}, lacc[cb]);
+    for (int cb = 0; cb < CB; ++cb) {
+      lacc[cb] = mfma16x16x32<PVT>(pa[cb], u32x4{kOnes, kOnes, kOnes, kOnes}, lacc[cb]);
+      if constexpr (FINE) lacc[cb] = mfma16x16x32<PVT>(pl[cb], u32x4{kOnes, kOnes, kOnes, kOnes}, lacc[cb]);
+    }
+  };
+  auto compute = [&](int t, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int hf = 0; hf < TK / kTileKeys; ++hf) compute_run(t, slot, hf);
   };
 
   // Tile t: (a) tile t+2 from register set t&1 into ring slot (t+2)%4; (b) tile t+4 into that
@@ -504,20 +660,18 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     constexpr int Q = decltype(phase)::value;  // t % 4: the ring slot of tile t
     constexpr int P = Q & 1;                   // register set of tile t+2
     // (a slot written past the last tile is never read)
-    if constexpr (P == 0) store(t + 2, (Q + 2) & 3, t_id[2][0], t_id[2][1], rk0, rv0);
-    else store(t + 2, (Q + 2) & 3, t_id[2][0], t_id[2][1], rk1, rv1);
-    if constexpr (P == 0) issue(id_n0, id_n1, rk0, rv0);
-    else issue(id_n0, id_n1, rk1, rv1);
+    if constexpr (P == 0) store(t + 2, (Q + 2) & 3, t_id[2], rk0, rv0);
+    else store(t + 2, (Q + 2) & 3, t_id[2], rk1, rv1);
+    if constexpr (P == 0) issue(id_n, rk0, rv0);
+    else issue(id_n, rk1, rv1);
     do_compute(t, Q);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      t_id[j][0] = t_id[j + 1][0];
-      t_id[j][1] = t_id[j + 1][1];
+    for (int i = 0; i < PPT; ++i) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) t_id[j][i] = t_id[j + 1][i];
+      t_id[3][i] = id_n[i];
     }
-    t_id[3][0] = id_n0;
-    t_id[3][1] = id_n1;
-    id_n0 = page_id(2 * (t + 5));
-    id_n1 = page_id(2 * (t + 5) + 1);
+    tile_ids(t + 5, id_n);
     if constexpr (P == 1) __syncthreads();
   };
   auto run = [&](auto do_compute) {
@@ -538,16 +692,33 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     vm_wait<0>(rk1[i], rv1[i]);
   }
 
-  // A bf16 V value that fp16 cannot hold anywhere in this workgroup's keys:
-  // recompute its columns on the fp32 fallback.
-  // (an fp16 magnitude pattern above 0x7BFF, the largest finite one, is an inf or a NaN)
-  const u16x2 mag = __builtin_elementwise_max(as_u16x2(__builtin_bit_cast(uint32_t, vmax) & 0x7fff7fffu),
-                                              as_u16x2(__builtin_bit_cast(uint32_t, vmin) & 0x7fff7fffu));
-  const bool wide_mine = kBf16 && __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(mag, u16x2{0x7BFF, 0x7BFF})) != 0u;
-  if (kBf16 && __syncthreads_or(wide_mine)) {
-    flag_obs_rows<WAVES>(a, b, g, C, max(q0, 0), min(C, q0 + qw));  // (none without statistics)
-    prefill_pairs_fp32<DT>(a, b, g, q_begin, C, P0, Lk, max(q0, 0), min(C, q0 + qw), wv, WAVES, lane);
-    return;
+  // A V the matrix cores got wrong anywhere in this workgroup's keys: its columns again on the fp32
+  // fallback.
+  bool redo_mine = false;
+  if constexpr (kConvert) {
+    // (an fp16 magnitude pattern above 0x7BFF, the largest finite one, is an inf or a NaN)
+    const u16x2 mag = __builtin_elementwise_max(as_u16x2(__builtin_bit_cast(uint32_t, vmax) & 0x7fff7fffu),
+                                                as_u16x2(__builtin_bit_cast(uint32_t, vmin) & 0x7fff7fffu));
+    redo_mine = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(mag, u16x2{0x7BFF, 0x7BFF})) != 0u;
+  }
+  if constexpr (FINE) {
+    // found from the accumulators: one that is not finite times zero is NaN
+    float z = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z = __builtin_fmaf(o[cb][e][r], 0.f, z);
+    redo_mine = z != 0.f;
+  }
+  if constexpr (kConvert || FINE) {
+    if (__syncthreads_or(redo_mine)) {
+      if (!PARTS) flag_obs_rows<WAVES>(a, b, g, C, max(q0, 0), min(C, q1));  // (none without statistics)
+      prefill_cols_fp32<DT, D>(a, b, g, q_begin, C, P0 + key_a, Lk + key_a, c0, WAVES * CB * 16, wv, WAVES, lane,
+                               PARTS ? part : -1, key_a, key_a + kend);
+      return;
+    }
   }
 
   // out[column] = o / l: lane (i16, kg) holds dims 16e + i16 of columns 4*kg + r,
@@ -558,21 +729,78 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int col = 4 * kg + r;
-      const int qi = wq0 + cb * qpb + col / a.n_rep;
-      const int hh = g * a.n_rep + col % a.n_rep;
+      const int qi = FINE ? col_query(cb * 16 + col) : wq0 + cb * qpb + col / a.n_rep;
+      const int hh = FINE ? col_head(cb * 16 + col) : g * a.n_rep + col % a.n_rep;
       // the column's running max, held by lane col (column i16 = col)
       const float m_col = __shfl(m_ref[cb], col);
       if (qi >= 0 && qi < C && hh < a.Hq) {
+        if constexpr (PARTS) {
+          // (FINE's lift by 2^kLift is in o and l alike: taken off the max)
+          const int64_t row = ((int64_t)part * a.total_q + q_begin + qi) * a.Hq + hh;
+          float* prow = a.part_o + row * D + i16;
+#pragma unroll
+          for (int e = 0; e < NE; ++e) prow[16 * e] = o[cb][e][r];
+          if (i16 == 0) a.part_ml[row] = make_float2(m_col - kLift, lacc[cb][r]);
+          continue;
+        }
         const float inv = 1.f / lacc[cb][r];
         uint16_t* orow = a.out + ((int64_t)(q_begin + qi) * a.Hq + hh) * D + i16;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) orow[16 * e] = Elem<DT>::from_float(o[cb][e][r] * inv);
+        for (int e = 0; e < NE; ++e) orow[16 * e] = Elem<DT>::from_float(o[cb][e][r] * inv);
         if (i16 == 0 && qi >= C - a.obs)  // (never without statistics: obs = 0)
           a.obs_stats[(int64_t)b * a.stats_seq_stride + (int64_t)hh * a.obs + (qi - (C - a.obs))] =
               make_float2(m_col, lacc[cb][r]);
       }
     }
   }
+}
+
+// Merges the parts of each (query, q head) row: with M the largest of the parts' m, out = sum(2^(m - M) O) / sum(2^(m - M) l). A group of D / 4 lanes takes
+// a row, float4 dims 4 * lane ..; its parts' rows are read four at a time. Part s holds a row's
+// keys iff it starts at or below the row's position; the others were not written.
+template <int DT, int D>
+__global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs a) {
+  constexpr int LANES = D / 4, ROWS = 256 / LANES;
+  constexpr int TK = PrefillLds<D>::kKeys;
+  const int64_t idx = (int64_t)blockIdx.x * ROWS + threadIdx.x / LANES;
+  if (idx >= (int64_t)a.total_q * a.Hq) return;
+  const int dq = threadIdx.x % LANES;
+  const int row = (int)(idx / a.Hq), h = (int)(idx % a.Hq);
+  int b = 0, hi = a.B;  // the last sequence starting at or before the row
+  while (hi - b > 1) {
+    const int mid = (b + hi) >> 1;
+    if (a.cu_q[mid] <= row) b = mid;
+    else hi = mid;
+  }
+  const int q_begin = a.cu_q[b], C = a.cu_q[b + 1] - q_begin, qi = row - q_begin;
+  if (qi < 0 || qi >= C || C > a.max_chunk) return;
+  const int Lk = kv_len_of(a, b);
+  const int nt = (Lk + TK - 1) / TK, np = part_count(a, nt);
+  const int pos = Lk - C + qi;
+  int n = 0;  // parts that hold the row's keys
+  while (n < np && pos >= 0 && (int)((int64_t)n * nt / np) * TK <= pos) ++n;
+  const int64_t stride = (int64_t)a.total_q * a.Hq;
+  float M = kNegFltMax;
+  for (int s = 0; s < n; ++s) M = fmaxf(M, a.part_ml[s * stride + idx].x);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+  bool flagged = false;
+#pragma unroll 4
+  for (int s = 0; s < n; ++s) {
+    const float2 ml = a.part_ml[s * stride + idx];
+    const f32x4 x = *reinterpret_cast<const f32x4*>(a.part_o + (s * stride + idx) * D + 4 * dq);
+    const float w = fast_exp2(ml.x - M);
+    flagged |= __builtin_signbit(ml.y);
+    l += w * fabsf(ml.y);
+    acc += w * x;
+  }
+  const float inv = 1.f / l;
+  const uint32_t w0 = Elem<DT>::from_float(acc[0] * inv) | (uint32_t)Elem<DT>::from_float(acc[1] * inv) << 16;
+  const uint32_t w1 = Elem<DT>::from_float(acc[2] * inv) | (uint32_t)Elem<DT>::from_float(acc[3] * inv) << 16;
+  *reinterpret_cast<u32x2*>(a.out + idx * D + 4 * dq) = u32x2{w0, w1};
+  if (dq == 0 && qi >= C - a.obs)  // (never without statistics: obs = 0)
+    a.obs_stats[(int64_t)b * a.stats_seq_stride + (int64_t)h * a.obs + (qi - (C - a.obs))] =
+        flagged ? make_float2(NAN, 1.f) : make_float2(M, l);
 }
 
 // Rows lo .. hi - 1 of sequence b's chunk, the q heads of KV group g, set to NaN (0x7FFF is a
@@ -623,6 +851,10 @@ __device__ __forceinline__ bool locate_item(int start, int end, int n, int nl, i
   return false;
 }
 
+// Column blocks per wave of the wide query blocks (the narrow ones have one fewer): the widest whose
+// accumulators, queries and weights stay in 256 VGPRs.
+constexpr int wide_blocks(bool fine, int d) { return fine && d == 128 ? 2 : 3; }
+
 // The range of work items [start, end) of a launch's n_items items that XCD xcd runs: dispatch
 // is round-robin over the 8 XCDs, so the workgroups with blockIdx.x % 8 == xcd run there, and
 // each XCD takes a contiguous range of the item numbers.
@@ -640,30 +872,47 @@ __device__ __forceinline__ void xcd_range(int total, int xcd, int& start, int& e
 // (prefill_tile), which obs_rows_finish_kernel turns into SnapKV row statistics. (Launches without
 // statistics run the same instance: compiled with that epilogue, the tile loop's schedule is 0.7 %
 // faster at config 4 than without it.)
-template <int DT, int WAVES>
+//
+// With PARTS each block comes n_parts times, the blocks of one part next to each other.
+template <int DT, int D, int WAVES, bool FINE, bool PARTS>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 paged_prefill_kernel(const PrefillArgs a) {
-  __shared__ PrefillLds lds;
-  const int n_items = a.n3 + a.n2;
+  __shared__ PrefillLds<D> lds;
+  constexpr int CB3 = wide_blocks(FINE, D), CB2 = CB3 - 1;
+  const int n_items = a.n3 + a.n2, parts = PARTS ? a.n_parts : 1;
   int start, end, pair, j;
-  xcd_range(n_items * a.n_groups * a.B, blockIdx.x & 7, start, end);
-  if (!locate_item(start, end, n_items, a.n3, blockIdx.x >> 3, pair, j)) return;  // (never: the grid holds total)
+  xcd_range(n_items * parts * a.n_groups * a.B, blockIdx.x & 7, start, end);
+  if (!locate_item(start, end, n_items * parts, a.n3 * parts, blockIdx.x >> 3, pair, j)) return;  // (never: the grid holds total)
+  int part = 0;
+  if constexpr (PARTS) {
+    if (j < a.n3 * parts) {
+      part = j / a.n3;
+      j -= part * a.n3;
+    } else {
+      j -= a.n3 * parts;
+      part = j / a.n2;
+      j += a.n3 - part * a.n2;
+    }
+  }
   const int g = pair % a.n_groups, b = pair / a.n_groups;
   const int C = a.cu_q[b + 1] - a.cu_q[b];
-  const int qpb = 16 / a.n_rep;
-  const int qw2 = WAVES * 2 * qpb, qw3 = WAVES * 3 * qpb;
+  constexpr int w2 = WAVES * CB2 * 16, w3 = WAVES * CB3 * 16;
   if (C > a.max_chunk) {
-    const int q0 = j < a.n3 ? C - qw3 * (j + 1) : C - qw3 * a.n3 - qw2 * (j - a.n3 + 1);
-    const int q1 = min(C, j < a.n3 ? q0 + qw3 : q0 + qw2);
-    const int lo = j == n_items - 1 ? 0 : max(0, q0);
-    prefill_nan_rows<WAVES>(a, b, g, lo, q1);
-    flag_obs_rows<WAVES>(a, b, g, C, lo, q1);  // (none without statistics)
+    if (part > 0) return;
+    const int cols = a.max_chunk * a.n_rep;  // the plan's columns, counted from the end of the chunk
+    const int c1 = cols - (j < a.n3 ? w3 * j : w3 * a.n3 + w2 * (j - a.n3)), c0 = c1 - (j < a.n3 ? w3 : w2);
+    const int skip = C - a.max_chunk;
+    const int lo = j == n_items - 1 ? 0 : max(0, skip + (max(c0, 0) / a.n_rep));
+    const int hi = min(C, skip + (max(c1, 0) + a.n_rep - 1) / a.n_rep);
+    prefill_nan_rows<WAVES>(a, b, g, lo, hi);
+    flag_obs_rows<WAVES>(a, b, g, C, lo, hi);  // (none without statistics)
     return;
   }
+  const int cols = C * a.n_rep;
   if (j < a.n3)
-    prefill_tile<DT, WAVES, 3>(a, b, g, C - qw3 * (j + 1), lds);
+    prefill_tile<DT, D, WAVES, CB3, FINE, PARTS>(a, b, g, cols - w3 * (j + 1), part, lds);
   else
-    prefill_tile<DT, WAVES, 2>(a, b, g, C - qw3 * a.n3 - qw2 * (j - a.n3 + 1), lds);
+    prefill_tile<DT, D, WAVES, CB2, FINE, PARTS>(a, b, g, cols - w3 * a.n3 - w2 * (j - a.n3 + 1), part, lds);
 }
 
 // SnapKV row statistics from the (m, l) pairs paged_prefill_kernel left in obs_stats.
@@ -988,18 +1237,21 @@ extern "C" int ukv_kv_write_varlen(void* k_pool_layer, void* v_pool_layer, const
 
 namespace {
 
-// Block plan of the tiled prefill: the numbers n3 and n2 of three- and two-column query blocks
-// per (sequence, KV group) that cover its chunk's max_chunk queries. A launch runs in rounds of
-// one block per CU; the plan with the shortest predicted launch is taken, modelling every block as streaming equally many keys (a long prefix) at its
-// measured cost relative to a three-column block (two columns 0.79: single blocks timed over the
-// same 32768 keys), and each XCD's CUs as taking the XCD's blocks in the kernel's order, each CU
-// the next block once free.
+// Block plan of the tiled prefill: the numbers n3 and n2 of wide and narrow query blocks per
+// (sequence, KV group) that cover its chunk's max_chunk queries, and the parts its keys are cut
+// into. A launch runs in rounds of one block per CU; the plan with the shortest predicted launch is
+// taken, modelling every block as streaming equally many keys (a long prefix) at its measured cost
+// relative to a wide block, and each XCD's CUs as taking the XCD's blocks in the kernel's order, each
+// CU the next block once free.
 struct BlockPlan {
   int n3, n2;
+  int parts, part_tiles;
 };
 
-double plan_makespan(int64_t pairs, int n3, int n2, int cus_per_xcd) {
-  const int n_items = n3 + n2;
+// One block's time is item * (cost of its width), plus a fixed start.
+double plan_makespan(int64_t pairs, int n3, int n2, int parts, double item, double start_cost, double narrow,
+                     int cus_per_xcd) {
+  const int n_items = (n3 + n2) * parts, nl = n3 * parts;
   const int64_t total = pairs * n_items;
   const int64_t per = total / 8, rem = total % 8;
   double worst = 0.0;
@@ -1011,9 +1263,9 @@ double plan_makespan(int64_t pairs, int n3, int n2, int cus_per_xcd) {
     if (end > start)
       for (int pass = 0; pass < 2; ++pass)
         for (int64_t p = start / n_items; p <= (end - 1) / n_items; ++p) {
-          const int64_t j0 = std::max<int64_t>(pass ? n3 : 0, start - p * n_items);
-          const int64_t j1 = std::min<int64_t>(pass ? n_items : n3, end - p * n_items);
-          for (int64_t j = j0; j < j1; ++j) order.push_back(j < n3 ? 1.0 : 0.79);
+          const int64_t j0 = std::max<int64_t>(pass ? nl : 0, start - p * n_items);
+          const int64_t j1 = std::min<int64_t>(pass ? n_items : nl, end - p * n_items);
+          for (int64_t j = j0; j < j1; ++j) order.push_back(start_cost + item * (j < nl ? 1.0 : narrow));
         }
     std::priority_queue<double, std::vector<double>, std::greater<double>> cu;
     for (int c = 0; c < cus_per_xcd; ++c) cu.push(0.0);
@@ -1029,27 +1281,54 @@ double plan_makespan(int64_t pairs, int n3, int n2, int cus_per_xcd) {
   return worst;
 }
 
-BlockPlan choose_plan(int max_chunk, int64_t pairs, int qw2, int qw3, int cus_per_xcd) {
-  const int n3_max = (std::max(0, max_chunk) + qw3 - 1) / qw3;
-  BlockPlan best{n3_max, 0};
-  // Large launches run many rounds, where the last one matters little: keep three-column blocks.
+// Cost of a narrow block relative to a wide one: single blocks timed over the same 32768 keys.
+constexpr double kNarrowCost = 0.79, kNarrowCostFine = 0.62;
+// Key parts: a block's fixed cost (first loads, page ids, the partial's store) and the merge's, in
+// tile times, and the fewest tiles a part is worth starting a block for.
+constexpr double kStartTiles = 4.0, kMergeTiles = 6.0;
+constexpr int kMinPartTiles = 12, kMaxParts = 16;
+
+// max_cols: columns (query, head) of the longest chunk; w2, w3: columns of a narrow and a wide block;
+// tiles: key tiles of the widest table row. Parts are considered where allow_parts and the launch
+// is short of two blocks per CU: there whole blocks leave CUs idle.
+BlockPlan choose_plan(int64_t max_cols, int64_t pairs, int w2, int w3, double narrow, int cus_per_xcd, int tiles,
+                      bool allow_parts) {
+  const int n3_max = (int)((max_cols + w3 - 1) / w3);
+  BlockPlan best{n3_max, 0, 1, std::max(1, tiles)};
+  // Large launches run many rounds, where the last one matters little: keep wide blocks.
   if (pairs * n3_max > (1 << 16) || cus_per_xcd <= 0 || n3_max == 0) return best;
+  const bool parts_ok = allow_parts && tiles >= 2 * kMinPartTiles && pairs * n3_max < 16 * cus_per_xcd;
   static std::mutex mu;
-  static std::map<std::tuple<int, int64_t, int, int>, BlockPlan> cache;
-  const auto key = std::make_tuple(max_chunk, pairs, qw2, cus_per_xcd);
+  static std::map<std::tuple<int64_t, int64_t, int, int, int, int>, BlockPlan> cache;
+  const auto key = std::make_tuple(max_cols, pairs, w2, w3, cus_per_xcd, parts_ok ? tiles : 0);
   std::lock_guard<std::mutex> lock(mu);
   const auto hit = cache.find(key);
   if (hit != cache.end()) return hit->second;
-  double best_t = plan_makespan(pairs, n3_max, 0, cus_per_xcd);
-  // Each three-column block traded for two-column ones adds work (0.79 x 1.5 > 1): a dozen
-  // trades fill any last round.
+  auto narrow_blocks = [&](int n3) { return (int)((max_cols - (int64_t)n3 * w3 + w2 - 1) / w2); };
+  double best_t = plan_makespan(pairs, n3_max, 0, 1, 1.0, 0.0, narrow, cus_per_xcd);
+  // Each wide block traded for narrow ones adds work: a dozen trades fill any last round.
   for (int n3 = n3_max - 1; n3 >= std::max(0, n3_max - 12); --n3) {
-    const int n2 = (max_chunk - n3 * qw3 + qw2 - 1) / qw2;
-    const double t = plan_makespan(pairs, n3, n2, cus_per_xcd);
+    const int n2 = narrow_blocks(n3);
+    const double t = plan_makespan(pairs, n3, n2, 1, 1.0, 0.0, narrow, cus_per_xcd);
     if (t < best_t - 1e-9) {
       best_t = t;
-      best = BlockPlan{n3, n2};
+      best.n3 = n3;
+      best.n2 = n2;
     }
+  }
+  if (parts_ok) {
+    best_t = best_t * tiles + kStartTiles;
+    const int max_parts = std::min(kMaxParts, tiles / kMinPartTiles);
+    for (int parts = 2; parts <= max_parts; ++parts)
+      for (int n3 = n3_max; n3 >= std::max(0, n3_max - 2); --n3) {
+        const int n2 = n3 == n3_max ? 0 : narrow_blocks(n3);
+        const double t = kMergeTiles + plan_makespan(pairs, n3, n2, parts, (double)tiles / parts, kStartTiles, narrow,
+                                                     cus_per_xcd);
+        if (t < 0.95 * best_t) {
+          best_t = t;
+          best = BlockPlan{n3, n2, parts, (tiles + parts - 1) / parts};
+        }
+      }
   }
   if (cache.size() >= 4096) cache.clear();  // a caller cycling through many shapes recomputes
   cache.emplace(key, best);
@@ -1077,11 +1356,67 @@ struct ObsStats {
   int sink, obs;
 };
 
+// The tiled kernel's instance for a head shape: FINE where n_rep does not divide 16 (a query's heads
+// straddle column blocks) or D is 64, shapes that were computed with fp32 weights before it and keep
+// that precision.
+bool tiled_shape(int head_dim, int n_rep) { return (head_dim == 128 || head_dim == 64) && n_rep <= 64; }
+bool fine_shape(int head_dim, int n_rep) { return head_dim != 128 || 16 % n_rep != 0; }
+
+BlockPlan plan_for(int batch, int max_chunk, int n_groups, int head_dim, int n_rep, int max_blocks, bool parts) {
+  constexpr int W = UKV_PREFILL_WAVES;
+  const bool fine = fine_shape(head_dim, n_rep);
+  const int cb3 = wide_blocks(fine, head_dim), cb2 = cb3 - 1;
+  const int tile_pages = head_dim == 64 ? PrefillLds<64>::kKeys / 16 : PrefillLds<128>::kKeys / 16;
+  return choose_plan((int64_t)max_chunk * n_rep, (int64_t)n_groups * batch, W * cb2 * 16, W * cb3 * 16,
+                     cb3 == 2 ? kNarrowCostFine : kNarrowCost, cus_per_xcd(), (max_blocks + tile_pages - 1) / tile_pages,
+                     parts);
+}
+
+size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
+size_t part_o_bytes(int parts, int64_t rows, int head_dim) { return up256((size_t)parts * rows * head_dim * sizeof(float)); }
+size_t part_bytes(int parts, int64_t rows, int head_dim) {
+  return part_o_bytes(parts, rows, head_dim) + up256((size_t)parts * rows * sizeof(float2));
+}
+// Partials above this are not worth their traffic: the launch is large enough without parts.
+constexpr size_t kMaxPartBytes = size_t(512) << 20;
+
+template <int DT, int D, bool FINE, bool PARTS>
+void launch_tiled(const PrefillArgs& a, unsigned wgs, hipStream_t stream) {
+  constexpr int W = UKV_PREFILL_WAVES;
+  hipLaunchKernelGGL((paged_prefill_kernel<DT, D, W, FINE, PARTS>), dim3(wgs), dim3(64 * W), 0, stream, a);
+  if constexpr (PARTS) {
+    constexpr int ROWS = 256 / (D / 4);
+    const int64_t rows = (int64_t)a.total_q * a.Hq;
+    hipLaunchKernelGGL((prefill_combine_kernel<DT, D>), dim3((unsigned)((rows + ROWS - 1) / ROWS)), dim3(256), 0,
+                       stream, a);
+  }
+}
+
+template <int DT, bool PARTS>
+void launch_tiled_dt(const PrefillArgs& a, bool fine, unsigned wgs, hipStream_t stream) {
+  if (a.D == 64)
+    launch_tiled<DT, 64, true, PARTS>(a, wgs, stream);
+  else if (fine)
+    launch_tiled<DT, 128, true, PARTS>(a, wgs, stream);
+  else
+    launch_tiled<DT, 128, false, PARTS>(a, wgs, stream);
+}
+
+void launch_tiled_any(const PrefillArgs& a, int dtype, bool fine, unsigned wgs, hipStream_t stream) {
+  const bool parts = a.n_parts > 1;
+  if (dtype == UKV_DTYPE_BF16)
+    parts ? launch_tiled_dt<UKV_DTYPE_BF16, true>(a, fine, wgs, stream)
+          : launch_tiled_dt<UKV_DTYPE_BF16, false>(a, fine, wgs, stream);
+  else
+    parts ? launch_tiled_dt<UKV_DTYPE_F16, true>(a, fine, wgs, stream)
+          : launch_tiled_dt<UKV_DTYPE_F16, false>(a, fine, wgs, stream);
+}
+
 int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
                  const int32_t* cu_seqlens_q, const int32_t* kv_lens, void* out, int batch, int total_q, int max_chunk,
                  int num_q_heads, int num_kv_heads, int head_dim, int n_rep, int max_blocks, int num_pages,
                  const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides, float softmax_scale,
-                 int dtype, ukv_stream_t stream_handle, const ObsStats* obs) {
+                 int dtype, void* workspace, size_t workspace_bytes, ukv_stream_t stream_handle, const ObsStats* obs) {
   if (batch <= 0 || num_q_heads <= 0 || head_dim <= 0) return UKV_ERR_EMPTY;
   if (head_dim > 256) return UKV_ERR_HEAD_DIM;
   if (dtype != UKV_DTYPE_F16 && dtype != UKV_DTYPE_BF16) return UKV_ERR_DTYPE;
@@ -1130,8 +1465,7 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
   const bool strides_ok = mul8(a.q_st) && mul8(a.q_sh) && mul8(a.k_sp) && mul8(a.k_st) && mul8(a.k_sh) &&
                           mul8(a.v_sp) && mul8(a.v_st) && mul8(a.v_sh) && in_page_ok(a.k_st, a.k_sh) &&
                           in_page_ok(a.v_st, a.v_sh) && page_stride_ok(a.k_sp) && page_stride_ok(a.v_sp);
-  const bool fast = head_dim == 128 && softmax_scale > 0.f && std::isfinite(softmax_scale) && (n_rep == 1 || n_rep == 2 || n_rep == 4 || n_rep == 8 || n_rep == 16) &&
-                    strides_ok && al16(q) && al16(out) && al16(k_cache) && al16(v_cache) && max_blocks > 0;
+  const bool fast = tiled_shape(head_dim, n_rep) && softmax_scale > 0.f && std::isfinite(softmax_scale) && strides_ok && al16(q) && al16(out) && al16(k_cache) && al16(v_cache) && max_blocks > 0;
   if (obs) {
     a.obs_stats = static_cast<float2*>(obs->stats);
     a.stats_seq_stride = obs->seq_stride;
@@ -1139,22 +1473,38 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
     a.obs = obs->obs;
   }
   if (fast) {
-    constexpr int W = UKV_PREFILL_WAVES;
-    const int qw2 = W * 2 * (16 / n_rep), qw3 = W * 3 * (16 / n_rep);
-    const int64_t pairs = (int64_t)n_groups * batch;
-    const BlockPlan plan = choose_plan(max_chunk, pairs, qw2, qw3, cus_per_xcd());
+    const bool fine = fine_shape(head_dim, n_rep);
+    const int64_t pairs = (int64_t)n_groups * batch, rows = (int64_t)total_q * num_q_heads;
+    BlockPlan plan = plan_for(batch, max_chunk, n_groups, head_dim, n_rep, max_blocks, workspace != nullptr);
+    // (the caller sizes the workspace by the same plan; a smaller one runs without parts)
+    if (plan.parts > 1 && (part_bytes(plan.parts, rows, head_dim) > workspace_bytes ||
+                           (rows + 7) / 8 > INT32_MAX || (reinterpret_cast<uintptr_t>(workspace) & 15u)))
+      plan = plan_for(batch, max_chunk, n_groups, head_dim, n_rep, max_blocks, false);
     a.n3 = plan.n3;
     a.n2 = plan.n2;
-    const int64_t wgs = (int64_t)(a.n3 + a.n2) * pairs;
-    const int64_t finish_waves = obs ? (int64_t)batch * n_groups * ((a.obs * n_rep + 15) / 16) : 0;
+    a.n_parts = plan.parts;
+    a.part_tiles = plan.part_tiles;
+    a.total_q = total_q;
+    if (plan.parts > 1) {
+      a.part_o = static_cast<float*>(workspace);
+      a.part_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + part_o_bytes(plan.parts, rows, head_dim));
+    }
+    const int64_t wgs = (int64_t)(a.n3 + a.n2) * plan.parts * pairs;
+    // FINE instances write no statistics: every row is flagged, and the scoring pass recomputes
+    // them from the keys.
+    const int obs_rows = obs && fine ? a.obs : 0;
+    if (fine) a.obs = 0;
+    const int64_t finish_waves = obs && !fine ? (int64_t)batch * n_groups * ((a.obs * n_rep + 15) / 16) : 0;
     if (wgs > INT32_MAX || (finish_waves + 3) / 4 > INT32_MAX) return UKV_ERR_INVALID_ARGUMENT;
     if (wgs > 0) {
       // With statistics, the prefill kernel writes the observation rows' (m, l) pairs and
       // obs_rows_finish_kernel, next on the same stream, turns them into the rows.
-      if (dtype == UKV_DTYPE_BF16)
-        hipLaunchKernelGGL((paged_prefill_kernel<UKV_DTYPE_BF16, W>), dim3((unsigned)wgs), dim3(64 * W), 0, stream, a);
-      else
-        hipLaunchKernelGGL((paged_prefill_kernel<UKV_DTYPE_F16, W>), dim3((unsigned)wgs), dim3(64 * W), 0, stream, a);
+      launch_tiled_any(a, dtype, fine, (unsigned)wgs, stream);
+    }
+    if (obs_rows > 0) {
+      a.obs = obs_rows;
+      const int64_t flags = (int64_t)batch * num_q_heads * a.obs;
+      hipLaunchKernelGGL(obs_flag_kernel, dim3((unsigned)((flags + 255) / 256)), dim3(256), 0, stream, a, flags);
     }
     if (finish_waves > 0) {
       const dim3 fgrid((unsigned)((finish_waves + 3) / 4));
@@ -1190,7 +1540,7 @@ extern "C" int ukv_paged_prefill(const void* q, const void* k_cache, const void*
                                  int dtype, ukv_stream_t stream_handle) {
   return prefill_impl(q, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, out, batch, total_q, max_chunk,
                       num_q_heads, num_kv_heads, head_dim, n_rep, max_blocks, num_pages, q_strides, k_strides,
-                      v_strides, softmax_scale, dtype, stream_handle, nullptr);
+                      v_strides, softmax_scale, dtype, nullptr, 0, stream_handle, nullptr);
 }
 
 extern "C" int ukv_paged_prefill_obs_stats(const void* q, const void* k_cache, const void* v_cache,
@@ -1207,5 +1557,35 @@ extern "C" int ukv_paged_prefill_obs_stats(const void* q, const void* k_cache, c
   const ObsStats st{obs_stats, stats_seq_stride, sink_len, obs_len};
   return prefill_impl(q, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, out, batch, total_q, max_chunk,
                       num_q_heads, num_kv_heads, head_dim, n_rep, max_blocks, num_pages, q_strides, k_strides,
-                      v_strides, softmax_scale, dtype, stream_handle, &st);
+                      v_strides, softmax_scale, dtype, nullptr, 0, stream_handle, &st);
+}
+
+extern "C" size_t ukv_paged_prefill_workspace_bytes(int batch, int total_q, int max_chunk, int num_q_heads,
+                                                    int num_kv_heads, int head_dim, int n_rep, int max_blocks) {
+  if (batch <= 0 || total_q <= 0 || max_chunk <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || n_rep < 1 ||
+      max_blocks <= 0 || !tiled_shape(head_dim, n_rep))
+    return 0;
+  const int n_groups = (num_q_heads + n_rep - 1) / n_rep;
+  const BlockPlan plan = plan_for(batch, max_chunk, n_groups, head_dim, n_rep, max_blocks, true);
+  if (plan.parts <= 1) return 0;
+  const size_t bytes = part_bytes(plan.parts, (int64_t)total_q * num_q_heads, head_dim);
+  return bytes > kMaxPartBytes ? 0 : bytes;
+}
+
+extern "C" int ukv_paged_prefill_parts(const void* q, const void* k_cache, const void* v_cache,
+                                       const int32_t* block_table, const int32_t* cu_seqlens_q,
+                                       const int32_t* kv_lens, void* out, int batch, int total_q, int max_chunk,
+                                       int num_q_heads, int num_kv_heads, int head_dim, int n_rep, int max_blocks,
+                                       int num_pages, const int64_t* q_strides, const int64_t* k_strides,
+                                       const int64_t* v_strides, float softmax_scale, int dtype, int sink_len,
+                                       int obs_len, float* obs_stats, int64_t stats_seq_stride, void* workspace,
+                                       size_t workspace_bytes, ukv_stream_t stream_handle) {
+  if (obs_stats && (sink_len < 0 || obs_len <= 0 || (reinterpret_cast<uintptr_t>(obs_stats) & 7u) ||
+                    stats_seq_stride < (int64_t)num_q_heads * obs_len))
+    return UKV_ERR_INVALID_ARGUMENT;
+  const ObsStats st{obs_stats, stats_seq_stride, sink_len, obs_len};
+  return prefill_impl(q, k_cache, v_cache, block_table, cu_seqlens_q, kv_lens, out, batch, total_q, max_chunk,
+                      num_q_heads, num_kv_heads, head_dim, n_rep, max_blocks, num_pages, q_strides, k_strides,
+                      v_strides, softmax_scale, dtype, workspace, workspace_bytes, stream_handle,
+                      obs_stats ? &st : nullptr);
 }

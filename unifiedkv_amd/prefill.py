@@ -157,14 +157,15 @@ def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
             min(int(k_cache.shape[0]), int(v_cache.shape[0])), _ext.i64_array(q.stride()[:2]),
             _ext.i64_array(k_cache.stride()[:3]), _ext.i64_array(v_cache.stride()[:3]), float(softmax_scale),
             _DTYPE_CODES[q.dtype]]
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    if stats_view is None:
-        code = _ext.load().ukv_paged_prefill(*args, stream)
-    else:
-        code = _ext.load().ukv_paged_prefill_obs_stats(*args, obs_stats.sink_len, obs_stats.obs_len, *stats_view,
-                                                        stream)
-        if code == _ext.UKV_OK:
-            obs_stats.mark(layer_id, seq_lens)
+    lib = _ext.load()
+    # The parts' scratch comes from the caching allocator, which keeps it for this stream's kernels.
+    need = lib.ukv_paged_prefill_workspace_bytes(B, total_q, mc, Hq, Hkv, D, int(n_rep), int(bt.shape[1]))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    stats_args = (0, 0, None, 0) if stats_view is None else (obs_stats.sink_len, obs_stats.obs_len, *stats_view)
+    code = lib.ukv_paged_prefill_parts(*args, *stats_args, ws.data_ptr() if ws is not None else None, need,
+                                       torch.cuda.current_stream(dev).cuda_stream)
+    if code == _ext.UKV_OK and stats_view is not None:
+        obs_stats.mark(layer_id, seq_lens)
     if code != _ext.UKV_OK:
         raise RuntimeError(f"paged_prefill_error:{_ext.status_string(code)}")
     return out
