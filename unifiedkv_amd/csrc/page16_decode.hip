@@ -55,6 +55,7 @@ struct DecodeArgs {
   int64_t v_sp, v_st, v_sh;
   int B, Hq, n_rep, n_groups, D, max_blocks, num_pages;
   int grid_wgs;      // G: workgroups sharing the batch's pages
+  int subs;          // waves of a workgroup that share each KV head's pages (split kernel, SHARED)
   // Decode-token append (fused variant): k_new/v_new [B][n_groups][D] rows with
   // strides n_sb, n_sh; the token of sequence b goes to position lens[b] - 1.
   const uint16_t* k_new;
@@ -71,20 +72,24 @@ __device__ __forceinline__ int clamp_len(int L, int max_blocks) {
 
 __device__ __forceinline__ int pages_of(int len, int max_blocks) { return (clamp_len(len, max_blocks) + 15) >> 4; }
 
-__device__ __forceinline__ int wave_sum_i32(int x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+// Inclusive prefix sum over the wave's 64 lanes, in registers: DPP row shifts inside each 16-lane
+// row, then the rows' totals broadcast onwards (0x111 + n - 1 = row_shr:n, 0x142 / 0x143 =
+// row_bcast:15 / :31). Six dependent VALU adds; six cross-lane LDS permutes took ~0.3 us here.
+__device__ __forceinline__ int wave_inclusive_scan_i32(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
   return x;
 }
 
-__device__ __forceinline__ int wave_inclusive_scan_i32(int x) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
-  return x;
+// floor(x * y / z) for 0 <= x, y and 0 < z: one 32-bit division where the product fits.
+__device__ __forceinline__ int mul_div(int x, int y, int z) {
+  const uint64_t p = (uint64_t)(uint32_t)x * (uint32_t)y;
+  if ((p >> 32) == 0) return (int)((uint32_t)p / (uint32_t)z);
+  return (int)(p / (uint32_t)z);
 }
 
 // Splits fp32 softmax weights into two 16-bit parts (p ~= hi + lo, relative
@@ -123,9 +128,6 @@ template <> struct PSplit<UKV_DTYPE_F16> {
   }
 };
 
-#ifndef UKV_PAGE16_PIPE
-#define UKV_PAGE16_PIPE 2
-#endif
 #ifndef UKV_PAGE16_NT
 #define UKV_PAGE16_NT 1
 #endif
@@ -207,17 +209,31 @@ __device__ __forceinline__ void load_vrow(const uint16_t* p, VRow<DPL>& r) {
 // pipelined loop). Every (page, KV head) is read by exactly one wave, so each
 // token row is written once, and the attention sees the same values as an
 // append followed by a plain decode.
-template <int DT, int D, bool APPEND>
+//
+// SHARED (fewer KV heads than half the waves of a workgroup): a.subs waves serve each KV head, wave
+// sub * n_groups + g taking every a.subs-th page of the workgroup's segment, and their partials meet in
+// LDS before one is written. One wave per head would leave the chip with 1/8 (one KV head) of the waves
+// it needs to cover HBM's latency.
+//
+// DIRECT (short tables): workgroup (b, g) takes the whole of sequence b for KV head g, its waves
+// sharing the pages as under SHARED, and writes the output itself: no partials, no second kernel, and
+// the table row is read beside the length instead of after it.
+enum SplitMode { kSplit = 0, kShared = 1, kDirect = 2 };
+template <int DT, int D, bool APPEND, int MODE>
 __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PER_EU) page16_split_kernel(const DecodeArgs a) {
   constexpr int STEPS = D / 32;  // QK k-steps of 32 dims
   constexpr int DPL = D / 16;    // V dims per lane = P.V output tiles
   constexpr float kTau = 8.f;
-  constexpr int kPipe = D > 128 ? 1 : UKV_PAGE16_PIPE;  // D=256 has no registers for a second page
+  constexpr int kPipe = D > 128 ? 1 : 2;  // register sets (D=256 has no registers for a second page)
 
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
-  const int g = blockIdx.z * (blockDim.x >> 6) + wv;
-  if (g >= a.n_groups) return;  // whole wave leaves; no workgroup barrier below
+  constexpr bool SHARED = MODE != kSplit, DIRECT = MODE == kDirect;
+  const int wg_heads = DIRECT ? 1 : a.n_groups;  // SHARED: KV heads of this workgroup
+  const int sub = SHARED ? __builtin_amdgcn_readfirstlane(wv / wg_heads) : 0;
+  const int subs = DIRECT ? UKV_PAGE16_WAVES : SHARED ? a.subs : 1;
+  const int g = DIRECT ? (int)blockIdx.y : SHARED ? wv - sub * a.n_groups : blockIdx.z * (blockDim.x >> 6) + wv;
+  if (!SHARED && g >= a.n_groups) return;  // whole wave leaves; only SHARED has barriers below
   const int G = a.grid_wgs;
   // Share w of the page list runs on workgroup blockIdx.x = 8 * (w % (G/8)) + w / (G/8): dispatch
   // puts workgroup i on XCD i % 8, so XCD x runs the contiguous shares x*G/8 .. (x+1)*G/8 - 1 and
@@ -228,39 +244,64 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   const bool writer = blockIdx.x == 0 && blockIdx.z == 0 && wv == 0;
 
   // The batch's pages in sequence order form one list of P pages; workgroup w
-  // takes pages [w*P/G, (w+1)*P/G), crossing sequence boundaries as needed.
-  int P = 0;
-  for (int c0 = 0; c0 < a.B; c0 += 64) {
-    const int bb = c0 + lane;
-    P += wave_sum_i32(bb < a.B ? pages_of(a.lens[bb], a.max_blocks) : 0);
-  }
-  const int x0 = (int)(((int64_t)w * P) / G);
-  const int x1 = (int)(((int64_t)(w + 1) * P) / G);
-  if (x0 >= x1 && !writer) return;
-
-  // Exclusive prefix sums of pages per sequence; the sequence holding page x0.
-  int b_first = -1, s_first = 0, carry = 0;
-  for (int c0 = 0; c0 < a.B; c0 += 64) {
-    const int bb = c0 + lane;
-    const int n = bb < a.B ? pages_of(a.lens[bb], a.max_blocks) : 0;
+  // takes pages [w*P/G, (w+1)*P/G), crossing sequence boundaries as needed. Exclusive
+  // prefix sums of pages per sequence give P and the sequence holding page x0. A batch of up
+  // to 64 sequences is scanned once and its lengths stay in the lanes' registers.
+  const bool one = a.B <= 64;  // (uniform)
+  int len_reg = 0, P = 0;
+  uint64_t nonempty = 0;
+  int x0, x1, b_first = -1, s_first = 0;
+  if constexpr (DIRECT) {
+    b_first = blockIdx.x;
+    x0 = 0;
+    x1 = pages_of(a.lens[b_first], a.max_blocks);
+  } else if (one) {
+    len_reg = lane < a.B ? clamp_len(a.lens[lane], a.max_blocks) : 0;
+    const int n = (len_reg + 15) >> 4;
     const int incl = wave_inclusive_scan_i32(n);
-    const int start = carry + incl - n;
-    if (writer && bb < a.B) {
-      a.seq_start[bb] = start;
-      a.seq_pages[bb] = n;
+    P = __builtin_amdgcn_readlane(incl, 63);
+    nonempty = __ballot(n > 0);
+    if (writer && lane < a.B) {
+      a.seq_start[lane] = incl - n;
+      a.seq_pages[lane] = n;
     }
-    if (b_first < 0) {
-      const uint64_t hit = __ballot(n > 0 && start + n > x0);
-      if (hit) {
-        const int l = __builtin_ctzll(hit);
-        b_first = c0 + l;
-        s_first = __builtin_amdgcn_readlane(start, l);
-        if (!writer) break;
+    x0 = mul_div(w, P, G);
+    x1 = mul_div(w + 1, P, G);
+    if (x0 >= x1) return;
+    b_first = __builtin_ctzll(__ballot(n > 0 && incl > x0));
+    s_first = __builtin_amdgcn_readlane(incl - n, b_first);
+  } else {
+    for (int c0 = 0; c0 < a.B; c0 += 64) {
+      const int bb = c0 + lane;
+      P += __builtin_amdgcn_readlane(wave_inclusive_scan_i32(bb < a.B ? pages_of(a.lens[bb], a.max_blocks) : 0), 63);
+    }
+    x0 = mul_div(w, P, G);
+    x1 = mul_div(w + 1, P, G);
+    if (x0 >= x1 && !writer) return;
+    int carry = 0;
+    for (int c0 = 0; c0 < a.B; c0 += 64) {
+      const int bb = c0 + lane;
+      const int n = bb < a.B ? pages_of(a.lens[bb], a.max_blocks) : 0;
+      const int incl = wave_inclusive_scan_i32(n);
+      const int start = carry + incl - n;
+      if (writer && bb < a.B) {
+        a.seq_start[bb] = start;
+        a.seq_pages[bb] = n;
       }
+      if (b_first < 0) {
+        const uint64_t hit = __ballot(n > 0 && start + n > x0);
+        if (hit) {
+          const int l = __builtin_ctzll(hit);
+          b_first = c0 + l;
+          s_first = __builtin_amdgcn_readlane(start, l);
+          if (!writer) break;
+        }
+      }
+      carry += __builtin_amdgcn_readlane(incl, 63);
     }
-    carry += __builtin_amdgcn_readlane(incl, 63);
+    if (x0 >= x1) return;
   }
-  if (x0 >= x1) return;
+  (void)P;
 
   const int i16 = lane & 15;
   const int kg = lane >> 4;
@@ -276,6 +317,9 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   constexpr int KP = D + 16;
   __shared__ __attribute__((aligned(16))) uint16_t k_lds[UKV_PAGE16_WAVES][16 * KP];
   uint16_t* ks = k_lds[wv];
+  // SHARED: the waves' partial rows and (m, l) of a segment.
+  __shared__ __attribute__((aligned(16))) float part_lds[SHARED ? UKV_PAGE16_WAVES * 16 * D : 4];
+  __shared__ float2 ml_lds[SHARED ? UKV_PAGE16_WAVES * 16 : 1];
   const uint16_t* vbase = a.v + (int64_t)(4 * kg) * a.v_st + (int64_t)g * a.v_sh + DPL * i16;
 
   // Per-segment state (one sequence's share of this workgroup's pages).
@@ -284,7 +328,8 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   int pa = 0;        // first page of the segment (within the sequence)
   int pb = 0;        // one past the last page
   const int32_t* btrow = nullptr;
-  int bid_win = 0;   // page ids pa + 64*k + lane of the current 64-page window
+  int n_mine = 0;    // pages of the segment this wave takes: pa + sub + i * subs, i < n_mine
+  int bid_win = 0;   // ids of this wave's pages 64*k + lane of the current 64-page window
   int tail_page = -1;  // APPEND: page of the decode token if this segment holds it, else -1
   int tail_slot = 0;   // APPEND: its slot in that page
   int tail_pid = -1;   // APPEND: that page's id, -1 if invalid
@@ -296,9 +341,12 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   float lsum;        // this lane's share of that head's sum of weights
   f32x4 acc[DPL];
 
-  auto load_page = [&](int p, VRow<DPL> (&kr)[4], VRow<DPL> (&vr)[4], int& nv) {
-    const int idx = p - pa;
-    if (idx != 0 && (idx & 63) == 0) bid_win = (p + lane < pb) ? btrow[p + lane] : 0;
+  auto page_window = [&](int i0) {
+    bid_win = i0 + lane < n_mine ? btrow[SHARED ? pa + sub + (i0 + lane) * subs : pa + i0 + lane] : 0;
+  };
+  auto load_page = [&](int idx, VRow<DPL> (&kr)[4], VRow<DPL> (&vr)[4], int& nv) {
+    const int p = SHARED ? pa + sub + idx * subs : pa + idx;
+    if (!DIRECT && idx != 0 && (idx & 63) == 0) page_window(idx);
     int bid = __builtin_amdgcn_readlane(bid_win, idx & 63);
     const bool ok = (unsigned)bid < (unsigned)a.num_pages;
     if constexpr (APPEND)
@@ -391,16 +439,21 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   int seg_start = s_first;  // global index of page 0 of sequence b
   int x = x0;
   while (true) {
-    const int n_b = pages_of(a.lens[b], a.max_blocks);
-    L = clamp_len(a.lens[b], a.max_blocks);
+    L = one && !DIRECT ? __builtin_amdgcn_readlane(len_reg, b) : clamp_len(a.lens[b], a.max_blocks);
+    const int n_b = (L + 15) >> 4;
     pa = x - seg_start;
     pb = min(x1, seg_start + n_b) - seg_start;
+    n_mine = SHARED ? max(0, pb - pa - sub + subs - 1) / subs : pb - pa;
     btrow = a.bt + (int64_t)b * a.max_blocks;
-    bid_win = (pa + lane < pb) ? btrow[pa + lane] : 0;
+    if constexpr (DIRECT)  // (not after the length: columns past it are inside the row and unused)
+      bid_win = sub + lane * subs < a.max_blocks ? btrow[sub + lane * subs] : 0;
+    else
+      page_window(0);
     if constexpr (APPEND) {
       // A length beyond the table is clamped; its token has no slot and is not written.
       tail_page = (L > 0 && L == a.lens[b]) ? ((L - 1) >> 4) : -1;
       if (tail_page < pa || tail_page >= pb) tail_page = -1;  // another workgroup's page
+      if (SHARED && tail_page >= 0 && (tail_page - pa) % subs != sub) tail_page = -1;  // another wave's
       tail_pid = -1;
       if (tail_page >= 0) {
         tail_slot = (L - 1) & 15;
@@ -420,21 +473,48 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
 #pragma unroll
     for (int e = 0; e < DPL; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Software pipeline over PIPE register sets: while page p is reduced, the
-    // loads of pages p+1 .. p+PIPE-1 are in flight.
+    auto reduce = [&](int i, VRow<DPL> (&kr)[4], VRow<DPL> (&vr)[4], int nv) {
+      if constexpr (APPEND)
+        if ((SHARED ? pa + sub + i * subs : pa + i) == tail_page) swap_in_token(kr, vr);
+      process_page(kr, vr, nv);
+    };
+    if constexpr (DIRECT) {
+      // Page i + 1 is in flight while page i is reduced: every load of the loop is unconditional, so
+      // that the compiler's waits count loads of known age (8 % faster at 256 tokens than the loop
+      // below, where the prefetch's branch makes them wait for it too; long segments, whose waves
+      // saturate HBM, are 2 % faster with that one).
+      constexpr int B1 = kPipe - 1;
+      if (n_mine > 0) {
+        load_page(0, kb[0], vb[0], nvb[0]);
+        int i = 0;
+        for (; i + 2 < n_mine; i += 2) {
+          load_page(i + 1, kb[B1], vb[B1], nvb[B1]);
+          reduce(i, kb[0], vb[0], nvb[0]);
+          load_page(i + 2, kb[0], vb[0], nvb[0]);
+          reduce(i + 1, kb[B1], vb[B1], nvb[B1]);
+        }
+        if (i + 1 < n_mine) {
+          load_page(i + 1, kb[B1], vb[B1], nvb[B1]);
+          reduce(i, kb[0], vb[0], nvb[0]);
+          reduce(i + 1, kb[B1], vb[B1], nvb[B1]);
+        } else {
+          reduce(i, kb[0], vb[0], nvb[0]);
+        }
+      }
+    } else {
+      // Register sets in turn: the loads of page i + kPipe - 1 are issued before page i is reduced.
 #pragma unroll
-    for (int i = 0; i < kPipe - 1; ++i)
-      if (pa + i < pb) load_page(pa + i, kb[i], vb[i], nvb[i]);
-    for (int base = pa; base < pb; base += kPipe) {
+      for (int i = 0; i < kPipe - 1; ++i)
+        if (i < n_mine) load_page(i, kb[i], vb[i], nvb[i]);
+      for (int base = 0; base < n_mine; base += kPipe) {
 #pragma unroll
-      for (int u = 0; u < kPipe; ++u) {
-        const int p = base + u;
-        if (p < pb) {
-          const int nxt = (u + kPipe - 1) % kPipe;  // constant after unrolling
-          if (p + kPipe - 1 < pb) load_page(p + kPipe - 1, kb[nxt], vb[nxt], nvb[nxt]);
-          if constexpr (APPEND)
-            if (p == tail_page) swap_in_token(kb[u], vb[u]);
-          process_page(kb[u], vb[u], nvb[u]);
+        for (int u = 0; u < kPipe; ++u) {
+          const int i = base + u;
+          if (i < n_mine) {
+            const int nxt = (u + kPipe - 1) % kPipe;  // constant after unrolling
+            if (i + kPipe - 1 < n_mine) load_page(i + kPipe - 1, kb[nxt], vb[nxt], nvb[nxt]);
+            reduce(i, kb[u], vb[u], nvb[u]);
+          }
         }
       }
     }
@@ -460,36 +540,76 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
     for (int r = 0; r < 4; ++r) {
       const int h = 4 * kg + r;
       if (h < n_here) {
-        f32x4* dst = reinterpret_cast<f32x4*>(a.part_o + (slot + h) * D + DPL * i16);
+        f32x4* dst = reinterpret_cast<f32x4*>(SHARED ? part_lds + (wv * 16 + h) * D + DPL * i16
+                                                     : a.part_o + (slot + h) * D + DPL * i16);
 #pragma unroll
         for (int c = 0; c < DPL / 4; ++c)
           dst[c] = f32x4{acc[4 * c][r], acc[4 * c + 1][r], acc[4 * c + 2][r], acc[4 * c + 3][r]} * kUnscale;
       }
     }
-    if (kg == 0 && live) a.part_ml[slot + i16] = make_float2(m_ref, lcol);
+    if (kg == 0 && live) (SHARED ? ml_lds + wv * 16 : a.part_ml + slot)[i16] = make_float2(m_ref, lcol);
+    if constexpr (SHARED) {
+      // The head's waves add their rows up, each 64 * subs-th float4 of the n_here rows, and write
+      // the segment's partial. (Every wave of the workgroup walks the same segments.)
+      __syncthreads();
+      for (int it = sub * 64 + lane; it < n_here * (D / 4); it += 64 * subs) {
+        const int h = it / (D / 4), dq = it % (D / 4);
+        float M = kNegFltMax;
+        const int gl = DIRECT ? 0 : g;
+        for (int s = 0; s < subs; ++s) M = fmaxf(M, ml_lds[(s * wg_heads + gl) * 16 + h].x);
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        float l = 0.f;
+        for (int s = 0; s < subs; ++s) {
+          const int sw = s * wg_heads + gl;
+          const float2 ml = ml_lds[sw * 16 + h];
+          const float f = fast_exp2(ml.x - M);
+          sum += f * *reinterpret_cast<const f32x4*>(part_lds + (sw * 16 + h) * D + 4 * dq);
+          l += f * ml.y;
+        }
+        if constexpr (DIRECT) {  // (a sequence without keys: 0 / 0)
+          const uint32_t o01 = Elem<DT>::from_float(sum[0] / l) | (uint32_t)Elem<DT>::from_float(sum[1] / l) << 16;
+          const uint32_t o23 = Elem<DT>::from_float(sum[2] / l) | (uint32_t)Elem<DT>::from_float(sum[3] / l) << 16;
+          *reinterpret_cast<u32x2*>(a.out + ((int64_t)b * a.Hq + qh0 + h) * D + 4 * dq) = u32x2{o01, o23};
+        } else {
+          *reinterpret_cast<f32x4*>(a.part_o + (slot + h) * D + 4 * dq) = sum;
+          if (dq == 0) a.part_ml[slot + h] = make_float2(M, l);
+        }
+      }
+      if constexpr (DIRECT) break;
+      __syncthreads();  // read before the next segment's rows
+    }
 
     x = seg_start + pb;
     if (x >= x1) break;
     seg_start += n_b;
-    ++b;
-    while (b < a.B && pages_of(a.lens[b], a.max_blocks) == 0) ++b;  // empty sequences hold no page
-    if (b >= a.B) break;  // unreachable while x1 <= P; keeps every read inside the batch
+    ++b;  // the next sequence with pages; past the batch only unreachably (x1 <= P)
+    if (one) {
+      const uint64_t rest = b < 64 ? nonempty >> b : 0;
+      if (rest == 0) break;
+      b += __builtin_ctzll(rest);
+    } else {
+      while (b < a.B && pages_of(a.lens[b], a.max_blocks) == 0) ++b;
+      if (b >= a.B) break;
+    }
   }
 }
 
-__device__ __forceinline__ float block_reduce_256(float x, float* red, bool is_max) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float y = __shfl_xor(x, o);
-    x = is_max ? fmaxf(x, y) : x + y;
-  }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
-  __syncthreads();
-  float r = red[0];
-#pragma unroll
-  for (int w = 1; w < 4; ++w) r = is_max ? fmaxf(r, red[w]) : r + red[w];
-  __syncthreads();
-  return r;
+// Maximum / sum over the wave's 64 lanes, in every lane (the steps of wave_inclusive_scan_i32).
+#define UKV_WAVE_REDUCE(x, op, old)                                                                        \
+  x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(old, __float_as_int(x), 0x111, 0xf, 0xf, false))); \
+  x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(old, __float_as_int(x), 0x112, 0xf, 0xf, false))); \
+  x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(old, __float_as_int(x), 0x114, 0xf, 0xf, false))); \
+  x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(old, __float_as_int(x), 0x118, 0xf, 0xf, false))); \
+  x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(old, __float_as_int(x), 0x142, 0xa, 0xf, false))); \
+  x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(old, __float_as_int(x), 0x143, 0xc, 0xf, false)));
+__device__ __forceinline__ float wave_max(float x) {
+  UKV_WAVE_REDUCE(x, fmaxf, (int)0xff800000)  // -inf
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+__device__ __forceinline__ float add_f32(float x, float y) { return x + y; }
+__device__ __forceinline__ float wave_sum(float x) {
+  UKV_WAVE_REDUCE(x, add_f32, 0)
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
 
 // Merges the partials of one (sequence, q head): log-sum-exp in log2 units.
@@ -497,32 +617,36 @@ __device__ __forceinline__ float block_reduce_256(float x, float* red, bool is_m
 // workgroups w = floor(((S+1)G - 1)/P) .. floor(((S+n)G - 1)/P), whose partials
 // sit in slots w + b. 256 threads: thread (cs, dq) owns float4 dims 4*dq.. of
 // partials cs, cs+CS, ...; it issues the loads of its first kPre rows together
-// with the (m, l) loads, so that one memory round trip serves both; the weights
-// are computed once into LDS, and the CS partial sums meet in LDS.
+// with the (m, l) loads, so that one memory round trip serves both. Every wave computes
+// all the weights itself, with register reductions, and reads back what it wrote to LDS
+// (every wave writes the same values): the one barrier is the CS partial sums' meeting in LDS.
 template <int DT, int D>
 __global__ void __launch_bounds__(256) page16_combine_kernel(const DecodeArgs a) {
   constexpr int TD = D / 4;       // threads per partial row (float4 each)
   constexpr int CS = 256 / TD;    // chunk groups
   constexpr int kPre = 4;         // partial rows per thread loaded before the weights
-  extern __shared__ float w_s[];  // [grid_wgs] weights, then [CS][D] sums
-  __shared__ float red[4];
+  extern __shared__ float sums[];  // [CS][D] sums, then [grid_wgs] weights
 
   const int h = blockIdx.x;
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int n_pages = a.seq_pages[b];
-  const int64_t P = (int64_t)a.seq_start[a.B - 1] + a.seq_pages[a.B - 1];
-  const int64_t S = a.seq_start[b];
+  const int P = a.seq_start[a.B - 1] + a.seq_pages[a.B - 1];
+  const int S = a.seq_start[b];
   const int G = a.grid_wgs;
-  const int w_first = n_pages > 0 ? (int)(((S + 1) * G - 1) / P) : 0;
-  const int w_last = n_pages > 0 ? (int)(((S + n_pages) * G - 1) / P) : -1;
+  auto share_of = [&](int x) -> int {  // floor(((x + 1) G - 1) / P): the share holding page x
+    const uint64_t p = (uint64_t)(uint32_t)(x + 1) * (uint32_t)G - 1;
+    return (p >> 32) == 0 ? (int)((uint32_t)p / (uint32_t)P) : (int)(p / (uint32_t)P);
+  };
+  const int w_first = n_pages > 0 ? share_of(S) : 0;
+  const int w_last = n_pages > 0 ? share_of(S + n_pages - 1) : -1;
   const int n_chunks = w_last - w_first + 1;
   const int64_t base = (int64_t)(w_first + b) * a.Hq + h;
   // With fewer pages than workgroups (P < G) some workgroups in [w_first, w_last]
   // own no page and wrote no partial: their slots hold stale data and are skipped.
   auto owns_pages = [&](int c) {
-    const int64_t w = w_first + c;
-    return ((w + 1) * P) / G > (w * P) / G;
+    const int w = w_first + c;
+    return P >= G || mul_div(w + 1, P, G) > mul_div(w, P, G);
   };
 
   const int cs = tid / TD;
@@ -535,26 +659,31 @@ __global__ void __launch_bounds__(256) page16_combine_kernel(const DecodeArgs a)
     const int c = cs + k * CS;
     rows[k] = c < n_chunks ? *reinterpret_cast<const f32x4*>(po + (int64_t)c * cstride) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const bool own0 = tid < n_chunks && owns_pages(tid);
-  const float2 ml0 = own0 ? a.part_ml[base + (int64_t)tid * a.Hq] : make_float2(-INFINITY, 0.f);
+  const int lane = tid & 63;
+  float* w_s = sums + CS * D;
+  const bool own0 = lane < n_chunks && owns_pages(lane);
+  const float2 ml0 = own0 ? a.part_ml[base + (int64_t)lane * a.Hq] : make_float2(-INFINITY, 0.f);
 
   float mx = ml0.x;
-  for (int c = tid + 256; c < n_chunks; c += 256)
+  for (int c = lane + 64; c < n_chunks; c += 64)
     if (owns_pages(c)) mx = fmaxf(mx, a.part_ml[base + (int64_t)c * a.Hq].x);
-  const float M = block_reduce_256(mx, red, true);
+  const float M = wave_max(mx);
   float dsum = 0.f;
-  for (int c = tid; c < n_chunks; c += 256) {
-    const bool own = c == tid ? own0 : owns_pages(c);
+  for (int c = lane; c < n_chunks; c += 64) {
+    const bool own = c == lane ? own0 : owns_pages(c);
     if (!own) {
       w_s[c] = -1.f;  // marks an empty slot (real weights are >= 0 or NaN)
       continue;
     }
-    const float2 ml = c == tid ? ml0 : a.part_ml[base + (int64_t)c * a.Hq];
+    const float2 ml = c == lane ? ml0 : a.part_ml[base + (int64_t)c * a.Hq];
     const float w = exp2f(ml.x - M);
     w_s[c] = w;
     dsum += ml.y * w;
   }
-  const float den = block_reduce_256(dsum, red, false);  // also orders the w_s writes
+  const float den = wave_sum(dsum);
+  // the wave's own LDS writes, by other lanes, before the reads below
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -570,7 +699,6 @@ __global__ void __launch_bounds__(256) page16_combine_kernel(const DecodeArgs a)
     const float w = w_s[c];
     if (!(w < 0.f)) acc += w * *reinterpret_cast<const f32x4*>(po + (int64_t)c * cstride);
   }
-  float* sums = w_s + ((a.grid_wgs + 3) & ~3);
   *reinterpret_cast<f32x4*>(sums + cs * D + 4 * dq) = acc;
   __syncthreads();
   if (tid < D) {
@@ -639,7 +767,7 @@ __global__ void __launch_bounds__(256) page16_scalar_kernel(const DecodeArgs a) 
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr int kMinPagesPerWg = 8;  // below this a workgroup's setup outweighs its pages
+constexpr int kMinPagesPerWg = 4;  // below this a workgroup's setup outweighs its pages
 
 // CU count of the current device, cached per device id (0 = not yet read; a
 // racing first read stores the same value twice).
@@ -669,13 +797,31 @@ int env_wgs() {
 
 // Workgroups G sharing the batch's pages: one per CU (a single round of equal
 // workgroups measured fastest), fewer when even the largest possible batch
-// (batch * max_blocks pages) gives each fewer than kMinPagesPerWg pages;
-// UKV_PAGE16_WGS overrides it for launch-shape sweeps.
-int split_wgs_for(int batch, int max_blocks) {
+// (batch * max_blocks pages) gives each fewer than kMinPagesPerWg pages, but one per sequence (a
+// workgroup takes its segments one after another); a multiple of 8 for the XCDs' equal runs. Four
+// sequences of 256-2048 tokens: 12.7 us with 4 pages, 16.1 with 8, 15.4 with 2. Partials
+// beyond kMaxPartials bytes keep the coarser rule. UKV_PAGE16_WGS overrides it for launch-shape sweeps.
+constexpr size_t kMaxPartials = size_t(16) << 20;
+int split_wgs_for(int batch, int hq, int d, int max_blocks) {
   if (const int v = env_wgs()) return v;
   const long long bound = (long long)batch * (long long)std::max(max_blocks, 1);
-  const long long g = std::min<long long>(device_cu_count(), (bound + kMinPagesPerWg - 1) / kMinPagesPerWg);
-  return (int)std::max<long long>(1, g);
+  const long long cus = device_cu_count();
+  const long long coarse = std::max<long long>(1, std::min(cus, (bound + 7) / 8));
+  const long long want = std::max<long long>((bound + kMinPagesPerWg - 1) / kMinPagesPerWg, batch);
+  const long long g = std::max(coarse, std::min(cus, (want + 7) / 8 * 8));
+  const bool fits = (size_t)(g + batch) * hq * (d + 2) * sizeof(float) <= kMaxPartials;
+  return (int)(fits ? g : coarse);
+}
+
+// kDirect: a CU streams at most ~47 GB/s (32 KB in flight against ~0.7 us), so a sequence on one
+// workgroup per KV head pays only while its pages are few: per layer of a step at 512 tokens 7-10 us
+// against 9-13 (1-8 sequences) and 14.5 / 24.7 against 19.4 / 29.3 us (32 / 64 sequences, 8 KV heads); at
+// 1024 it wins where the (sequence, head) pairs fill half of the CUs (24.9 / 44.0 against 28.7 / 48.8 us)
+// and loses below (15.7 against 14.3 us at 8 x 8, 11.4 against 9.4 at 8 x 1).
+constexpr int kDirectPages = 32, kDirectPagesWide = 64;
+bool direct_shape(int batch, int n_groups, int head_dim, int max_blocks) {
+  if (head_dim > 128 || n_groups > 65535 || env_wgs()) return false;
+  return max_blocks <= ((long long)batch * n_groups >= device_cu_count() / 2 ? kDirectPagesWide : kDirectPages);
 }
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -689,7 +835,7 @@ struct WorkspaceLayout {
 // starts and counts; slots = G + batch.
 WorkspaceLayout workspace_layout(int batch, int hq, int d, int max_blocks) {
   WorkspaceLayout w{};
-  w.wgs = split_wgs_for(batch, max_blocks);
+  w.wgs = split_wgs_for(batch, hq, d, max_blocks);
   const size_t slots = ((size_t)w.wgs + (size_t)batch) * hq;
   w.part_o_off = 0;
   w.part_ml_off = align256(slots * d * sizeof(float));
@@ -702,18 +848,39 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 template <int DT, int D>
 void launch_split(const DecodeArgs& a, hipStream_t stream) {
+  // Waves left over by the KV heads share the heads' pages (D = 256 has no LDS for their rows).
+  if constexpr (D <= 128) {
+    if (direct_shape(a.B, a.n_groups, a.D, a.max_blocks)) {
+      const dim3 grid(a.B, a.n_groups), block(64 * UKV_PAGE16_WAVES);
+      if (a.k_new)
+        hipLaunchKernelGGL((page16_split_kernel<DT, D, true, kDirect>), grid, block, 0, stream, a);
+      else
+        hipLaunchKernelGGL((page16_split_kernel<DT, D, false, kDirect>), grid, block, 0, stream, a);
+      return;
+    }
+    if (a.n_groups <= UKV_PAGE16_WAVES / 2) {
+      DecodeArgs s = a;
+      for (s.subs = 2; 2 * s.subs * a.n_groups <= UKV_PAGE16_WAVES;) s.subs *= 2;
+      const dim3 grid(a.grid_wgs), block(64 * s.subs * a.n_groups);
+      if (a.k_new)
+        hipLaunchKernelGGL((page16_split_kernel<DT, D, true, kShared>), grid, block, 0, stream, s);
+      else
+        hipLaunchKernelGGL((page16_split_kernel<DT, D, false, kShared>), grid, block, 0, stream, s);
+      return;
+    }
+  }
   const int waves = std::min(UKV_PAGE16_WAVES, a.n_groups);
   const dim3 grid(a.grid_wgs, 1, (a.n_groups + waves - 1) / waves);
   if (a.k_new)
-    hipLaunchKernelGGL((page16_split_kernel<DT, D, true>), grid, dim3(64 * waves), 0, stream, a);
+    hipLaunchKernelGGL((page16_split_kernel<DT, D, true, kSplit>), grid, dim3(64 * waves), 0, stream, a);
   else
-    hipLaunchKernelGGL((page16_split_kernel<DT, D, false>), grid, dim3(64 * waves), 0, stream, a);
+    hipLaunchKernelGGL((page16_split_kernel<DT, D, false, kSplit>), grid, dim3(64 * waves), 0, stream, a);
 }
 
 template <int DT>
 void launch_combine_dt(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid(a.Hq, a.B);
-  const size_t lds = (size_t)(((a.grid_wgs + 3) & ~3) + 256 * 4) * sizeof(float);
+  const size_t lds = (size_t)(a.grid_wgs + 256 * 4) * sizeof(float);
   switch (a.D) {
     case 64: hipLaunchKernelGGL((page16_combine_kernel<DT, 64>), grid, dim3(256), lds, stream, a); break;
     case 128: hipLaunchKernelGGL((page16_combine_kernel<DT, 128>), grid, dim3(256), lds, stream, a); break;
@@ -839,7 +1006,7 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
         dtype == UKV_DTYPE_BF16 ? dispatch_split<UKV_DTYPE_BF16>(a, stream) : dispatch_split<UKV_DTYPE_F16>(a, stream);
     if (!launched) return UKV_ERR_LAUNCH;
     if (hipGetLastError() != hipSuccess) return UKV_ERR_LAUNCH;
-    launch_combine(a, dtype, stream);
+    if (!direct_shape(batch, n_groups, head_dim, max_blocks)) launch_combine(a, dtype, stream);
   } else {
     const dim3 grid(num_q_heads, batch);
     if (dtype == UKV_DTYPE_BF16)
