@@ -45,7 +45,8 @@
 //     (query, head) pairs laid end to end, so every column of the matrix cores is used, V keeps its
 //     type and P goes in as two 16-bit parts (fp32-grade weights, as the scalar kernel they ran on
 //     before had): 28 q heads on 4 KV heads, 4 x 512 queries over 0.5-8K keys in 0.33 ms against
-//     72.7 ms; twelve 64-dim prompts of 16-700 tokens in 0.10 ms against 6.4 ms;
+//     72.7 ms; twelve 64-dim prompts of 16-700 tokens in 0.055 ms against 6.4 ms (0.10 ms with one
+//     workgroup per CU, three column blocks, 64-key tiles and the pairs' blocks in turn);
 //   * key parts: a launch of few query blocks leaves CUs idle however long its prefix. Its keys are
 //     then cut into equal parts, each (block, part) a workgroup, and a merge kernel adds the parts
 //     up: one 389-query chunk behind 32256 keys (40 blocks) in 0.23 ms against 0.86 ms;
@@ -90,6 +91,9 @@ struct PrefillArgs {
   // prefill_combine_kernel merges the parts' (m, l, O) from part_o / part_ml, rows
   // [part][query row][q head] of D floats / one float2.
   int n_parts, part_tiles;
+  // Work items in block order (block j of every pair, then block j + 1) instead of pair after pair: for
+  // launches whose blocks see very different key counts, longest first.
+  int by_block;
   int total_q;
   float* part_o;
   float2* part_ml;
@@ -129,6 +133,9 @@ __device__ __forceinline__ uint32_t bf16x2_to_f16x2(uint32_t w) {
 // loaded registers follow the wait.
 __device__ __forceinline__ void gload16(u32x4& r, const void* p) {
   asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(r) : "v"(p));
+}
+template <int N> __device__ __forceinline__ void vm_wait(u32x4& x) {
+  asm volatile("s_waitcnt vmcnt(%1)" : "+v"(x) : "n"(N));
 }
 template <int N> __device__ __forceinline__ void vm_wait(u32x4& x, u32x4& y) {
   asm volatile("s_waitcnt vmcnt(%2)" : "+v"(x), "+v"(y) : "n"(N));
@@ -238,13 +245,12 @@ __device__ void flag_obs_rows(const PrefillArgs& a, int b, int g, int C, int lo,
   }
 }
 
-// LDS of one workgroup: kStages ring slots of K and V (fp16, or the pool's type) tiles. At D = 64 a
-// tile is 64 keys, so that every thread still loads one 16-byte chunk of K and one of V per tile
-// or more; the row pitch D + 16 elements keeps the bank pattern (a multiple of 8 banks per row).
+// LDS of one workgroup: kStages ring slots of K and V (fp16, or the pool's type) tiles. The 144-byte
+// pitch at D = 64 spreads eight rows' 16-byte reads over the banks and lets two workgroups share a CU.
 template <int D> struct PrefillLds {
-  static constexpr int kKeys = kTileKeys * 128 / D;
-  __attribute__((aligned(16))) uint16_t k_s[kStages][kKeys][kRowPad - 128 + D];
-  __attribute__((aligned(16))) uint16_t v_s[kStages][kKeys][kVRowPad - 128 + D];
+  static constexpr int kPitch = D == 64 ? 72 : kRowPad, kVPitch = D == 64 ? 72 : kVRowPad;
+  __attribute__((aligned(16))) uint16_t k_s[kStages][kTileKeys][kPitch];
+  __attribute__((aligned(16))) uint16_t v_s[kStages][kTileKeys][kVPitch];
 };
 
 // Softmax weights for P.V on 16-bit MFMAs with fp32-grade precision: p ~= hi + lo, both in V's
@@ -266,8 +272,10 @@ template <> struct PrefillSplit<UKV_DTYPE_F16> {
   static constexpr uint32_t kOnes = 0x3C003C00u;
   static __device__ __forceinline__ void split(float x0, float x1, uint32_t& hi, uint32_t& lo) {
     hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0 - Elem<UKV_DTYPE_F16>::lo(hi),
-                                                                 x1 - Elem<UKV_DTYPE_F16>::hi(hi)));
+    // lo = fp16(x - hi): one mixed-precision FMA per weight (a subtraction of the converted halves
+    // and a pack are five instructions; the compiler does not form these two)
+    asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(x0));
+    asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(x1));
   }
 };
 
@@ -289,15 +297,17 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   constexpr int STEPS = D / 32;
   constexpr int NE = D / 16;  // output tiles of 16 dims
   constexpr int NT = 64 * WAVES;
-  constexpr int TK = PrefillLds<D>::kKeys;  // keys per tile
-  constexpr int PPT = TK / 16;              // pages per tile
-  constexpr int CH = D / 8;                 // 16-byte chunks per key row
-  constexpr int ITEMS = TK * CH / NT;       // 16-byte chunks per thread per tensor per tile
+  constexpr int TK = kTileKeys;  // keys per tile
+  constexpr int PPT = TK / 16;   // pages per tile
+  constexpr int CH = D / 8;      // 16-byte chunks per key row
+  // A thread loads one 16-byte chunk of K and one of V per tile or, HALF (D = 64), one of either: the
+  // lower half of the waves takes K.
+  constexpr bool HALF = 2 * TK * CH == NT;
   constexpr int PVT = FINE ? DT : (int)UKV_DTYPE_F16;  // type of the P.V operands
   constexpr float kTau = 8.f;
   constexpr float kLift = FINE ? PrefillSplit<DT>::kLift : 0.f;
   constexpr bool kConvert = DT == UKV_DTYPE_BF16 && !FINE;  // the loader converts V to fp16
-  static_assert(ITEMS * NT == TK * CH, "loader mapping");
+  static_assert(HALF || TK * CH == NT, "loader mapping");
   auto& k_s = lds.k_s;
   auto& v_s = lds.v_s;
 
@@ -376,7 +386,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     for (int e = 0; e < NE; ++e) o[cb][e] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // ---- tile loader: chunk idx = tid + i * NT is 16-byte chunk idx % CH of key row idx / CH.
+  // ---- tile loader: thread idx takes 16-byte chunk idx % CH of key row idx / CH.
   // Tile u is loaded into register set u & 1 four tiles ahead, written into
   // ring slot u % 4 two tiles ahead (zeroing rows past the sequence or on an
   // invalid page and converting a bf16 V to fp16), and computed at tile u.
@@ -388,74 +398,66 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   auto page_id = [&](int pg) -> int { return pg < n_pg ? btrow[pg] : -1; };
   auto page_ok = [&](int id) -> bool { return (unsigned)id < (unsigned)a.num_pages; };
   // Within a page, this thread's chunk sits at a fixed offset; the page base is wave-uniform.
-  uint32_t koff[ITEMS], voff[ITEMS];
-  int lds_row[ITEMS], lds_ch[ITEMS];
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    const int idx = tid + i * NT;
-    const int tok = (idx / CH) & 15, ch = idx % CH;
-    koff[i] = (uint32_t)(tok * a.k_st + g * a.k_sh + 8 * ch);
-    voff[i] = (uint32_t)(tok * a.v_st + g * a.v_sh + 8 * ch);
-    lds_row[i] = idx / CH;
-    lds_ch[i] = ch;
-  }
-  u32x4 rk0[ITEMS], rv0[ITEMS], rk1[ITEMS], rv1[ITEMS];
-  // the page of chunk i of this thread among a tile's PPT (rows 16 j .. 16 j + 15 are page j); wave-uniform
-  auto chunk_page = [&](int i, const int (&ids)[PPT]) -> int {
-    const int j = __builtin_amdgcn_readfirstlane((tid + i * NT) / (16 * CH));
-    if constexpr (PPT == 2) {
-      return j ? ids[1] : ids[0];
-    } else {
-      const int i0 = ids[0], i1 = ids[1], i2 = ids[2], i3 = ids[3];  // (values: the array stays in registers)
-      return j < 2 ? (j ? i1 : i0) : (j == 2 ? i2 : i3);
-    }
+  const int idx = HALF ? tid & (NT / 2 - 1) : tid;
+  const bool half_v = HALF && wv >= WAVES / 2;  // (wave-uniform) this wave loads V
+  const int lds_row = idx / CH, lds_ch = idx % CH;
+  const int tok = lds_row & 15;
+  const uint32_t koff = (uint32_t)(tok * (half_v ? a.v_st : a.k_st) + g * (half_v ? a.v_sh : a.k_sh) + 8 * lds_ch);
+  const uint32_t voff = (uint32_t)(tok * a.v_st + g * a.v_sh + 8 * lds_ch);
+  const uint16_t* kbase = half_v ? a.v : a.k;
+  const uint32_t k_sp = (uint32_t)(half_v ? a.v_sp : a.k_sp);
+  u32x4 rk0, rv0, rk1, rv1;
+  // the page of this thread's chunk among a tile's two (rows 0-15 and 16-31); wave-uniform
+  auto chunk_page = [&](const int (&ids)[PPT]) -> int {
+    return __builtin_amdgcn_readfirstlane(idx / (16 * CH)) ? ids[1] : ids[0];
   };
-  auto issue = [&](const int (&ids)[PPT], u32x4 (&rk)[ITEMS], u32x4 (&rv)[ITEMS]) {
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      const int id = chunk_page(i, ids);
-      // page strides fit 32 bits (checked on the host): a 32 x 32 -> 64-bit scalar product
-      const uint32_t pg = page_ok(id) ? (uint32_t)id : 0u;
-      gload16(rk[i], a.k + (uint64_t)pg * (uint32_t)a.k_sp + koff[i]);
-      gload16(rv[i], a.v + (uint64_t)pg * (uint32_t)a.v_sp + voff[i]);
-    }
+  auto issue = [&](const int (&ids)[PPT], u32x4& rk, u32x4& rv) {
+    const int id = chunk_page(ids);
+    // page strides fit 32 bits (checked on the host): a 32 x 32 -> 64-bit scalar product
+    const uint32_t pg = page_ok(id) ? (uint32_t)id : 0u;
+    gload16(rk, kbase + (uint64_t)pg * k_sp + koff);
+    if constexpr (!HALF) gload16(rv, a.v + (uint64_t)pg * (uint32_t)a.v_sp + voff);
   };
   // The largest and the smallest fp16 V value this thread stored, over every tile (three-input
   // packed maximum / minimum, which carry a NaN through): checked once after the loop for an
   // inf or NaN, i.e. a bf16 value fp16 cannot hold.
   typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
   hv2 vmax = {0, 0}, vmin = {0, 0};
-  auto store = [&](int u, int slot, const int (&ids)[PPT], u32x4 (&rk)[ITEMS], u32x4 (&rv)[ITEMS]) {
-    bool full = TK * (u + 1) <= Lk;
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) full = full && page_ok(ids[j]);
-    // The other register set's 2 * ITEMS loads were issued after this set's.
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) vm_wait<2 * ITEMS>(rk[i], rv[i]);
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      // (converted before the junk rows are zeroed: the conversion writes new registers, which
-      // the zeroing then selects in place, with no copy of the loaded ones)
-      u32x4 v;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) v[c] = kConvert ? bf16x2_to_f16x2(rv[i][c]) : rv[i][c];
-      if (!full) {  // (wave-uniform) rows past the sequence or on an invalid page hold junk
-        const bool ok = page_ok(chunk_page(i, ids)) && TK * u + lds_row[i] < Lk;
+  auto store = [&](int u, int slot, const int (&ids)[PPT], u32x4& rk, u32x4& rv) {
+    const bool full = page_ok(ids[0]) && page_ok(ids[1]) && TK * (u + 1) <= Lk;
+    // rows past the sequence or on an invalid page hold junk (wave-uniform: the tile has some)
+    auto clear_junk = [&](u32x4& v) {
+      if (!full) {
+        const bool ok = page_ok(chunk_page(ids)) && TK * u + lds_row < Lk;
 #pragma unroll
         for (int c = 0; c < 4; ++c) v[c] = ok ? v[c] : 0u;
       }
-      if constexpr (kConvert) {
-        const uint32_t w0 = v[0], w1 = v[1], w2 = v[2], w3 = v[3];
-        const hv2 c0 = __builtin_bit_cast(hv2, w0), c1 = __builtin_bit_cast(hv2, w1);
-        const hv2 c2 = __builtin_bit_cast(hv2, w2), c3 = __builtin_bit_cast(hv2, w3);
-        vmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(vmax, c0), c1);
-        vmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(vmax, c2), c3);
-        vmin = __builtin_elementwise_minimum(__builtin_elementwise_minimum(vmin, c0), c1);
-        vmin = __builtin_elementwise_minimum(__builtin_elementwise_minimum(vmin, c2), c3);
-      }
-      *reinterpret_cast<u32x4*>(&k_s[slot][lds_row[i]][8 * lds_ch[i]]) = rk[i];
-      *reinterpret_cast<u32x4*>(&v_s[slot][lds_row[i]][8 * lds_ch[i]]) = v;
+    };
+    if constexpr (HALF) {
+      vm_wait<1>(rk);  // the other register set's load was issued after this one's
+      clear_junk(rk);
+      uint16_t* dst = half_v ? &v_s[slot][lds_row][8 * lds_ch] : &k_s[slot][lds_row][8 * lds_ch];
+      *reinterpret_cast<u32x4*>(dst) = rk;
+      return;
     }
+    vm_wait<2>(rk, rv);  // the other register set's two loads were issued after this set's
+    // (converted before the junk rows are zeroed: the conversion writes new registers, which
+    // the zeroing then selects in place, with no copy of the loaded ones)
+    u32x4 v;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = kConvert ? bf16x2_to_f16x2(rv[c]) : rv[c];
+    clear_junk(v);
+    if constexpr (kConvert) {
+      const uint32_t w0 = v[0], w1 = v[1], w2 = v[2], w3 = v[3];
+      const hv2 c0 = __builtin_bit_cast(hv2, w0), c1 = __builtin_bit_cast(hv2, w1);
+      const hv2 c2 = __builtin_bit_cast(hv2, w2), c3 = __builtin_bit_cast(hv2, w3);
+      vmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(vmax, c0), c1);
+      vmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(vmax, c2), c3);
+      vmin = __builtin_elementwise_minimum(__builtin_elementwise_minimum(vmin, c0), c1);
+      vmin = __builtin_elementwise_minimum(__builtin_elementwise_minimum(vmin, c2), c3);
+    }
+    *reinterpret_cast<u32x4*>(&k_s[slot][lds_row][8 * lds_ch]) = rk;
+    *reinterpret_cast<u32x4*>(&v_s[slot][lds_row][8 * lds_ch]) = v;
   };
 
   // Page ids of tiles t .. t+3 (t_id[j] = tile t + j) and of tile t+4.
@@ -481,17 +483,15 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
 
-  // 32-key runs t < n_full end below the sequence end and below every column's diagonal (key
+  // Tiles t < n_full end below the sequence end and below every column's diagonal (key
   // 32t + 31 <= min(Lk - 1, wpos_min)).
   const int n_full = max(0, min(Lk, wpos_min + 1)) / kTileKeys;
   const float sl2 = a.scale_log2;
 
-  // 32 keys at a time: run hf of tile t holds keys t * TK + 32 hf ..
-  auto compute_run = [&](int t, int slot, int hf) __attribute__((always_inline)) {
-    const int run = t * (TK / kTileKeys) + hf, row0 = hf * kTileKeys;
-    const int key0 = run * kTileKeys;
-    const bool pg0 = page_ok(t_id[0][2 * hf]), pg1 = page_ok(t_id[0][2 * hf + 1]);
-    const bool full = pg0 && pg1 && run < n_full;
+  auto compute = [&](int t, int slot) {
+    const int key0 = t * kTileKeys;
+    const bool pg0 = page_ok(t_id[0][0]), pg1 = page_ok(t_id[0][1]);
+    const bool full = pg0 && pg1 && t < n_full;
     // S^T[key][column] for the tile's two 16-key blocks and every column block, masked. (As one
     // inlined function the register allocator keeps the three-column loop within 256 VGPRs with
     // no scratch under the iterative-ILP schedule this file is built with; written out in line,
@@ -503,7 +503,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
         for (int cb = 0; cb < CB; ++cb) sacc[kb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
-          const u32x4 ka = *reinterpret_cast<const u32x4*>(&k_s[slot][row0 + kb * 16 + i16][32 * s + 8 * kg]);
+          const u32x4 ka = *reinterpret_cast<const u32x4*>(&k_s[slot][kb * 16 + i16][32 * s + 8 * kg]);
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb) sacc[kb][cb] = mfma16x16x32<DT>(ka, qv[cb][s], sacc[kb][cb]);
         }
@@ -625,11 +625,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     // key order of P's A operand). ds_read_b64_tr_b16 builds it from row-major
     // V: within each 16-lane group, lane L names 4 dims 4(L%4).. of key row
     // L/4, and lane j receives dim j of the 4 rows.
-    const uint16_t* vlane = &v_s[slot][row0 + 4 * kg + (i16 >> 2)][4 * (i16 & 3)];
+    const uint16_t* vlane = &v_s[slot][4 * kg + (i16 >> 2)][4 * (i16 & 3)];
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const u32x2 lo = ds_read_tr16(vlane + 16 * e);
-      const u32x2 hi = ds_read_tr16(vlane + 16 * (kVRowPad - 128 + D) + 16 * e);
+      const u32x2 hi = ds_read_tr16(vlane + 16 * PrefillLds<D>::kVPitch + 16 * e);
       const u32x4 bv = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) o[cb][e] = mfma16x16x32<PVT>(pa[cb], bv, o[cb][e]);
@@ -644,10 +644,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
       lacc[cb] = mfma16x16x32<PVT>(pa[cb], u32x4{kOnes, kOnes, kOnes, kOnes}, lacc[cb]);
       if constexpr (FINE) lacc[cb] = mfma16x16x32<PVT>(pl[cb], u32x4{kOnes, kOnes, kOnes, kOnes}, lacc[cb]);
     }
-  };
-  auto compute = [&](int t, int slot) __attribute__((always_inline)) {
-#pragma unroll
-    for (int hf = 0; hf < TK / kTileKeys; ++hf) compute_run(t, slot, hf);
   };
 
   // Tile t: (a) tile t+2 from register set t&1 into ring slot (t+2)%4; (b) tile t+4 into that
@@ -686,10 +682,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   else run([](int, int) {});
   // Loads of tiles past the end are still in flight: retire them while their
   // registers are still held, so that nothing else is placed in them first.
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    vm_wait<0>(rk0[i], rv0[i]);
-    vm_wait<0>(rk1[i], rv1[i]);
+  vm_wait<0>(rk0);
+  vm_wait<0>(rk1);
+  if constexpr (!HALF) {
+    vm_wait<0>(rv0);
+    vm_wait<0>(rv1);
   }
 
   // A V the matrix cores got wrong anywhere in this workgroup's keys: its columns again on the fp32
@@ -761,7 +758,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
 template <int DT, int D>
 __global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs a) {
   constexpr int LANES = D / 4, ROWS = 256 / LANES;
-  constexpr int TK = PrefillLds<D>::kKeys;
+  constexpr int TK = kTileKeys;
   const int64_t idx = (int64_t)blockIdx.x * ROWS + threadIdx.x / LANES;
   if (idx >= (int64_t)a.total_q * a.Hq) return;
   const int dq = threadIdx.x % LANES;
@@ -852,8 +849,9 @@ __device__ __forceinline__ bool locate_item(int start, int end, int n, int nl, i
 }
 
 // Column blocks per wave of the wide query blocks (the narrow ones have one fewer): the widest whose
-// accumulators, queries and weights stay in 256 VGPRs.
-constexpr int wide_blocks(bool fine, int d) { return fine && d == 128 ? 2 : 3; }
+// accumulators, queries and weights stay in 256 VGPRs, and in 128 at D = 64, where two workgroups
+// then share a CU and cover each other's first loads (one 96-token prompt 7.5 us against 11.6).
+constexpr int wide_blocks(bool fine, int d) { return fine ? 2 : 3; }
 
 // The range of work items [start, end) of a launch's n_items items that XCD xcd runs: dispatch
 // is round-robin over the 8 XCDs, so the workgroups with blockIdx.x % 8 == xcd run there, and
@@ -875,14 +873,20 @@ __device__ __forceinline__ void xcd_range(int total, int xcd, int& start, int& e
 //
 // With PARTS each block comes n_parts times, the blocks of one part next to each other.
 template <int DT, int D, int WAVES, bool FINE, bool PARTS>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 paged_prefill_kernel(const PrefillArgs a) {
   __shared__ PrefillLds<D> lds;
   constexpr int CB3 = wide_blocks(FINE, D), CB2 = CB3 - 1;
   const int n_items = a.n3 + a.n2, parts = PARTS ? a.n_parts : 1;
   int start, end, pair, j;
-  xcd_range(n_items * parts * a.n_groups * a.B, blockIdx.x & 7, start, end);
+  if (!PARTS && a.by_block) {
+    const int pairs = a.n_groups * a.B;
+    j = blockIdx.x / pairs;
+    pair = blockIdx.x - j * pairs;
+  } else {
+    xcd_range(n_items * parts * a.n_groups * a.B, blockIdx.x & 7, start, end);
   if (!locate_item(start, end, n_items * parts, a.n3 * parts, blockIdx.x >> 3, pair, j)) return;  // (never: the grid holds total)
+  }
   int part = 0;
   if constexpr (PARTS) {
     if (j < a.n3 * parts) {
@@ -1239,77 +1243,87 @@ namespace {
 
 // Block plan of the tiled prefill: the numbers n3 and n2 of wide and narrow query blocks per
 // (sequence, KV group) that cover its chunk's max_chunk queries, and the parts its keys are cut
-// into. A launch runs in rounds of one block per CU; the plan with the shortest predicted launch is
-// taken, modelling every block as streaming equally many keys (a long prefix) at its measured cost
-// relative to a wide block, and each XCD's CUs as taking the XCD's blocks in the kernel's order, each
-// CU the next block once free.
+// into. A launch runs in rounds of one block per slot (CU, or half a CU where two workgroups share
+// one); the plan with the shortest predicted launch is taken, modelling each XCD's slots as taking
+// the XCD's blocks in the kernel's order, each slot the next block once free.
 struct BlockPlan {
   int n3, n2;
   int parts, part_tiles;
 };
 
-// One block's time is item * (cost of its width), plus a fixed start.
-double plan_makespan(int64_t pairs, int n3, int n2, int parts, double item, double start_cost, double narrow,
-                     int cus_per_xcd) {
-  const int n_items = (n3 + n2) * parts, nl = n3 * parts;
+// The launch's predicted time when the blocks of every pair cost cost[0 .. n_items - 1], the first nl
+// of them dispatched before the others.
+double plan_makespan(int64_t pairs, const std::vector<double>& cost, int nl, int slots_per_xcd) {
+  const int n_items = (int)cost.size();
   const int64_t total = pairs * n_items;
   const int64_t per = total / 8, rem = total % 8;
   double worst = 0.0;
-  std::vector<double> order;
   for (int x = 0; x < 8; ++x) {
     const int64_t start = x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per;
     const int64_t end = start + per + (x < rem ? 1 : 0);
-    order.clear();
+    std::priority_queue<double, std::vector<double>, std::greater<double>> slot;
+    for (int c = 0; c < slots_per_xcd; ++c) slot.push(0.0);
     if (end > start)
       for (int pass = 0; pass < 2; ++pass)
         for (int64_t p = start / n_items; p <= (end - 1) / n_items; ++p) {
           const int64_t j0 = std::max<int64_t>(pass ? nl : 0, start - p * n_items);
           const int64_t j1 = std::min<int64_t>(pass ? n_items : nl, end - p * n_items);
-          for (int64_t j = j0; j < j1; ++j) order.push_back(start_cost + item * (j < nl ? 1.0 : narrow));
+          for (int64_t j = j0; j < j1; ++j) {
+            const double t = slot.top() + cost[j];
+            slot.pop();
+            slot.push(t);
+            worst = std::max(worst, t);
+          }
         }
-    std::priority_queue<double, std::vector<double>, std::greater<double>> cu;
-    for (int c = 0; c < cus_per_xcd; ++c) cu.push(0.0);
-    double last = 0.0;
-    for (double c : order) {
-      const double t = cu.top() + c;
-      cu.pop();
-      cu.push(t);
-      last = std::max(last, t);
-    }
-    worst = std::max(worst, last);
   }
   return worst;
 }
 
-// Cost of a narrow block relative to a wide one: single blocks timed over the same 32768 keys.
+// Cost of a narrow block relative to a wide one: single blocks timed over the same 32768 keys (3 and
+// 2 column blocks), and estimated from the instruction counts (2 and 1).
 constexpr double kNarrowCost = 0.79, kNarrowCostFine = 0.62;
-// Key parts: a block's fixed cost (first loads, page ids, the partial's store) and the merge's, in
-// tile times, and the fewest tiles a part is worth starting a block for.
-constexpr double kStartTiles = 4.0, kMergeTiles = 6.0;
+// Key parts: a block's fixed cost (first loads, page ids, the output) and the merge launch, in tile
+// times of a wide block (1.16 us), the bytes of partials merged per tile time (read at 4 TB/s and
+// half of them again for the blocks' stores), and the fewest tiles a part is worth a block for.
+constexpr double kStartTiles = 5.0, kMergeTiles = 4.0, kMergeBytesPerTile = 3.1e6;
 constexpr int kMinPartTiles = 12, kMaxParts = 16;
 
-// max_cols: columns (query, head) of the longest chunk; w2, w3: columns of a narrow and a wide block;
-// tiles: key tiles of the widest table row. Parts are considered where allow_parts and the launch
-// is short of two blocks per CU: there whole blocks leave CUs idle.
-BlockPlan choose_plan(int64_t max_cols, int64_t pairs, int w2, int w3, double narrow, int cus_per_xcd, int tiles,
-                      bool allow_parts) {
-  const int n3_max = (int)((max_cols + w3 - 1) / w3);
-  BlockPlan best{n3_max, 0, 1, std::max(1, tiles)};
+// A launch: pairs of (sequence, KV group) whose longest chunk has max_cols columns (query, head), blocks
+// of w2 / w3 columns, tables of `tiles` key tiles.
+struct PlanShape {
+  int64_t max_cols, pairs, part_row_bytes;  // part_row_bytes: one part's partials of the whole call
+  int w2, w3, n_rep, slots_per_xcd, tiles;
+  double narrow;
+  bool allow_parts;
+};
+
+BlockPlan choose_plan(const PlanShape& f) {
+  const int n3_max = (int)((f.max_cols + f.w3 - 1) / f.w3);
+  BlockPlan best{n3_max, 0, 1, std::max(1, f.tiles)};
   // Large launches run many rounds, where the last one matters little: keep wide blocks.
-  if (pairs * n3_max > (1 << 16) || cus_per_xcd <= 0 || n3_max == 0) return best;
-  const bool parts_ok = allow_parts && tiles >= 2 * kMinPartTiles && pairs * n3_max < 16 * cus_per_xcd;
+  if (f.pairs * n3_max > (1 << 16) || f.slots_per_xcd <= 0 || n3_max == 0) return best;
+  // Parts are considered for launches of few blocks: there whole blocks leave CUs idle.
+  const bool parts_ok = f.allow_parts && f.tiles >= 2 * kMinPartTiles && f.pairs * n3_max < 16 * f.slots_per_xcd;
   static std::mutex mu;
-  static std::map<std::tuple<int64_t, int64_t, int, int, int, int>, BlockPlan> cache;
-  const auto key = std::make_tuple(max_cols, pairs, w2, w3, cus_per_xcd, parts_ok ? tiles : 0);
+  static std::map<std::tuple<int64_t, int64_t, int64_t, int, int, int, int>, BlockPlan> cache;
+  const auto key = std::make_tuple(f.max_cols, f.pairs, parts_ok ? f.part_row_bytes : 0, f.w2, f.n_rep, f.slots_per_xcd,
+                                   parts_ok ? f.tiles : 0);
   std::lock_guard<std::mutex> lock(mu);
   const auto hit = cache.find(key);
   if (hit != cache.end()) return hit->second;
-  auto narrow_blocks = [&](int n3) { return (int)((max_cols - (int64_t)n3 * w3 + w2 - 1) / w2); };
-  double best_t = plan_makespan(pairs, n3_max, 0, 1, 1.0, 0.0, narrow, cus_per_xcd);
+  auto narrow_blocks = [&](int n3) { return (int)((f.max_cols - (int64_t)n3 * f.w3 + f.w2 - 1) / f.w2); };
+  std::vector<double> cost;
+  // Every block as streaming equally many keys (a long prefix).
+  auto flat = [&](int n3, int n2) {
+    cost.assign(n3, 1.0);
+    cost.insert(cost.end(), n2, f.narrow);
+    return plan_makespan(f.pairs, cost, n3, f.slots_per_xcd);
+  };
+  double best_t = flat(n3_max, 0);
   // Each wide block traded for narrow ones adds work: a dozen trades fill any last round.
   for (int n3 = n3_max - 1; n3 >= std::max(0, n3_max - 12); --n3) {
     const int n2 = narrow_blocks(n3);
-    const double t = plan_makespan(pairs, n3, n2, 1, 1.0, 0.0, narrow, cus_per_xcd);
+    const double t = flat(n3, n2);
     if (t < best_t - 1e-9) {
       best_t = t;
       best.n3 = n3;
@@ -1317,18 +1331,33 @@ BlockPlan choose_plan(int64_t max_cols, int64_t pairs, int w2, int w3, double na
     }
   }
   if (parts_ok) {
-    best_t = best_t * tiles + kStartTiles;
-    const int max_parts = std::min(kMaxParts, tiles / kMinPartTiles);
-    for (int parts = 2; parts <= max_parts; ++parts)
-      for (int n3 = n3_max; n3 >= std::max(0, n3_max - 2); --n3) {
-        const int n2 = n3 == n3_max ? 0 : narrow_blocks(n3);
-        const double t = kMergeTiles + plan_makespan(pairs, n3, n2, parts, (double)tiles / parts, kStartTiles, narrow,
-                                                     cus_per_xcd);
-        if (t < 0.95 * best_t) {
-          best_t = t;
-          best = BlockPlan{n3, n2, parts, (tiles + parts - 1) / parts};
+    // In tile times, each block as streaming the keys up to its last query's own.
+    auto causal = [&](int n3, int n2, int parts) {
+      cost.assign((size_t)(n3 + n2) * parts, 0.0);
+      for (int j = 0; j < n3 + n2; ++j) {
+        const int64_t after = j < n3 ? (int64_t)f.w3 * j : (int64_t)f.w3 * n3 + (int64_t)f.w2 * (j - n3);
+        const int seen = std::max<int64_t>(1, f.tiles - after / f.n_rep / kTileKeys);
+        for (int s = 0; s < parts; ++s) {
+          const int t0 = (int)((int64_t)s * f.tiles / parts), t1 = (int)((int64_t)(s + 1) * f.tiles / parts);
+          const double c = seen > t0 ? kStartTiles + (std::min(seen, t1) - t0) * (j < n3 ? 1.0 : f.narrow) : 0.3;
+          cost[j < n3 ? (size_t)s * n3 + j : (size_t)parts * n3 + (size_t)s * n2 + (j - n3)] = c;
         }
       }
+      return plan_makespan(f.pairs, cost, n3 * parts, f.slots_per_xcd);
+    };
+    best_t = causal(best.n3, best.n2, 1);
+    const int max_parts = std::min(kMaxParts, f.tiles / kMinPartTiles);
+    for (int parts = 2; parts <= max_parts; ++parts) {
+      const double merge = kMergeTiles + parts * (double)f.part_row_bytes / kMergeBytesPerTile;
+      for (int n3 = n3_max; n3 >= std::max(0, n3_max - 2); --n3) {
+        const int n2 = n3 == n3_max ? 0 : narrow_blocks(n3);
+        const double t = merge + causal(n3, n2, parts);
+        if (t < 0.97 * best_t) {
+          best_t = t;
+          best = BlockPlan{n3, n2, parts, (f.tiles + parts - 1) / parts};
+        }
+      }
+    }
   }
   if (cache.size() >= 4096) cache.clear();  // a caller cycling through many shapes recomputes
   cache.emplace(key, best);
@@ -1362,14 +1391,22 @@ struct ObsStats {
 bool tiled_shape(int head_dim, int n_rep) { return (head_dim == 128 || head_dim == 64) && n_rep <= 64; }
 bool fine_shape(int head_dim, int n_rep) { return head_dim != 128 || 16 % n_rep != 0; }
 
-BlockPlan plan_for(int batch, int max_chunk, int n_groups, int head_dim, int n_rep, int max_blocks, bool parts) {
-  constexpr int W = UKV_PREFILL_WAVES;
-  const bool fine = fine_shape(head_dim, n_rep);
-  const int cb3 = wide_blocks(fine, head_dim), cb2 = cb3 - 1;
-  const int tile_pages = head_dim == 64 ? PrefillLds<64>::kKeys / 16 : PrefillLds<128>::kKeys / 16;
-  return choose_plan((int64_t)max_chunk * n_rep, (int64_t)n_groups * batch, W * cb2 * 16, W * cb3 * 16,
-                     cb3 == 2 ? kNarrowCostFine : kNarrowCost, cus_per_xcd(), (max_blocks + tile_pages - 1) / tile_pages,
-                     parts);
+BlockPlan plan_for(int batch, int64_t rows, int max_chunk, int n_groups, int head_dim, int n_rep, int max_blocks,
+                   bool parts) {
+  constexpr int W = UKV_PREFILL_WAVES, tile_pages = kTileKeys / 16;
+  const int cb3 = wide_blocks(fine_shape(head_dim, n_rep), head_dim);
+  PlanShape f{};
+  f.max_cols = (int64_t)max_chunk * n_rep;
+  f.pairs = (int64_t)n_groups * batch;
+  f.part_row_bytes = rows * head_dim * (int64_t)sizeof(float);
+  f.w2 = W * (cb3 - 1) * 16;
+  f.w3 = W * cb3 * 16;
+  f.n_rep = n_rep;
+  f.slots_per_xcd = cus_per_xcd() * (head_dim == 64 ? 2 : 1);  // (two 64-dim workgroups share a CU)
+  f.tiles = (max_blocks + tile_pages - 1) / tile_pages;
+  f.narrow = cb3 == 2 ? kNarrowCostFine : kNarrowCost;
+  f.allow_parts = parts;
+  return choose_plan(f);
 }
 
 size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -1475,15 +1512,19 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
   if (fast) {
     const bool fine = fine_shape(head_dim, n_rep);
     const int64_t pairs = (int64_t)n_groups * batch, rows = (int64_t)total_q * num_q_heads;
-    BlockPlan plan = plan_for(batch, max_chunk, n_groups, head_dim, n_rep, max_blocks, workspace != nullptr);
+    BlockPlan plan = plan_for(batch, rows, max_chunk, n_groups, head_dim, n_rep, max_blocks, workspace != nullptr);
     // (the caller sizes the workspace by the same plan; a smaller one runs without parts)
     if (plan.parts > 1 && (part_bytes(plan.parts, rows, head_dim) > workspace_bytes ||
                            (rows + 7) / 8 > INT32_MAX || (reinterpret_cast<uintptr_t>(workspace) & 15u)))
-      plan = plan_for(batch, max_chunk, n_groups, head_dim, n_rep, max_blocks, false);
+      plan = plan_for(batch, rows, max_chunk, n_groups, head_dim, n_rep, max_blocks, false);
     a.n3 = plan.n3;
     a.n2 = plan.n2;
     a.n_parts = plan.parts;
     a.part_tiles = plan.part_tiles;
+    // No more keys than twice the chunk's: the blocks' key counts differ by a factor of two or more, and
+    // every pair's longest blocks go first. (With a long prefix they are alike, and the blocks of one
+    // pair stay together for their XCD's L2.)
+    a.by_block = (int64_t)max_blocks * 16 <= 2 * (int64_t)max_chunk;
     a.total_q = total_q;
     if (plan.parts > 1) {
       a.part_o = static_cast<float*>(workspace);
@@ -1566,9 +1607,10 @@ extern "C" size_t ukv_paged_prefill_workspace_bytes(int batch, int total_q, int 
       max_blocks <= 0 || !tiled_shape(head_dim, n_rep))
     return 0;
   const int n_groups = (num_q_heads + n_rep - 1) / n_rep;
-  const BlockPlan plan = plan_for(batch, max_chunk, n_groups, head_dim, n_rep, max_blocks, true);
+  const int64_t rows = (int64_t)total_q * num_q_heads;
+  const BlockPlan plan = plan_for(batch, rows, max_chunk, n_groups, head_dim, n_rep, max_blocks, true);
   if (plan.parts <= 1) return 0;
-  const size_t bytes = part_bytes(plan.parts, (int64_t)total_q * num_q_heads, head_dim);
+  const size_t bytes = part_bytes(plan.parts, rows, head_dim);
   return bytes > kMaxPartBytes ? 0 : bytes;
 }
 
