@@ -12,7 +12,7 @@
 // range) where the matrix cores sum it.
 //
 // Work decomposition: an item's mid keys form Kt tiles of 64 keys, split into
-// S contiguous ranges; one workgroup (8 waves) per (range, item). A unit is
+// S contiguous ranges; one workgroup (8 waves) per (range, item, unit group). A unit is
 // one KV group's q heads, or part of them when n_rep * obs > 512 rows: the
 // unit's Q rows (up to 512 = 8 waves x 4 tiles of 16) stay in registers while
 // its K tiles stream through LDS (64 keys, 16-byte rows loaded once per
@@ -27,6 +27,10 @@
 //           max over units per key in LDS, then the sums over 16-key blocks of
 //           the range;
 //   finish: the 3-wide max pool over each item's blocks.
+// Many items fill the device by themselves and a workgroup takes all units (one group). Few items are
+// split by unit as well, one or a few units per workgroup, so that ranges stay long (a unit's
+// queries and first keys cost ~4 tiles): pass 2 then leaves the running max of each group per key, and
+// the finish takes the max over the groups before the block sums.
 // Both passes compute Q K^T, so the cost is 2 * (2 * H_q * obs * aligned * D)
 // FLOPs per item on the matrix cores; K is read twice.
 //
@@ -66,10 +70,12 @@ struct SnapArgs {
   int Hq, Hkv, n_rep, D;
   int hp, parts;         // q heads per unit, units per KV group
   int S, Kt;             // key ranges per item, 64-key tiles per item
+  int groups;            // unit groups per item (grid.z)
   float scale_log2;
   float2* part_stats;    // [items][S][Hq*obs] (m, l) per range
   float2* stats;         // [items][Hq*obs] (m + log2(l), unused)
-  float* raw;            // [items][n_blocks] block sums before pooling
+  float* raw;            // [items][n_blocks] block sums before pooling (one group)
+  float* colbuf;         // [items][groups][aligned] running max per key (several groups)
   int32_t* redo;         // [items] or null: pass 1 and the merge run only for items with redo != 0
   float* out;            // [items][out_stride]
   int64_t out_stride;
@@ -148,13 +154,9 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
   if (!SCORES && a.redo && a.redo[item] == 0) return;  // whole workgroup: statistics given
   const int t0 = (int)((int64_t)s * a.Kt / a.S), t1 = (int)((int64_t)(s + 1) * a.Kt / a.S);
   const int key0 = t0 * kSnapTile;
-  const int R = a.hp * a.obs;  // rows of a unit
-  const int T = R / 16;        // row tiles of a unit
   const int tph = a.obs / 16;  // row tiles per q head
   const int rows_all = a.Hq * a.obs;
   const float c = a.scale_log2;
-  const bool hp_pow2 = (a.hp & (a.hp - 1)) == 0;
-  const int hp_log2 = 31 - __builtin_clz(a.hp);
   const int item_b = item / a.layers, item_l = item - item_b * a.layers;  // sequence, layer
   const int32_t* trow = a.table ? a.table + (int64_t)item_b * a.max_blocks : nullptr;
   // The kernel never writes the table: read it through the constant address space, so that
@@ -171,9 +173,15 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
   if constexpr (SCORES)
     for (int i = tid; i < (t1 - t0) * kSnapTile; i += blockDim.x) lds.colmax[i] = 0.f;
 
-  for (int u = 0; u < a.Hkv * a.parts; ++u) {
+  const int units = a.Hkv * a.parts;
+  const int u0 = (int)(blockIdx.z * units / a.groups), u1 = (int)((blockIdx.z + 1) * units / a.groups);
+  for (int u = u0; u < u1; ++u) {
     const int g = u / a.parts;
     const int h0 = g * a.n_rep + (u % a.parts) * a.hp;  // first q head of the unit
+    const int hp = min(a.hp, (g + 1) * a.n_rep - h0);   // its q heads (fewer in a group's last unit)
+    const int T = hp * tph;                             // its row tiles
+    const bool hp_pow2 = (hp & (hp - 1)) == 0;
+    const int hp_log2 = 31 - __builtin_clz(hp);
 
     // This wave's row tiles: w*TW .. w*TW+TW-1 (tiles past T are zero and unused).
     u32x4 qa[TW][STEPS];
@@ -256,17 +264,17 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
     // take the max over the unit's heads, and fold it into the range's running max.
     auto head_sum = [&](int tile, int b) {
       const int kb0 = tile * kSnapTile - key0;
-      if (hp_pow2 && kSnapTile * a.hp <= (int)blockDim.x) {
-        if (tid < kSnapTile * a.hp) {
-          const int key = tid >> hp_log2, h = tid & (a.hp - 1);
+      if (hp_pow2 && kSnapTile * hp <= (int)blockDim.x) {
+        if (tid < kSnapTile * hp) {
+          const int key = tid >> hp_log2, h = tid & (hp - 1);
           float x = 0.f;
           for (int q = h * tph; q < (h + 1) * tph; q += TW) x += lds.colpart[b][q][key];
-          for (int o = 1; o < a.hp; o <<= 1) x = fmaxf(x, __shfl_xor(x, o));  // hp consecutive lanes
+          for (int o = 1; o < hp; o <<= 1) x = fmaxf(x, __shfl_xor(x, o));  // hp consecutive lanes
           if (h == 0) lds.colmax[kb0 + key] = fmaxf(lds.colmax[kb0 + key], x);
         }
       } else if (tid < kSnapTile) {
         float mx = 0.f;
-        for (int h = 0; h < a.hp; ++h) {
+        for (int h = 0; h < hp; ++h) {
           float x = 0.f;
           for (int q = h * tph; q < (h + 1) * tph; q += TW) x += lds.colpart[b][q][tid];
           mx = fmaxf(mx, x);
@@ -441,6 +449,12 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
 
   if constexpr (SCORES) {
     __syncthreads();
+    if (a.groups > 1) {
+      float* col = a.colbuf + ((int64_t)item * a.groups + blockIdx.z) * a.aligned + key0;
+      for (int i = tid; i < (t1 - t0) * kSnapTile; i += blockDim.x)
+        if (key0 + i < a.aligned) col[i] = lds.colmax[i];
+      return;
+    }
     // Sums over 16-key blocks of the range, divided by obs (the mean over queries).
     const float inv_obs = 1.f / (float)a.obs;
     const int nb = (t1 - t0) * (kSnapTile / 16);
@@ -456,30 +470,48 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
 }
 
 // (m, l) partials of the S ranges -> m' = m + log2(l) per (item, row), so that
-// the weight of a score x (log2 units) is exp2(x - m').
+// the weight of a score x (log2 units) is exp2(x - m'). A block takes 16 rows of an item, its
+// threads 16 interleaved runs of the ranges each (a thread per row walked 64 ranges in 24 us).
 __global__ void __launch_bounds__(256) snap_stats_merge_kernel(const SnapArgs a) {
+  __shared__ float2 part[16][16];
   const int rows_all = a.Hq * a.obs;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)a.items * rows_all) return;
-  const int64_t item = idx / rows_all, row = idx % rows_all;
-  if (a.redo && a.redo[item] == 0) return;
-  float mx = -INFINITY;
-  for (int s = 0; s < a.S; ++s) mx = fmaxf(mx, a.part_stats[(item * a.S + s) * rows_all + row].x);
-  float l = 0.f;
-  for (int s = 0; s < a.S; ++s) {
-    const float2 p = a.part_stats[(item * a.S + s) * rows_all + row];
-    l += p.y * fast_exp2(p.x - mx);
+  const int64_t item = blockIdx.y;
+  if (a.redo && a.redo[item] == 0) return;  // whole workgroup
+  const int r = threadIdx.x & 15, run = threadIdx.x >> 4;
+  const int row = blockIdx.x * 16 + r;
+  const float2* ps = a.part_stats + item * a.S * rows_all + row;
+  float m = -INFINITY, l = 0.f;
+  if (row < rows_all)
+    for (int s = run; s < a.S; s += 16) {
+      const float2 p = ps[(int64_t)s * rows_all];
+      const float mn = fmaxf(m, p.x);
+      // (-inf - -inf: nothing summed yet on either side)
+      l = (m == mn ? l : l * fast_exp2(m - mn)) + (p.x == mn ? p.y : p.y * fast_exp2(p.x - mn));
+      m = mn;
+    }
+  part[run][r] = make_float2(m, l);
+  __syncthreads();
+  if (threadIdx.x < 16 && row < rows_all) {
+    float mx = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, part[i][r].x);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float2 p = part[i][r];
+      if (p.x > -INFINITY || p.y != 0.f) sum += p.y * fast_exp2(p.x - mx);
+    }
+    a.stats[item * rows_all + row] = make_float2(mx + log2f(sum), 0.f);
   }
-  a.stats[idx] = make_float2(mx + log2f(l), 0.f);
 }
 
 // Row statistics supplied by the caller (the prefill's observation rows): copied into
 // a.stats; an item with a row marked y != 0 (a sum that lost precision) or a non-finite
 // one gets redo[item] = 1, so that pass 1 recomputes its rows from the keys.
-__global__ void __launch_bounds__(256) snap_stats_import_kernel(const SnapArgs a, const float2* given) {
+__global__ void __launch_bounds__(1024) snap_stats_import_kernel(const SnapArgs a, const float2* given) {
   const int rows_all = a.Hq * a.obs;
   const int64_t item = blockIdx.x;
   bool bad = false;
+#pragma unroll 4
   for (int row = threadIdx.x; row < rows_all; row += blockDim.x) {
     const float2 v = given[item * rows_all + row];
     a.stats[item * rows_all + row] = v;
@@ -487,6 +519,43 @@ __global__ void __launch_bounds__(256) snap_stats_import_kernel(const SnapArgs a
   }
   bad = __syncthreads_or(bad);
   if (threadIdx.x == 0) a.redo[item] = bad ? 1 : 0;
+}
+
+// Several unit groups: out[item][n] from the groups' running maxima per key, kFinishBlocks blocks a
+// workgroup and one on either side for the pool. The sums run over a block's keys in order, as the one-group pass's.
+constexpr int kFinishBlocks = 30;
+__global__ void __launch_bounds__(256) snap_finish_kernel(const SnapArgs a) {
+  constexpr int NB = kFinishBlocks + 2;
+  __shared__ float col[NB * 16];
+  __shared__ float raw[NB];
+  const int64_t item = blockIdx.y;
+  const int b0 = blockIdx.x * kFinishBlocks - 1;  // the first block in LDS
+  const float* src = a.colbuf + item * a.groups * (int64_t)a.aligned;
+  for (int i = threadIdx.x; i < NB * 16; i += 256) {
+    const int key = b0 * 16 + i;
+    float x = 0.f;
+    if (key >= 0 && key < a.aligned)
+      for (int g = 0; g < a.groups; ++g) x = fmaxf(x, src[(int64_t)g * a.aligned + key]);
+    col[i] = x;
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < NB) {
+    float x = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x += col[16 * t + k];
+    raw[t] = x * (1.f / (float)a.obs);
+  }
+  __syncthreads();
+  if (t < kFinishBlocks && b0 + 1 + t < a.n_blocks) {
+    const int n = b0 + 1 + t;
+    float x = raw[t + 1];
+    if (a.n_blocks >= 3) {
+      if (n > 0) x = fmaxf(x, raw[t]);
+      if (n + 1 < a.n_blocks) x = fmaxf(x, raw[t + 2]);
+    }
+    a.out[item * a.out_stride + n] = x;
+  }
 }
 
 // out[item][n] = max(raw[n-1], raw[n], raw[n+1]) when n_blocks >= 3, else raw[n].
@@ -575,9 +644,33 @@ size_t a256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct SnapPlan {
   bool tiled;
-  int hp, tw, parts, S, Kt, aligned, n_blocks, L_mid;
-  size_t part_off, stats_off, raw_off, redo_off, total;
+  int hp, tw, parts, S, Kt, groups, aligned, n_blocks, L_mid;
+  size_t part_off, stats_off, raw_off, redo_off, total;  // raw_off: raw, or colbuf with several groups
 };
+
+// Key ranges S and unit groups of a call: rounds of one workgroup per CU, each taking units / groups
+// units of Kt / S tiles and a fixed cost per unit, kUnitTiles tile times (queries, statistics and first
+// keys: 64 ranges of 4 tiles over 8 units took 4.2 us a tile against 2.4 in long ranges). Groups cost the
+// finish a read of their running maxima.
+constexpr double kUnitTiles = 4.0;
+void choose_ranges(SnapPlan& p, int items, int units, int cus) {
+  const int need = (p.Kt * kSnapTile + kSnapMaxKeys - 1) / kSnapMaxKeys;
+  double best = 0.0;
+  for (int groups = 1; groups <= units; ++groups) {
+    if (units % groups != 0) continue;
+    const double finish = groups > 1 ? 1.0 + (double)items * groups * p.aligned * 8.0 / 4e6 / 2.4 : 0.0;
+    for (int r = 0; r <= 8; ++r) {  // the most ranges that fill r rounds (0: the fewest allowed)
+      const int S = std::min(p.Kt, std::max<int>(need, (int)((int64_t)r * cus / ((int64_t)items * groups))));
+      const int64_t rounds = ((int64_t)S * items * groups + cus - 1) / cus;
+      const double t = finish + (double)rounds * (units / groups) * ((p.Kt + S - 1) / S + kUnitTiles);
+      if (best == 0.0 || t < 0.999 * best) {
+        best = t;
+        p.S = S;
+        p.groups = groups;
+      }
+    }
+  }
+}
 
 SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, int n_rep, int head_dim,
                    int block_size, bool aligned_rows) {
@@ -586,37 +679,37 @@ SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, i
   p.aligned = ((std::max(1, p.L_mid) + block_size - 1) / block_size) * block_size;
   p.n_blocks = p.aligned / block_size;
   p.Kt = (p.aligned + kSnapTile - 1) / kSnapTile;
-  // Heads per unit: the largest divisor of n_rep whose row tiles fit the waves
-  // with TW tiles each, TW (1, 2 or 4, the smallest that fits) dividing the
-  // tiles of one q head, so that a wave's tiles never span two heads.
+  // Heads per unit and row tiles per wave: TW (1, 2 or 4) divides the tiles of one q head, so that a
+  // wave's tiles never span two heads, and hp heads' tiles fit the waves with TW each. The cheapest of
+  // the three is taken at the measured cost of a key tile under each TW; a group's last unit may hold
+  // fewer heads (7 heads x 128 queries: units of 4 and 3 instead of seven of 1).
   p.hp = 0;
   p.tw = 0;
   const int tph = obs / 16;
-  if (obs % 16 == 0 && tph > 0)
-    for (int h = std::min(n_rep, 32); h >= 1 && p.hp == 0; --h) {
-      if (n_rep % h != 0) continue;
-      for (int tw = 1; tw <= kSnapMaxTW; tw *= 2)
-        if (tph % tw == 0 && h * tph <= kSnapWaves * tw) {
-          p.hp = h;
-          p.tw = tw;
-          break;
-        }
+  if (obs % 16 == 0 && tph > 0) {
+    constexpr double kTileCost[3] = {0.9, 1.4, 2.4};
+    double best = 0.0;
+    for (int i = 0; i < 3; ++i) {
+      const int tw = 1 << i, h = std::min({n_rep, 32, kSnapWaves * tw / tph});
+      if (tw > kSnapMaxTW || tph % tw != 0 || h == 0) continue;
+      const int parts = (n_rep + h - 1) / h;
+      const double t = parts * kTileCost[i];
+      if (best == 0.0 || t < best) {
+        best = t;
+        p.hp = (n_rep + parts - 1) / parts;
+        p.tw = tw;
+      }
     }
-  p.tiled = (head_dim == 64 || head_dim == 128) && p.hp > 0 && aligned_rows;
-  p.parts = p.tiled ? n_rep / p.hp : 1;
-  if (p.tiled) {
-    const int want = (2 * snap_cu_count() + items - 1) / std::max(1, items);
-    const int need = (p.Kt * kSnapTile + kSnapMaxKeys - 1) / kSnapMaxKeys;
-    p.S = std::max(need, std::min(want, std::max(1, p.Kt / 4)));
-    p.S = std::min(p.S, p.Kt);
-  } else {
-    p.S = 1;
   }
+  p.tiled = (head_dim == 64 || head_dim == 128) && p.hp > 0 && aligned_rows;
+  p.parts = p.tiled ? (n_rep + p.hp - 1) / p.hp : 1;
+  p.S = p.groups = 1;
+  if (p.tiled) choose_ranges(p, items, num_q_heads / n_rep * p.parts, snap_cu_count());
   const size_t rows_all = (size_t)num_q_heads * obs;
   p.part_off = 0;
   p.stats_off = a256((size_t)items * p.S * rows_all * sizeof(float2));
   p.raw_off = p.stats_off + a256((size_t)items * rows_all * sizeof(float2));
-  p.redo_off = p.raw_off + a256((size_t)items * p.n_blocks * sizeof(float));
+  p.redo_off = p.raw_off + a256((size_t)items * (p.groups > 1 ? (size_t)p.groups * p.aligned : p.n_blocks) * sizeof(float));
   p.total = p.redo_off + a256((size_t)items * sizeof(int32_t));
   return p;
 }
@@ -624,10 +717,9 @@ SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, i
 // With a.redo set, pass 1 and the merge skip the items whose statistics were imported.
 template <int DT, int D, int TW>
 void launch_tiled(const SnapArgs& a, const SnapPlan& p, hipStream_t st) {
-  const int64_t rows = (int64_t)a.items * a.Hq * a.obs;
-  const dim3 grid(p.S, a.items);
+  const dim3 grid(p.S, a.items, p.groups);
   hipLaunchKernelGGL((snap_tile_kernel<DT, D, false, TW>), grid, dim3(64 * kSnapWaves), 0, st, a);
-  hipLaunchKernelGGL(snap_stats_merge_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(snap_stats_merge_kernel, dim3((unsigned)((a.Hq * a.obs + 15) / 16), a.items), dim3(256), 0, st, a);
   hipLaunchKernelGGL((snap_tile_kernel<DT, D, true, TW>), grid, dim3(64 * kSnapWaves), 0, st, a);
 }
 
@@ -644,7 +736,7 @@ void launch_tiled_tw(const SnapArgs& a, const SnapPlan& p, hipStream_t st) {
 template <int DT>
 void launch_snap(const SnapArgs& a, const SnapPlan& p, hipStream_t st, const float2* given) {
   if (given)
-    hipLaunchKernelGGL(snap_stats_import_kernel, dim3((unsigned)a.items), dim3(256), 0, st, a, given);
+    hipLaunchKernelGGL(snap_stats_import_kernel, dim3((unsigned)a.items), dim3(1024), 0, st, a, given);
   if (p.tiled) {
     if (a.D == 64)
       launch_tiled_tw<DT, 64>(a, p, st);
@@ -654,6 +746,11 @@ void launch_snap(const SnapArgs& a, const SnapPlan& p, hipStream_t st, const flo
     const int64_t rows = (int64_t)a.items * a.Hq * a.obs;
     hipLaunchKernelGGL(snap_scalar_stats_kernel<DT>, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(snap_scalar_scores_kernel<DT>, dim3(a.n_blocks, a.items), dim3(64), 0, st, a);
+  }
+  if (a.groups > 1) {
+    hipLaunchKernelGGL(snap_finish_kernel, dim3((unsigned)((a.n_blocks + kFinishBlocks - 1) / kFinishBlocks), a.items),
+                       dim3(256), 0, st, a);
+    return;
   }
   const int64_t nout = (int64_t)a.items * a.n_blocks;
   hipLaunchKernelGGL(snap_pool_kernel, dim3((unsigned)((nout + 255) / 256)), dim3(256), 0, st, a);
@@ -743,11 +840,13 @@ int snapkv_scores_impl(const void* q_obs, const int64_t* q_strides, const void* 
   a.parts = p.parts;
   a.S = p.S;
   a.Kt = p.Kt;
+  a.groups = p.groups;
   a.scale_log2 = softmax_scale * kLog2e;
   char* ws = static_cast<char*>(workspace);
   a.part_stats = reinterpret_cast<float2*>(ws + p.part_off);
   a.stats = reinterpret_cast<float2*>(ws + p.stats_off);
   a.raw = reinterpret_cast<float*>(ws + p.raw_off);
+  a.colbuf = a.raw;
   a.redo = given_stats ? reinterpret_cast<int32_t*>(ws + p.redo_off) : nullptr;
   a.out = scores;
   a.out_stride = scores_stride;
