@@ -6,52 +6,54 @@
 // lower index; NaN ranks above every number (as torch.topk treats it). The
 // winners are written in ascending index order.
 //
-// One 256-thread workgroup per row. Each element gets a unique 64-bit key,
-//   key = (~orderable(score) << 32) | index,
-// so "k smallest keys" is exactly the selection. A radix select over the 64
-// key bits (8 passes of 8-bit digits, LDS histograms) finds the k-th smallest
-// key T; the winners are the elements with key <= T, compacted in index order
-// with a block-wide prefix sum. Any row length works; the row is re-read from
-// global memory (L2) on each pass.
+// One workgroup per row, latency-bound: a handful of short phases between barriers. A score's key is
+// the bitwise complement of its order-preserving integer image, so "k smallest keys" is the selection. A radix
+// select over the key's 11, 11 and 10 bits (LDS histograms, scanned by all threads) finds the k-th
+// smallest key T and how many keys equal to T belong to the selection: the ones of lowest index.
+// Each wave owns a contiguous run of the row, so the winners' places in index order follow from
+// ballots and the waves' counts. The row is read once, into registers (rows past 16 per thread are
+// read again by each phase). 32 rows of 2036 scores: 7.5 us against 57 for eight 8-bit passes over
+// 64-bit (score, index) keys whose histograms one thread walked.
 #include "ukv_common.h"
 
 namespace ukv {
 
-__device__ __forceinline__ uint64_t select_key(float s, int idx) {
+__device__ __forceinline__ uint32_t select_key(float s) {
   uint32_t u = __float_as_uint(s);
   if (s != s) u = 0x7fc00000u;  // canonical NaN ranks highest
   if (u == 0x80000000u) u = 0u;  // -0 equals +0: the tie goes to the lower index
   const uint32_t ord = (u & 0x80000000u) ? ~u : (u | 0x80000000u);  // ascending with the float value
-  return (uint64_t(~ord) << 32) | uint32_t(idx);
+  return ~ord;
 }
 
-// Exclusive prefix sum of one value per thread over a 256-thread block.
-__device__ __forceinline__ int block_exclusive_scan_256(int v, int* sh) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) sh[wv] = x;
-  __syncthreads();
-  int base = 0;
-  for (int w = 0; w < wv; ++w) base += sh[w];
-  __syncthreads();
-  return base + x - v;
+// Inclusive prefix sum over the wave (DPP row shifts, then the rows' totals broadcast onwards).
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
 }
 
-__global__ void __launch_bounds__(256) select_topk_kernel(const float* __restrict__ scores, int64_t row_stride,
-                                                          const int32_t* __restrict__ row_n,
-                                                          const int32_t* __restrict__ row_k, int n_max, int k_max,
-                                                          int32_t* __restrict__ out, int64_t out_stride) {
-  __shared__ unsigned hist[256];
-  __shared__ int scan_sh[4];
-  __shared__ uint64_t s_prefix;
-  __shared__ int s_need;
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
 
-  const int row = blockIdx.x;
+// NT threads; R > 0: rows of up to NT * R scores, held in registers; R = 0: any row.
+template <int NT, int R>
+__global__ void __launch_bounds__(NT) select_topk_kernel(const float* __restrict__ scores, int64_t row_stride,
+                                                         const int32_t* __restrict__ row_n,
+                                                         const int32_t* __restrict__ row_k, int n_max, int k_max,
+                                                         int32_t* __restrict__ out, int64_t out_stride) {
+  constexpr int NW = NT / 64, kBits = 11, kBins = 1 << kBits, PER = kBins / NT;
+  __shared__ int hist[kBins];
+  __shared__ int wave_sum[NW];
+  __shared__ int2 wave_cnt[NW];
+  __shared__ int s_bin, s_need;
+
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const float* sc = scores + (int64_t)row * row_stride;
   int32_t* o = out + (int64_t)row * out_stride;
   int n = row_n ? row_n[row] : n_max;
@@ -60,52 +62,106 @@ __global__ void __launch_bounds__(256) select_topk_kernel(const float* __restric
   k = k < 0 ? 0 : (k > n ? n : k);
   k = k > k_max ? k_max : k;
 
-  for (int i = k + threadIdx.x; i < k_max; i += blockDim.x) o[i] = -1;
-  if (k == 0) return;
-
-  // Radix select of the k-th smallest key: prefix holds the decided high bits.
-  if (threadIdx.x == 0) {
-    s_prefix = 0;
-    s_need = k;  // rank (1-based) of the wanted key among keys matching the prefix
+  for (int i = k + tid; i < k_max; i += NT) o[i] = -1;
+  if (k == 0) return;  // whole workgroup
+  if (k == n) {        // (uniform) the whole row
+    for (int i = tid; i < n; i += NT) o[i] = i;
+    return;
   }
-  uint64_t T = ~uint64_t(0);
-  if (k < n) {
-    for (int pass = 0; pass < 8; ++pass) {
-      const int shift = 56 - 8 * pass;
-      const uint64_t hi_mask = pass == 0 ? 0 : (~uint64_t(0) << (shift + 8));
-      hist[threadIdx.x] = 0;
-      __syncthreads();
-      const uint64_t prefix = s_prefix;
-      for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const uint64_t key = select_key(sc[i], i);
-        if ((key & hi_mask) == prefix) atomicAdd(&hist[(key >> shift) & 0xff], 1u);
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        int need = s_need;
-        int d = 0;
-        for (; d < 256; ++d) {
-          if ((int)hist[d] >= need) break;
-          need -= (int)hist[d];
-        }
-        s_prefix = prefix | (uint64_t(d) << shift);
-        s_need = need;
-      }
-      __syncthreads();
+
+  // The wave's run: `steps` times 64 scores from run0.
+  const int steps = R > 0 ? R : (n + NT - 1) / NT;
+  const int run0 = wv * steps * 64;
+  uint32_t keys[R > 0 ? R : 1];
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = run0 + r * 64 + lane;
+      keys[r] = i < n ? select_key(sc[i]) : 0u;
     }
-    T = s_prefix;  // keys are unique, so the full 64-bit prefix is the k-th key
   }
+  auto key_of = [&](int r, int i) -> uint32_t { return R > 0 ? keys[R > 0 ? r : 0] : select_key(sc[i]); };
+  auto each = [&](auto f) {  // f(score index, key) for the wave's scores; lanes past the row take index -1
+    if constexpr (R > 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int i = run0 + r * 64 + lane;
+        if (run0 + r * 64 < n) f(i < n ? i : -1, key_of(r, i));  // (wave-uniform)
+      }
+    } else {
+      for (int r = 0; r < steps && run0 + r * 64 < n; ++r) {
+        const int i = run0 + r * 64 + lane;
+        f(i < n ? i : -1, i < n ? key_of(r, i) : 0u);
+      }
+    }
+  };
 
-  // Winners (key <= T) in ascending index order.
-  int written = 0;
-  for (int base = 0; base < n; base += blockDim.x) {
-    const int i = base + threadIdx.x;
-    const int flag = (i < n) && (select_key(sc[i], i) <= T);
-    const int pos = written + block_exclusive_scan_256(flag, scan_sh);
-    if (flag) o[pos] = i;
-    const int total = __syncthreads_count(flag);
-    written += total;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) hist[tid * PER + j] = 0;
+  __syncthreads();
+  uint32_t prefix = 0;  // the k-th smallest key's decided high bits
+  int need = k;         // its rank (1-based) among the keys that share them
+#pragma unroll
+  for (int pass = 0; pass < 3; ++pass) {
+    const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0;
+    const uint32_t mask = pass == 2 ? 1023u : 2047u;
+    each([&](int i, uint32_t key) {
+      if (i >= 0 && (pass == 0 || (key >> (pass == 1 ? 21 : 10)) == prefix)) atomicAdd(&hist[(key >> shift) & mask], 1);
+    });
+    __syncthreads();
+    // Each thread's bins (cleared for the next pass); the thread whose bins hold rank `need` names the digit.
+    int c[PER], sum = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      c[j] = hist[tid * PER + j];
+      hist[tid * PER + j] = 0;
+      sum += c[j];
+    }
+    const int incl = wave_scan(sum);
+    if (lane == 63) wave_sum[wv] = incl;
+    __syncthreads();
+    int before = incl - sum;
+    for (int w = 0; w < wv; ++w) before += wave_sum[w];
+    if (before < need && before + sum >= need) {  // exactly one thread
+      int left = need - before, bin = tid * PER;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        if (left > c[j] && bin == tid * PER + j) {
+          left -= c[j];
+          ++bin;
+        }
+      }
+      s_bin = bin;
+      s_need = left;
+    }
+    __syncthreads();
+    prefix = pass == 0 ? (uint32_t)s_bin : pass == 1 ? (prefix << 11) | (uint32_t)s_bin : (prefix << 10) | (uint32_t)s_bin;
+    need = s_need;
   }
+  const uint32_t T = prefix;
+
+  // Winners: keys below T, and the first `need` keys equal to it, in ascending index order.
+  int lt = 0, eq = 0;
+  each([&](int i, uint32_t key) {
+    lt += __popcll(__ballot(i >= 0 && key < T));
+    eq += __popcll(__ballot(i >= 0 && key == T));
+  });
+  if (lane == 0) wave_cnt[wv] = make_int2(lt, eq);
+  __syncthreads();
+  int lt0 = 0, eq0 = 0;
+  for (int w = 0; w < wv; ++w) {
+    lt0 += wave_cnt[w].x;
+    eq0 += wave_cnt[w].y;
+  }
+  int pos = lt0 + min(eq0, need);
+  each([&](int i, uint32_t key) {
+    const uint64_t meq = __ballot(i >= 0 && key == T);
+    const bool take = i >= 0 && (key < T || (key == T && eq0 + lanes_below(meq) < need));
+    const uint64_t mt = __ballot(take);
+    if (take) o[pos + lanes_below(mt)] = i;
+    pos += __popcll(mt);
+    eq0 += __popcll(meq);
+  });
 }
 
 }  // namespace ukv
@@ -120,7 +176,17 @@ extern "C" int ukv_select_topk(const float* scores, int64_t row_stride, const in
   if (rows < 0 || n_max < 0 || k_max < 0 || row_stride < n_max || out_stride < k_max) return UKV_ERR_INVALID_ARGUMENT;
   if (rows == 0 || k_max == 0) return UKV_OK;
   if (!scores || !out) return UKV_ERR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL(select_topk_kernel, dim3(rows), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), scores,
-                     row_stride, row_n, row_k, n_max, k_max, out, out_stride);
+  const dim3 grid(rows);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // Four waves while a row fits their registers (fewer waves to meet at a barrier), then sixteen.
+  if (n_max <= 256 * 8)
+    hipLaunchKernelGGL((select_topk_kernel<256, 8>), grid, dim3(256), 0, st, scores, row_stride, row_n, row_k, n_max,
+                       k_max, out, out_stride);
+  else if (n_max <= 1024 * 16)
+    hipLaunchKernelGGL((select_topk_kernel<1024, 16>), grid, dim3(1024), 0, st, scores, row_stride, row_n, row_k, n_max,
+                       k_max, out, out_stride);
+  else
+    hipLaunchKernelGGL((select_topk_kernel<1024, 0>), grid, dim3(1024), 0, st, scores, row_stride, row_n, row_k, n_max,
+                       k_max, out, out_stride);
   return hipGetLastError() == hipSuccess ? UKV_OK : UKV_ERR_LAUNCH;
 }
