@@ -298,6 +298,27 @@ int ukv_kv_write_varlen(void* k_pool_layer, void* v_pool_layer, const int64_t* k
                         int max_chunk, int num_heads, int head_dim, int num_pages, ukv_stream_t stream);
 
 /*
+ * Retained logical pages of a block-aligned compaction (core/scheduler.py:762-779): row l of out
+ * ([layers][sink_blocks + k + obs_blocks] int32, contiguous) is 0 .. sink_blocks - 1, then sel[l] (int32,
+ * row stride sel_layer_stride) + sink_blocks, then obs_first .. obs_first + obs_blocks - 1. *bad is set
+ * to 1 when a selected block lies outside [0, n_mid), and left alone otherwise; it may be pinned host
+ * memory, cleared by the caller and read after synchronising the stream.
+ */
+int ukv_retained_pages(const int32_t* sel, int layers, int64_t sel_layer_stride, int k, int n_mid, int sink_blocks,
+                       int obs_first, int obs_blocks, int32_t* out, int32_t* bad, ukv_stream_t stream);
+
+/*
+ * Physical source pages of a compaction: for sequence s (host arrays of seqs entries: keep[s], a device
+ * pointer to int32 [layers][n_keep[s]] logical pages with row stride keep_layer_strides[s]; n_pages[s],
+ * its pages in the concatenated device list `pages`), columns n_keep[0] + .. + n_keep[s - 1] onwards of
+ * out ([layers][out_cols] int32) receive pages_s[keep_s[l][j]]; an index outside [0, n_pages[s])
+ * gives -1 and sets bad[s] to 1 (bad as in ukv_retained_pages, one entry per sequence).
+ */
+int ukv_compact_sources(const void* const* keep, const int64_t* keep_layer_strides, const int32_t* n_keep,
+                        const int32_t* n_pages, int seqs, int layers, const int32_t* pages, int32_t* out,
+                        int64_t out_cols, int32_t* bad, ukv_stream_t stream);
+
+/*
  * Chunked prefill attention over the paged pool. Query row cu_seqlens_q[b] + i (i < C_b) of
  * sequence b is at position P_b + i, P_b = kv_lens[b] - C_b, and attends to keys
  * 0 .. P_b + i of the sequence (causal, bottom-right aligned) read through block_table

@@ -26,6 +26,7 @@ SOURCES = [
     "page_ops.hip",
     "retain_copy.hip",
     "select.hip",
+    "compact_plan.hip",
     "paged_prefill.hip",
     "snapkv_score.hip",
 ]

@@ -105,6 +105,17 @@ SIGNATURES = {
             _c_int, _c_int, _c_int, _c_void_p,  # layers, heads, head_dim, stream
         ],
     ),
+    "ukv_retained_pages": (
+        _c_int,
+        [_c_void_p, _c_int, ctypes.c_int64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p],
+    ),
+    "ukv_compact_sources": (
+        _c_int,
+        [
+            ctypes.POINTER(_c_void_p), _c_i64p, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32),
+            _c_int, _c_int, _c_void_p, _c_void_p, ctypes.c_int64, _c_void_p, _c_void_p,
+        ],
+    ),
     "ukv_kv_append": (
         _c_int,
         [

@@ -31,6 +31,8 @@ retained indices (out-of-range entries would otherwise copy the wrong page).
 """
 from __future__ import annotations
 
+import array
+import ctypes
 import math
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
@@ -99,6 +101,9 @@ def retained_pages(L: int, selected_mid: torch.Tensor, *, block_size: int = 16, 
     if L % B or sink_len % B or obs_len % B:
         raise ValueError("retained_pages: the page-granular path needs block-aligned L, sink and window")
     n_mid = (L - sink_len - obs_len) // B
+    if (selected_mid.is_cuda and selected_mid.dtype == torch.int32 and selected_mid.dim() == 2
+            and selected_mid.stride(1) == 1 and n_mid >= 0):
+        return _retained_pages_gpu(selected_mid, n_mid, sink_len // B, (L - obs_len) // B, obs_len // B)
     if selected_mid.numel() and bool(((selected_mid < 0) | (selected_mid >= n_mid)).any()):
         # select_blocks pads short rows with -1, which the sink offset would turn into a real page
         raise ValueError(f"retained_pages: selected middle blocks outside [0, {n_mid})")
@@ -107,6 +112,25 @@ def retained_pages(L: int, selected_mid: torch.Tensor, *, block_size: int = 16, 
     sink = torch.arange(sink_len // B, dtype=torch.int32, device=dev).expand(layers, -1)
     obs = torch.arange((L - obs_len) // B, L // B, dtype=torch.int32, device=dev).expand(layers, -1)
     return torch.cat([sink, selected_mid + sink_len // B, obs], dim=1)
+
+
+def _flags(n: int) -> torch.Tensor:
+    """n cleared int32 flags in pinned host memory, which kernels set directly; read after a stream sync."""
+    return torch.zeros(n, dtype=torch.int32, pin_memory=True)
+
+
+def _retained_pages_gpu(sel: torch.Tensor, n_mid: int, sink_blocks: int, obs_first: int,
+                        obs_blocks: int) -> torch.Tensor:
+    layers, k = (int(x) for x in sel.shape)
+    out = torch.empty((layers, sink_blocks + k + obs_blocks), dtype=torch.int32, device=sel.device)
+    bad = _flags(1)
+    code = _ext.load().ukv_retained_pages(sel.data_ptr(), layers, int(sel.stride(0)), k, n_mid, sink_blocks, obs_first,
+                                          obs_blocks, out.data_ptr(), bad.data_ptr(), _stream(sel.device))
+    _ext.check(code, "ukv_retained_pages")
+    torch.cuda.current_stream(sel.device).synchronize()
+    if int(bad[0]):
+        raise ValueError(f"retained_pages: selected middle blocks outside [0, {n_mid})")
+    return out
 
 
 @dataclass
@@ -124,10 +148,50 @@ def _host_ids(ids, dev) -> torch.Tensor:
     return torch.tensor([int(x) for x in ids], dtype=torch.int32).pin_memory().to(dev, non_blocking=True)
 
 
-def _check_pool_ids(pool, ids, what):
-    bad = [int(x) for x in ids if not 0 <= int(x) < pool.N_total]
-    if bad:
-        raise ValueError(f"{what}: page ids outside the pool: {bad[:4]}")
+def _id_array(ids) -> np.ndarray:
+    """A list of ids as an integer array (int32 where they fit)."""
+    try:
+        return np.frombuffer(array.array("i", ids), dtype=np.int32) if len(ids) else np.zeros(0, np.int32)
+    except (TypeError, OverflowError):  # not plain ints, or beyond 32 bits
+        return np.array([int(x) for x in ids], dtype=np.int64)
+
+
+def _check_pool_ids(pool, ids, what) -> np.ndarray:
+    """The ids as an array, each inside the pool."""
+    arr = _id_array(ids)
+    if arr.size and (int(arr.min()) < 0 or int(arr.max()) >= pool.N_total):
+        bad = arr[(arr < 0) | (arr >= pool.N_total)]
+        raise ValueError(f"{what}: page ids outside the pool: {[int(x) for x in bad[:4]]}")
+    return arr
+
+
+def _upload_ids(arrays, dev) -> torch.Tensor:
+    """The id arrays, one after another, as one int32 device tensor (one pinned copy)."""
+    host = np.concatenate(arrays) if arrays else np.zeros(0, np.int32)
+    return torch.from_numpy(host.astype(np.int32, copy=False)).pin_memory().to(dev, non_blocking=True)
+
+
+def _source_ids(pool, page_arrays, keeps) -> torch.Tensor:
+    """int32 [layers, sum of n_keep] physical source pages of every sequence, side by side; ValueError when
+    a retained index lies outside its sequence's list (one host synchronisation)."""
+    dev, layers, seqs = pool.device, pool.num_layers, len(keeps)
+    n_keep = [int(k.shape[1]) for k in keeps]
+    src = torch.empty((layers, sum(n_keep)), dtype=torch.int32, device=dev)
+    if src.numel() == 0:
+        return src
+    pages = _upload_ids(page_arrays, dev)
+    bad = _flags(seqs)
+    i32s = ctypes.c_int32 * seqs
+    code = _ext.load().ukv_compact_sources(
+        _ext.ptr_array([k.data_ptr() for k in keeps]), _ext.i64_array([k.stride(0) for k in keeps]), i32s(*n_keep),
+        i32s(*[len(a) for a in page_arrays]), seqs, layers, pages.data_ptr(), src.data_ptr(), int(src.shape[1]),
+        bad.data_ptr(), _stream(dev))
+    _ext.check(code, "ukv_compact_sources")
+    torch.cuda.current_stream(dev).synchronize()
+    if bool(bad.any()):
+        s = int(torch.nonzero(bad)[0, 0])
+        raise ValueError(f"compact: sequence {s}: retained page indices outside [0, {len(page_arrays[s])})")
+    return src
 
 
 def _check_keep(keep: torch.Tensor, n_pages: int, what: str) -> None:
@@ -154,14 +218,17 @@ def compact(pool, seq_page_lists: Sequence[Sequence[int]], retained: Sequence[to
     """
     dev = pool.device
     L = pool.num_layers
-    keeps = []
+    keeps, page_arrays = [], []
     for s, (pages, keep) in enumerate(zip(seq_page_lists, retained)):
         if keep.dim() != 2 or int(keep.shape[0]) != L:
             raise ValueError("compact: retained index rows must match the pool's layers")
-        _check_pool_ids(pool, pages, f"compact: sequence {s}")
-        keep = keep.to(device=dev, dtype=torch.long)
-        _check_keep(keep, len(pages), f"compact: sequence {s}")
-        keeps.append(keep)
+        page_arrays.append(_check_pool_ids(pool, pages, f"compact: sequence {s}"))
+        if keep.dtype != torch.int32:  # checked at its own width before it is narrowed
+            _check_keep(keep, len(pages), f"compact: sequence {s}")
+        keep = keep.to(device=dev, dtype=torch.int32)
+        keeps.append(keep if keep.stride(1) == 1 else keep.contiguous())
+    src = _source_ids(pool, page_arrays, keeps)
+    at = 0
     if free_sources:
         dst_lists: List[List[int]] = []
         for s, (pages, keep) in enumerate(zip(seq_page_lists, keeps)):
@@ -172,8 +239,8 @@ def compact(pool, seq_page_lists: Sequence[Sequence[int]], retained: Sequence[to
                 err.partial = dst_lists
                 raise err
             if n_keep:
-                src = _host_ids(pages, dev)[keep].to(torch.int32).contiguous()
-                pool.copy_pages(src, _host_ids(ids, dev))
+                pool.copy_pages(src[:, at:at + n_keep], _upload_ids([_id_array(ids)], dev))
+                at += n_keep
             pool.free_blocks_by_ids(list(pages))
             dst_lists.append(ids)
     else:
@@ -189,11 +256,8 @@ def compact(pool, seq_page_lists: Sequence[Sequence[int]], retained: Sequence[to
             for ids in dst_lists:
                 pool.free_blocks_by_ids(ids)
             raise
-        src_parts = [_host_ids(pages, dev)[keep] for pages, keep in zip(seq_page_lists, keeps)
-                     if int(keep.shape[1]) > 0]
-        if src_parts:
-            src = torch.cat(src_parts, dim=1).to(torch.int32).contiguous()  # [L, n] physical ids
-            pool.copy_pages(src, _host_ids([p for ids in dst_lists for p in ids], dev))
+        if int(src.shape[1]):
+            pool.copy_pages(src, _upload_ids([_id_array(ids) for ids in dst_lists], dev))
     table = pool.block_table_for([list(x) for x in dst_lists]) if dst_lists else None
     return CompactionResult(page_lists=dst_lists, block_table=table, seq_lens=[int(x) for x in seq_lens])
 
