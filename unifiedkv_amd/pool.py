@@ -153,18 +153,19 @@ class PagedKVPool:
                 keep = -n
                 ids = [self._free.popleft() for _ in range(len(self._free) - keep)]
             else:
-                ids = [self._free.popleft() for _ in range(n)]
-            for bid in ids:
-                self.used_blocks[bid] = 1
+                pop = self._free.popleft
+                ids = [pop() for _ in range(n)]
+            self.used_blocks.update(dict.fromkeys(ids, 1))
             return ids
 
     def free_blocks_by_ids(self, block_ids: List[int]):
         """Appends every id to the free list, in order (core/pool.py:111-116)."""
         with self.lock:
-            for bid in block_ids:
-                if bid in self.used_blocks:
-                    del self.used_blocks[bid]
-                self._free.append(bid)
+            ids = list(block_ids)
+            used = self.used_blocks
+            for bid in ids:
+                used.pop(bid, None)
+            self._free.extend(ids)
 
     def check_watermark(self, n_required: int) -> str:
         with self.lock:
