@@ -932,18 +932,20 @@ paged_prefill_kernel(const PrefillArgs a) {
 // it is flagged (y = 1) for the scoring pass to recompute from the keys where the prefill flagged
 // it, where the sink and window hold half of its weight or more (the difference would lose bits),
 // or where the middle sum falls below 2^-100 of its max (m is the max over every key the query
-// sees: middle weights below 2^-126 of it lose bits). One wave per 16 columns (observation query,
-// q head of the group) of a (sequence, KV group); lane (i16, kg) holds column i16 and keys
-// 4kg .. 4kg + 3 of each 16-key page. (The (m, l) pairs exist only where the tiled kernel ran.)
+// sees: middle weights below 2^-126 of it lose bits). One workgroup per 16 columns (observation query,
+// q head of the group) of a (sequence, KV group), its four waves taking every fourth page: a 64-key
+// sink and a 128-key window are one round of loads (one wave took them in four, 13.5 us a layer at 2
+// x 8 x 32 column blocks). Lane (i16, kg) holds column i16 and keys 4kg .. 4kg + 3 of each 16-key
+// page. (The (m, l) pairs exist only where the tiled kernel ran.)
 template <int DT>
 __global__ void __launch_bounds__(256) obs_rows_finish_kernel(const PrefillArgs a) {
+  __shared__ float wave_part[4][16];
   const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cols = a.obs * a.n_rep;
   const int nblk = (cols + 15) >> 4;
-  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= (int64_t)a.B * a.n_groups * nblk) return;  // (wave-uniform)
-  const int blk = (int)(w % nblk);
-  const int64_t pair = w / nblk;
+  const int blk = (int)(blockIdx.x % nblk);
+  const int64_t pair = blockIdx.x / nblk;
   const int g = (int)(pair % a.n_groups), b = (int)(pair / a.n_groups);
   const int q_begin = a.cu_q[b], C = a.cu_q[b + 1] - q_begin;
   const int L = kv_len_of(a, b);
@@ -951,7 +953,7 @@ __global__ void __launch_bounds__(256) obs_rows_finish_kernel(const PrefillArgs 
   const int i = col / a.n_rep, h = g * a.n_rep + col % a.n_rep;
   const int qi = C - a.obs + i;
   const bool live = col < cols && h < a.Hq && qi >= 0 && C <= a.max_chunk;
-  if (!__any(live)) return;  // (wave-uniform: a chunk shorter than the window, or too long)
+  if (!__any(live)) return;  // (workgroup-uniform: a chunk shorter than the window, or too long)
   float2* slot = a.obs_stats + (int64_t)b * a.stats_seq_stride + (int64_t)h * a.obs + i;
   const float2 ml = live ? *slot : make_float2(0.f, 0.f);
   const bool ok = live && __builtin_isfinite(ml.x) && ml.y > 0.f && __builtin_isfinite(ml.y);
@@ -965,41 +967,49 @@ __global__ void __launch_bounds__(256) obs_rows_finish_kernel(const PrefillArgs 
   const float sl2 = a.scale_log2;
   const int32_t* btrow = a.bt + (int64_t)b * a.max_blocks;
   float part = 0.f;
-  // Keys [lo, hi) of pages p0 .. p1 - 1 (page pg holds keys 16 pg .. 16 pg + 15), four pages at a
-  // time with their loads issued together. A operand: dims 32s + 8kg .. of key 16 pg + i16.
-  auto pages = [&](int p0, int p1, int lo, int hi) {
-    for (int pg = p0; pg < p1; pg += 4) {
-      u32x4 ka[4][4];
-      bool pok[4];
+  // The sink's keys [0, s_end) and the window's [w_beg, L), page by page (page pg holds keys 16 pg ..
+  // 16 pg + 15): this wave's pages four at a time, their loads issued together. A operand: dims
+  // 32s + 8kg .. of key 16 pg + i16.
+  const int s_end = min(a.sink, L), w_beg = max(L - a.obs, a.sink);
+  const int n_sink = (s_end + 15) >> 4, w_page = w_beg >> 4;
+  const int n_all = n_sink + max(0, ((L + 15) >> 4) - w_page);
+  for (int t0 = wv; t0 < n_all; t0 += 16) {
+    u32x4 ka[4][4];
+    int pg[4];
+    bool pok[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int id = pg + u < p1 ? btrow[pg + u] : -1;
-        pok[u] = (unsigned)id < (unsigned)a.num_pages;
-        const uint16_t* kp =
-            a.k + (int64_t)(pok[u] ? id : 0) * a.k_sp + (int64_t)i16 * a.k_st + (int64_t)g * a.k_sh + 8 * kg;
+    for (int u = 0; u < 4; ++u) {
+      const int t = t0 + 4 * u;
+      pg[u] = t < n_sink ? t : w_page + t - n_sink;
+      const int id = t < n_all ? btrow[pg[u]] : -1;
+      pok[u] = (unsigned)id < (unsigned)a.num_pages;
+      const uint16_t* kp =
+          a.k + (int64_t)(pok[u] ? id : 0) * a.k_sp + (int64_t)i16 * a.k_st + (int64_t)g * a.k_sh + 8 * kg;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ka[u][s] = pok[u] ? ld16(kp + 32 * s) : u32x4{0u, 0u, 0u, 0u};
-      }
+      for (int s = 0; s < 4; ++s) ka[u][s] = pok[u] ? ld16(kp + 32 * s) : u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < 4; ++u) {
+      const bool in_sink = t0 + 4 * u < n_sink;
+      const int lo = in_sink ? 0 : w_beg, hi = in_sink ? s_end : L;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < 4; ++s) acc = mfma16x16x32<DT>(ka[u][s], qv[s], acc);
+      for (int s = 0; s < 4; ++s) acc = mfma16x16x32<DT>(ka[u][s], qv[s], acc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = 16 * (pg + u) + 4 * kg + r;
-          // the weight rounded to fp16 as the prefill kernel summed it (see above)
-          const float p = (float)(_Float16)fast_exp2(__builtin_fmaf(acc[r], sl2, -m));
-          part += (pok[u] && key >= lo && key < hi && key <= pos) ? p : 0.f;
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int key = 16 * pg[u] + 4 * kg + r;
+        // the weight rounded to fp16 as the prefill kernel summed it (see above)
+        const float p = (float)(_Float16)fast_exp2(__builtin_fmaf(acc[r], sl2, -m));
+        part += (pok[u] && key >= lo && key < hi && key <= pos) ? p : 0.f;
       }
     }
-  };
-  const int s_end = min(a.sink, L), w_beg = max(L - a.obs, a.sink);
-  pages(0, (s_end + 15) >> 4, 0, s_end);
-  pages(w_beg >> 4, (L + 15) >> 4, w_beg, L);
+  }
   part += __shfl_xor(part, 16);
   part += __shfl_xor(part, 32);
+  if (kg == 0) wave_part[wv][i16] = part;
+  __syncthreads();
+  if (wv > 0) return;
+  part = (wave_part[0][i16] + wave_part[1][i16]) + (wave_part[2][i16] + wave_part[3][i16]);
   if (kg == 0 && live) {
     float2 res = make_float2(0.f, 1.f);
     if (ok) {
@@ -1535,8 +1545,8 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
     // them from the keys.
     const int obs_rows = obs && fine ? a.obs : 0;
     if (fine) a.obs = 0;
-    const int64_t finish_waves = obs && !fine ? (int64_t)batch * n_groups * ((a.obs * n_rep + 15) / 16) : 0;
-    if (wgs > INT32_MAX || (finish_waves + 3) / 4 > INT32_MAX) return UKV_ERR_INVALID_ARGUMENT;
+    const int64_t finish_wgs = obs && !fine ? (int64_t)batch * n_groups * ((a.obs * n_rep + 15) / 16) : 0;
+    if (wgs > INT32_MAX || finish_wgs > INT32_MAX) return UKV_ERR_INVALID_ARGUMENT;
     if (wgs > 0) {
       // With statistics, the prefill kernel writes the observation rows' (m, l) pairs and
       // obs_rows_finish_kernel, next on the same stream, turns them into the rows.
@@ -1547,8 +1557,8 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
       const int64_t flags = (int64_t)batch * num_q_heads * a.obs;
       hipLaunchKernelGGL(obs_flag_kernel, dim3((unsigned)((flags + 255) / 256)), dim3(256), 0, stream, a, flags);
     }
-    if (finish_waves > 0) {
-      const dim3 fgrid((unsigned)((finish_waves + 3) / 4));
+    if (finish_wgs > 0) {
+      const dim3 fgrid((unsigned)finish_wgs);
       if (dtype == UKV_DTYPE_BF16)
         hipLaunchKernelGGL(obs_rows_finish_kernel<UKV_DTYPE_BF16>, fgrid, dim3(256), 0, stream, a);
       else
