@@ -139,3 +139,29 @@ def test_parts_are_taken_only_by_launches_short_of_blocks():
     assert lib.ukv_paged_prefill_workspace_bytes(0, 1, 1, 8, 2, 128, 4, 100) == 0
     assert lib.ukv_paged_prefill_workspace_bytes(1, 64, 64, 8, 2, 96, 4, 1000) == 0  # no tiled instance
     assert lib.ukv_paged_prefill_workspace_bytes(64, 64 * 2048, 2048, 32, 8, 128, 4, 1000) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("Hq,Hkv,sink,obs,chunks", [
+    (28, 4, 16, 64, [[700, 650], [400, 517]]), (7, 1, 4, 32, [[1900], [40]]), (6, 2, 0, 48, [[300, 90]]),
+    (10, 2, 64, 128, [[2500, 300], [128, 140]]),
+])
+def test_fine_statistics_match_the_oracle(cuda, dtype, Hq, Hkv, sink, obs, chunks):
+    """The statistics of head shapes whose n_rep does not divide 16: the weights' two parts are summed and
+    taken off alike, so a row's normaliser is off by the fp32 sums' rounding (well under 2^-15; log2 units)."""
+    from oracle import snapkv_oracle as so
+    from test_obs_stats import _f, _prefill
+
+    r = _prefill(cuda, dtype, chunks, Hq=Hq, Hkv=Hkv, layers=1, sink=sink, obs=obs, seed=13)
+    data = r["st"].data.cpu().numpy()
+    kept = 0
+    for b in range(len(chunks[0])):
+        want = so.obs_row_stats(_f(r["dense"][0][b], dtype), _f(r["q_obs"][b, 0], dtype), sink_len=sink, obs_len=obs,
+                                n_rep=r["n_rep"], scale=r["scale"])
+        got, flags = data[b, 0, :, :, 0], data[b, 0, :, :, 1]
+        ok = flags == 0
+        kept += int(ok.sum())
+        if ok.any():
+            assert np.abs(got - want)[ok].max() <= 2.0 ** -14, (b, np.abs(got - want)[ok].max())
+    assert kept > 0

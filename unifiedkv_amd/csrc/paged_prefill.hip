@@ -289,8 +289,9 @@ template <> struct PrefillSplit<UKV_DTYPE_F16> {
 //          parts' rounded weights are the ones an undivided pass would have summed.
 // With statistics (obs > 0) it also writes, for each of the sequence's last obs queries in the
 // block and each q head h, the pair (m, l) of the column's running max m (log2 units) and its
-// softmax denominator l (the sum of the fp16 weights 2^(s * scale * log2e - m) over every key the
-// query sees) into obs_stats[b * stats_seq_stride + h * obs + i], for obs_rows_finish_kernel.
+// softmax denominator l (the sum of the rounded weights 2^(s * scale * log2e - m) over every key the
+// query sees; FINE: with its lift, taken off m) into obs_stats[b * stats_seq_stride + h * obs + i],
+// for obs_rows_finish_kernel.
 template <int DT, int D, int WAVES, int CB, bool FINE, bool PARTS>
 __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, const int g, const int c0,
                                              const int part, PrefillLds<D>& lds) {
@@ -746,7 +747,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
         for (int e = 0; e < NE; ++e) orow[16 * e] = Elem<DT>::from_float(o[cb][e][r] * inv);
         if (i16 == 0 && qi >= C - a.obs)  // (never without statistics: obs = 0)
           a.obs_stats[(int64_t)b * a.stats_seq_stride + (int64_t)hh * a.obs + (qi - (C - a.obs))] =
-              make_float2(m_col, lacc[cb][r]);
+              make_float2(m_col - kLift, lacc[cb][r]);
       }
     }
   }
@@ -937,7 +938,8 @@ paged_prefill_kernel(const PrefillArgs a) {
 // sink and a 128-key window are one round of loads (one wave took them in four, 13.5 us a layer at 2
 // x 8 x 32 column blocks). Lane (i16, kg) holds column i16 and keys 4kg .. 4kg + 3 of each 16-key
 // page. (The (m, l) pairs exist only where the tiled kernel ran.)
-template <int DT>
+// FINE: the weights as the FINE instances sum them, in two parts.
+template <int DT, bool FINE>
 __global__ void __launch_bounds__(256) obs_rows_finish_kernel(const PrefillArgs a) {
   __shared__ float wave_part[4][16];
   const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
@@ -995,12 +997,26 @@ __global__ void __launch_bounds__(256) obs_rows_finish_kernel(const PrefillArgs 
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < 4; ++s) acc = mfma16x16x32<DT>(ka[u][s], qv[s], acc);
+      // the weights rounded as the prefill kernel summed them (see above)
+      float p[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p[r] = fast_exp2(__builtin_fmaf(acc[r], sl2, -m));
+      if constexpr (FINE) {
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          uint32_t h, l;
+          PrefillSplit<DT>::split(p[r], p[r + 1], h, l);
+          p[r] = Elem<DT>::lo(h) + Elem<DT>::lo(l);
+          p[r + 1] = Elem<DT>::hi(h) + Elem<DT>::hi(l);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = (float)(_Float16)p[r];
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = 16 * pg[u] + 4 * kg + r;
-        // the weight rounded to fp16 as the prefill kernel summed it (see above)
-        const float p = (float)(_Float16)fast_exp2(__builtin_fmaf(acc[r], sl2, -m));
-        part += (pok[u] && key >= lo && key < hi && key <= pos) ? p : 0.f;
+        part += (pok[u] && key >= lo && key < hi && key <= pos) ? p[r] : 0.f;
       }
     }
   }
@@ -1449,6 +1465,14 @@ void launch_tiled_dt(const PrefillArgs& a, bool fine, unsigned wgs, hipStream_t 
     launch_tiled<DT, 128, false, PARTS>(a, wgs, stream);
 }
 
+template <int DT>
+void launch_finish(const PrefillArgs& a, bool fine, dim3 grid, hipStream_t stream) {
+  if (fine)
+    hipLaunchKernelGGL((obs_rows_finish_kernel<DT, true>), grid, dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((obs_rows_finish_kernel<DT, false>), grid, dim3(256), 0, stream, a);
+}
+
 void launch_tiled_any(const PrefillArgs& a, int dtype, bool fine, unsigned wgs, hipStream_t stream) {
   const bool parts = a.n_parts > 1;
   if (dtype == UKV_DTYPE_BF16)
@@ -1541,11 +1565,11 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
       a.part_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + part_o_bytes(plan.parts, rows, head_dim));
     }
     const int64_t wgs = (int64_t)(a.n3 + a.n2) * plan.parts * pairs;
-    // FINE instances write no statistics: every row is flagged, and the scoring pass recomputes
+    // The 64-dim instances write no statistics: every row is flagged, and the scoring pass recomputes
     // them from the keys.
-    const int obs_rows = obs && fine ? a.obs : 0;
-    if (fine) a.obs = 0;
-    const int64_t finish_wgs = obs && !fine ? (int64_t)batch * n_groups * ((a.obs * n_rep + 15) / 16) : 0;
+    const int obs_rows = obs && head_dim == 64 ? a.obs : 0;
+    if (obs_rows > 0) a.obs = 0;
+    const int64_t finish_wgs = obs && obs_rows == 0 ? (int64_t)batch * n_groups * ((a.obs * n_rep + 15) / 16) : 0;
     if (wgs > INT32_MAX || finish_wgs > INT32_MAX) return UKV_ERR_INVALID_ARGUMENT;
     if (wgs > 0) {
       // With statistics, the prefill kernel writes the observation rows' (m, l) pairs and
@@ -1560,9 +1584,9 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
     if (finish_wgs > 0) {
       const dim3 fgrid((unsigned)finish_wgs);
       if (dtype == UKV_DTYPE_BF16)
-        hipLaunchKernelGGL(obs_rows_finish_kernel<UKV_DTYPE_BF16>, fgrid, dim3(256), 0, stream, a);
+        launch_finish<UKV_DTYPE_BF16>(a, fine, fgrid, stream);
       else
-        hipLaunchKernelGGL(obs_rows_finish_kernel<UKV_DTYPE_F16>, fgrid, dim3(256), 0, stream, a);
+        launch_finish<UKV_DTYPE_F16>(a, fine, fgrid, stream);
     }
   } else {
     const dim3 grid(total_q, num_q_heads);
