@@ -41,6 +41,7 @@ import numpy as np
 import torch
 
 from . import _ext, page_ops
+from .page16_native import _current_stream as _stream
 
 
 def selection_budget_blocks(L: int, *, block_size: int = 16, sink_len: int = 16, obs_len: int = 16,
@@ -85,7 +86,7 @@ def select_blocks(scores: torch.Tensor, k: int, n_valid: Optional[torch.Tensor] 
     code = _ext.load().ukv_select_topk(
         scores.data_ptr(), int(scores.stride(0)), rn.data_ptr() if rn is not None else None,
         rk.data_ptr() if rk is not None else None, rows, n, int(k), out.data_ptr(), int(out.stride(0)),
-        torch.cuda.current_stream(dev).cuda_stream)
+        _stream(dev))
     _ext.check(code, "ukv_select_topk")
     return out
 
@@ -138,10 +139,6 @@ class CompactionResult:
     page_lists: List[List[int]]  # new physical pages per sequence (shared by all layers)
     block_table: torch.Tensor    # int32 [batch, max_pages] device table of page_lists
     seq_lens: List[int]          # resident tokens per sequence (effective length)
-
-
-def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _host_ids(ids, dev) -> torch.Tensor:
@@ -301,7 +298,7 @@ def _pool_strides(pool):
     k = pool.k_cache
     if pool.v_cache.stride() != k.stride():
         raise ValueError("pool K and V must share strides")
-    return _ext.i64_array(k.stride()[:4])
+    return _ext.i64_tuple(k.stride()[:4])
 
 
 def write_block_indexed_layer(pool, layer_id: int, block_ids: Sequence[int], K: torch.Tensor, V: torch.Tensor,
@@ -396,7 +393,7 @@ def _writeback(pool, raw_by_layer, layer_id, block_ids, sel, *, src_len, sink, o
         _ext.ptr_array([t.data_ptr() for t in ks]), _ext.ptr_array([t.data_ptr() for t in vs]),
         _ext.i64_array(strides), int(src_len), int(sink), int(obs),
         sel.data_ptr() if sel is not None else None, int(sel.stride(0)) if sel is not None and sel.shape[0] > 1 else 0,
-        k, 1 if pad else 0, kc.data_ptr(), vc.data_ptr(), _ext.i64_array(kc.stride()[:4]), dst.data_ptr(),
+        k, 1 if pad else 0, kc.data_ptr(), vc.data_ptr(), _ext.i64_tuple(kc.stride()[:4]), dst.data_ptr(),
         len(block_ids), int(pool.N_total), len(layers), pool.num_kv_heads, pool.head_dim, _stream(dev))
     _ext.check(code, "ukv_retain_writeback_dense")
 

@@ -266,7 +266,7 @@ class DecodeBatch:
         flat = (ctypes.c_int32 * (3 * len(triples) or 1))(*[v for t in triples for v in t])
         lens_in = self._lens_dev[self._cur]
         lens_out = self._lens_dev[self._cur ^ 1] if lens else None
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = page16_native._current_stream(self.device)
         code = _ext.load().ukv_decode_prologue(
             self._table.data_ptr(), int(self._table.shape[1]), self.batch, lens_in.data_ptr(),
             lens_out.data_ptr() if lens_out is not None else None, flat, len(triples), stream)

@@ -139,7 +139,8 @@ def _current_stream(dev) -> int:
     """Handle of dev's current stream. torch's raw query costs ~0.2 us per call against ~4 us for
     torch.cuda.current_stream(dev).cuda_stream, which matters for small, launch-bound batches."""
     if _raw_stream is not None:
-        return _raw_stream(dev.index)
+        index = dev.index
+        return _raw_stream(torch.cuda.current_device() if index is None else index)
     return torch.cuda.current_stream(dev).cuda_stream
 
 

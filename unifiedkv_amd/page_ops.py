@@ -10,14 +10,13 @@ from typing import Optional, Sequence
 import torch
 
 from . import _ext
-
-
-def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+from .page16_native import _current_stream as _stream
 
 
 def _i32(ids, dev) -> torch.Tensor:
     if torch.is_tensor(ids):
+        if ids.dtype == torch.int32 and ids.device == dev and ids.is_contiguous():
+            return ids
         return ids.to(device=dev, dtype=torch.int32).contiguous()
     return torch.tensor(list(ids), dtype=torch.int32, device=dev)
 
@@ -59,8 +58,8 @@ def scatter_tokens(pool_layer: torch.Tensor, page_ids, dense: torch.Tensor, n_to
     if T <= 0:
         return
     code = _ext.load().ukv_kv_scatter_tokens(
-        pool_layer.data_ptr(), _ext.i64_array(pool_layer.stride()[:3]), dense.data_ptr(),
-        _ext.i64_array(dense.stride()[:2]), ids.data_ptr(), int(ids.numel()), int(pool_layer.shape[0]), T, bs,
+        pool_layer.data_ptr(), _ext.i64_tuple(pool_layer.stride()[:3]), dense.data_ptr(),
+        _ext.i64_tuple(dense.stride()[:2]), ids.data_ptr(), int(ids.numel()), int(pool_layer.shape[0]), T, bs,
         int(pool_layer.shape[2]), int(pool_layer.shape[3]), _stream(dev))
     _ext.check(code, "ukv_kv_scatter_tokens")
 
@@ -80,8 +79,8 @@ def gather_tokens(pool_layer: torch.Tensor, page_ids, n_tokens: int) -> torch.Te
     if T == 0:
         return out
     code = _ext.load().ukv_kv_gather_tokens(
-        pool_layer.data_ptr(), _ext.i64_array(pool_layer.stride()[:3]), out.data_ptr(),
-        _ext.i64_array(out.stride()[:2]), ids.data_ptr(), int(ids.numel()), int(pool_layer.shape[0]), T, bs, H, D,
+        pool_layer.data_ptr(), _ext.i64_tuple(pool_layer.stride()[:3]), out.data_ptr(),
+        _ext.i64_tuple(out.stride()[:2]), ids.data_ptr(), int(ids.numel()), int(pool_layer.shape[0]), T, bs, H, D,
         _stream(dev))
     _ext.check(code, "ukv_kv_gather_tokens")
     return out
@@ -119,7 +118,7 @@ def page_copy(src_pools: Sequence[torch.Tensor], dst_pools: Sequence[torch.Tenso
             raise ValueError("page_copy: per-layer id lists need one row per layer")
     code = _ext.load().ukv_page_copy(
         _ext.ptr_array([t.data_ptr() for t in src_pools]), _ext.ptr_array([t.data_ptr() for t in dst_pools]),
-        len(src_pools), _ext.i64_array(s0.stride()[:2]), _ext.i64_array(d0.stride()[:2]),
+        len(src_pools), _ext.i64_tuple(s0.stride()[:2]), _ext.i64_tuple(d0.stride()[:2]),
         si.data_ptr(), n if si.dim() == 2 else 0, di.data_ptr(), n if di.dim() == 2 else 0,
         n, L, page_elems, int(s0.shape[1]), int(d0.shape[1]), _stream(dev))
     _ext.check(code, "ukv_page_copy")
@@ -168,8 +167,8 @@ def kv_append(k_layer: torch.Tensor, v_layer: torch.Tensor, block_table: torch.T
     lens = old_lens.to(torch.int32).contiguous()
     new_lens = torch.empty_like(lens) if return_new_lens else None
     code = _ext.load().ukv_kv_append(
-        k_layer.data_ptr(), v_layer.data_ptr(), _ext.i64_array(k_layer.stride()[:3]),
-        _ext.i64_array(v_layer.stride()[:3]), k_new.data_ptr(), v_new.data_ptr(), _ext.i64_array(k_new.stride()[:2]),
+        k_layer.data_ptr(), v_layer.data_ptr(), _ext.i64_tuple(k_layer.stride()[:3]),
+        _ext.i64_tuple(v_layer.stride()[:3]), k_new.data_ptr(), v_new.data_ptr(), _ext.i64_tuple(k_new.stride()[:2]),
         bt.data_ptr(), int(bt.shape[1]), lens.data_ptr(), new_lens.data_ptr() if new_lens is not None else None,
         B, int(k_layer.shape[1]), int(k_layer.shape[2]), int(k_layer.shape[3]), int(k_layer.shape[0]), _stream(dev))
     _ext.check(code, "ukv_kv_append")

@@ -24,6 +24,8 @@ _DTYPE_CODES = {torch.float16: _ext.UKV_DTYPE_F16, torch.bfloat16: _ext.UKV_DTYP
 def _i32(t, dev):
     if not torch.is_tensor(t):
         t = torch.tensor(list(t), dtype=torch.int32)
+    elif t.dtype == torch.int32 and t.device == dev and t.is_contiguous():
+        return t
     return t.to(device=dev, dtype=torch.int32).contiguous()
 
 
@@ -85,10 +87,10 @@ def write_chunk_kv(k_layer: torch.Tensor, v_layer: torch.Tensor, k_new: torch.Te
         raise RuntimeError("paged_prefill_shape_unsupported:batch")
     mc = _max_chunk(cu_seqlens_q, max_chunk, chunk_lens)
     code = _ext.load().ukv_kv_write_varlen(
-        k_layer.data_ptr(), v_layer.data_ptr(), _ext.i64_array(k_layer.stride()[:3]),
-        _ext.i64_array(v_layer.stride()[:3]), k_new.data_ptr(), v_new.data_ptr(), _ext.i64_array(k_new.stride()[:2]),
+        k_layer.data_ptr(), v_layer.data_ptr(), _ext.i64_tuple(k_layer.stride()[:3]),
+        _ext.i64_tuple(v_layer.stride()[:3]), k_new.data_ptr(), v_new.data_ptr(), _ext.i64_tuple(k_new.stride()[:2]),
         bt.data_ptr(), int(bt.shape[1]), cu.data_ptr(), lens.data_ptr(), B, mc, int(k_layer.shape[2]),
-        int(k_layer.shape[3]), int(k_layer.shape[0]), torch.cuda.current_stream(dev).cuda_stream)
+        int(k_layer.shape[3]), int(k_layer.shape[0]), _current_stream(dev))
     _ext.check(code, "ukv_kv_write_varlen")
 
 
@@ -154,8 +156,8 @@ def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     out = torch.empty((total_q, Hq, D), dtype=q.dtype, device=dev)
     args = [q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr(), cu.data_ptr(), lens.data_ptr(),
             out.data_ptr(), B, total_q, mc, Hq, Hkv, D, int(n_rep), int(bt.shape[1]),
-            min(int(k_cache.shape[0]), int(v_cache.shape[0])), _ext.i64_array(q.stride()[:2]),
-            _ext.i64_array(k_cache.stride()[:3]), _ext.i64_array(v_cache.stride()[:3]), float(softmax_scale),
+            min(int(k_cache.shape[0]), int(v_cache.shape[0])), _ext.i64_tuple(q.stride()[:2]),
+            _ext.i64_tuple(k_cache.stride()[:3]), _ext.i64_tuple(v_cache.stride()[:3]), float(softmax_scale),
             _DTYPE_CODES[q.dtype]]
     lib = _ext.load()
     # The parts' scratch comes from the caching allocator, which keeps it for this stream's kernels.
@@ -163,7 +165,7 @@ def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
     stats_args = (0, 0, None, 0) if stats_view is None else (obs_stats.sink_len, obs_stats.obs_len, *stats_view)
     code = lib.ukv_paged_prefill_parts(*args, *stats_args, ws.data_ptr() if ws is not None else None, need,
-                                       torch.cuda.current_stream(dev).cuda_stream)
+                                       _current_stream(dev))
     if code == _ext.UKV_OK and stats_view is not None:
         obs_stats.mark(layer_id, seq_lens)
     if code != _ext.UKV_OK:
@@ -304,15 +306,15 @@ class PrefillPages:
             return
         if self._strides is None:  # the pool's layer strides, fixed for its life
             kl = pool.k_cache[0]
-            self._strides = (_ext.i64_array(kl.stride()[:3]), _ext.i64_array(pool.v_cache[0].stride()[:3]),
+            self._strides = (_ext.i64_tuple(kl.stride()[:3]), _ext.i64_array(pool.v_cache[0].stride()[:3]),
                              int(pool.k_cache.stride(0)) * pool.k_cache.element_size(),
                              int(pool.v_cache.stride(0)) * pool.v_cache.element_size())
         ks, vs, kl_bytes, vl_bytes = self._strides
         code = _ext.load().ukv_kv_write_varlen(
             pool.k_cache.data_ptr() + layer_id * kl_bytes, pool.v_cache.data_ptr() + layer_id * vl_bytes, ks, vs,
-            k_new.data_ptr(), v_new.data_ptr(), _ext.i64_array(k_new.stride()[:2]), c["bt"].data_ptr(),
+            k_new.data_ptr(), v_new.data_ptr(), _ext.i64_tuple(k_new.stride()[:2]), c["bt"].data_ptr(),
             int(c["bt"].shape[1]), c["cu"].data_ptr(), c["kv"].data_ptr(), len(self._lists), c["max_chunk"],
-            pool.num_kv_heads, pool.head_dim, pool.N_total, torch.cuda.current_stream(self.dev).cuda_stream)
+            pool.num_kv_heads, pool.head_dim, pool.N_total, _current_stream(self.dev))
         _ext.check(code, "ukv_kv_write_varlen")
 
     def attention(self, layer_id: int, q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, *,

@@ -23,6 +23,7 @@ from typing import Optional
 import torch
 
 from . import _ext
+from .page16_native import _current_stream
 
 _DTYPES = {torch.float16: _ext.UKV_DTYPE_F16, torch.bfloat16: _ext.UKV_DTYPE_BF16}
 
@@ -77,11 +78,11 @@ def _run(q, q_strides, k, k_strides, table, max_blocks, num_pages, layers, seqs,
     ws_bytes = int(lib.ukv_snapkv_workspace_bytes(layers, seqs, seq_len, sink_len, obs_len, num_q_heads,
                                                   num_kv_heads, head_dim, n_rep, block_size))
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=q.device)
-    args = [q.data_ptr(), _ext.i64_array(q_strides), k.data_ptr(), _ext.i64_array(k_strides),
+    args = [q.data_ptr(), _ext.i64_tuple(q_strides), k.data_ptr(), _ext.i64_tuple(k_strides),
             table.data_ptr() if table is not None else None, int(max_blocks), int(num_pages),
             layers, seqs, seq_len, sink_len, obs_len, num_q_heads, num_kv_heads, head_dim, n_rep, block_size,
             float(scale), _DTYPES[q.dtype]]
-    tail = [out.data_ptr(), int(out.stride(0)), ws.data_ptr(), ws.numel(), torch.cuda.current_stream(q.device).cuda_stream]
+    tail = [out.data_ptr(), int(out.stride(0)), ws.data_ptr(), ws.numel(), _current_stream(q.device)]
     if stats is None:
         code = lib.ukv_snapkv_scores(*args, *tail)
         _ext.check(code, "ukv_snapkv_scores")
