@@ -778,22 +778,36 @@ __global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs 
   const int Lk = kv_len_of(a, b);
   const int nt = (Lk + TK - 1) / TK, np = part_count(a, nt);
   const int pos = Lk - C + qi;
-  int n = 0;  // parts that hold the row's keys
-  while (n < np && pos >= 0 && (int)((int64_t)n * nt / np) * TK <= pos) ++n;
+  // Parts that start at or below the row's tile p: s * nt / np <= p iff s < ceil((p + 1) np / nt).
+  const int n = pos < 0 ? 0 : min(np, (int)(((uint32_t)(pos / TK + 1) * np + nt - 1) / (uint32_t)nt));
   const int64_t stride = (int64_t)a.total_q * a.Hq;
-  float M = kNegFltMax;
-  for (int s = 0; s < n; ++s) M = fmaxf(M, a.part_ml[s * stride + idx].x);
+  float M = kNegFltMax, l = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  float l = 0.f;
   bool flagged = false;
-#pragma unroll 4
-  for (int s = 0; s < n; ++s) {
-    const float2 ml = a.part_ml[s * stride + idx];
-    const f32x4 x = *reinterpret_cast<const f32x4*>(a.part_o + (s * stride + idx) * D + 4 * dq);
-    const float w = fast_exp2(ml.x - M);
-    flagged |= __builtin_signbit(ml.y);
-    l += w * fabsf(ml.y);
-    acc += w * x;
+  for (int s0 = 0; s0 < n; s0 += 4) {
+    float2 ml[4];
+    f32x4 x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool in = s0 + u < n;
+      const int64_t at = (int64_t)(in ? s0 + u : s0) * stride + idx;
+      ml[u] = a.part_ml[at];
+      x[u] = *reinterpret_cast<const f32x4*>(a.part_o + at * D + 4 * dq);
+      if (!in) ml[u] = make_float2(kNegFltMax, 0.f);
+    }
+    const float top = fmaxf(M, fmaxf(fmaxf(ml[0].x, ml[1].x), fmaxf(ml[2].x, ml[3].x)));
+    const float f = fast_exp2(M - top);
+    l *= f;
+    acc *= f;
+    M = top;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (s0 + u >= n) continue;
+      const float w = fast_exp2(ml[u].x - M);
+      flagged |= __builtin_signbit(ml[u].y);
+      l += w * fabsf(ml[u].y);
+      acc += w * x[u];
+    }
   }
   const float inv = 1.f / l;
   const uint32_t w0 = Elem<DT>::from_float(acc[0] * inv) | (uint32_t)Elem<DT>::from_float(acc[1] * inv) << 16;
