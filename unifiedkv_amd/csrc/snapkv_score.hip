@@ -170,6 +170,10 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
   const u32x4 colsel = u32x4{l16 == 0 ? kOnes : 0u, l16 == 0 ? kOnes : 0u, l16 == 4 ? kOnes : 0u,
                              l16 == 4 ? kOnes : 0u};
 
+  // The wave's row tiles belong to one q head of the unit (TW divides its tiles): which one, and its first query
+  // there. (Per-lane divisions by obs at every unit's start took ~2 us.)
+  const int wave_h = wv * TW / tph, wave_q0 = (wv * TW - wave_h * tph) * 16;
+
   if constexpr (SCORES)
     for (int i = tid; i < (t1 - t0) * kSnapTile; i += blockDim.x) lds.colmax[i] = 0.f;
 
@@ -196,20 +200,23 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
       lsum[k] = f32x4{0.f, 0.f, 0.f, 0.f};
       const int tile = wv * TW + k;
       const bool on = tile < T;
-      const int rr = tile * 16 + l16;  // A row of this lane
-      const uint16_t* qp = a.q + (int64_t)item * a.q_si + (int64_t)(h0 + rr / a.obs) * a.q_sh +
-                           (int64_t)(rr % a.obs) * a.q_st + 8 * lg;
+      const int q0 = wave_q0 + 16 * k;  // the tile's first query of q head h0 + wave_h
+      const uint16_t* qp = a.q + (int64_t)item * a.q_si + (int64_t)(h0 + wave_h) * a.q_sh +
+                           (int64_t)(q0 + l16) * a.q_st + 8 * lg;  // A row of this lane
 #pragma unroll
       for (int st = 0; st < STEPS; ++st) qa[k][st] = on ? ld16(qp + 32 * st) : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+      for (int r = 0; r < 4; ++r)
         m[k][r] = INFINITY;  // pass 1: kLift1 - max with max = -inf; pass 2: rows past the unit weigh 0
-        if constexpr (SCORES) {
-          if (on) {  // C rows 4*lg + r of the tile
-            const int row = tile * 16 + 4 * lg + r;
-            m[k][r] = a.stats[(int64_t)item * rows_all + (int64_t)(h0 + row / a.obs) * a.obs + row % a.obs].x -
-                      kLift2;
-          }
+      if constexpr (SCORES) {
+        if (on) {  // C rows 4*lg + r of the tile
+          const f32x4* st = reinterpret_cast<const f32x4*>(
+              a.stats + (int64_t)item * rows_all + (int64_t)(h0 + wave_h) * a.obs + q0 + 4 * lg);
+          const f32x4 s01 = st[0], s23 = st[1];
+          m[k][0] = s01[0] - kLift2;
+          m[k][1] = s01[2] - kLift2;
+          m[k][2] = s23[0] - kLift2;
+          m[k][3] = s23[2] - kLift2;
         }
       }
     }
@@ -438,8 +445,7 @@ __global__ void __launch_bounds__(64 * kSnapWaves, 2) snap_tile_kernel(const Sna
       for (int k = 0; k < TW; ++k) {
         const int tile = wv * TW + k;
         if (tile < T && lg == 0) {
-          const int row = tile * 16 + l16;
-          const int64_t grow = (int64_t)(h0 + row / a.obs) * a.obs + row % a.obs;
+          const int64_t grow = (int64_t)(h0 + wave_h) * a.obs + wave_q0 + 16 * k + l16;
           a.part_stats[((int64_t)item * a.S + s) * rows_all + grow] =
               make_float2(kLift1 - m[k][0], lsum[k][0] * (1.f / 128.f));
         }
