@@ -44,12 +44,12 @@
 //   * shapes whose n_rep does not divide 16, and 64-dim heads, run FINE instances: columns are
 //     (query, head) pairs laid end to end, so every column of the matrix cores is used, V keeps its
 //     type and P goes in as two 16-bit parts (fp32-grade weights, as the scalar kernel they ran on
-//     before had): 28 q heads on 4 KV heads, 4 x 512 queries over 0.5-8K keys in 0.33 ms against
+//     before had): 28 q heads on 4 KV heads, 4 x 512 queries over 5-8K keys in 0.314 ms against
 //     72.7 ms; twelve 64-dim prompts of 16-700 tokens in 0.055 ms against 6.4 ms (0.10 ms with one
 //     workgroup per CU, three column blocks, 64-key tiles and the pairs' blocks in turn);
 //   * key parts: a launch of few query blocks leaves CUs idle however long its prefix. Its keys are
 //     then cut into equal parts, each (block, part) a workgroup, and a merge kernel adds the parts
-//     up: one 389-query chunk behind 32256 keys (40 blocks) in 0.23 ms against 0.86 ms;
+//     up: one 389-query chunk behind 32256 keys (40 blocks) in 0.22 ms against 0.86 ms;
 //   * SnapKV row statistics: the blocks holding each sequence's last obs queries
 //     also write those rows' running max and denominator; obs_rows_finish_kernel
 //     then sums the sink and window keys' weights again from the same scores and
