@@ -197,6 +197,16 @@ def _check_keep(keep: torch.Tensor, n_pages: int, what: str) -> None:
         raise ValueError(f"{what}: retained page indices outside [0, {n_pages})")
 
 
+def _keep_ids(keep: torch.Tensor, n_pages: int, dev, what: str) -> torch.Tensor:
+    """Retained indices as int32 rows on dev. Other types are checked at 64 bits first: a narrower one
+    cannot hold every page count it would be compared with, a wider one would wrap when narrowed."""
+    if keep.dtype != torch.int32:
+        keep = keep.to(device=dev, dtype=torch.long)
+        _check_keep(keep, n_pages, what)
+    keep = keep.to(device=dev, dtype=torch.int32)
+    return keep if keep.stride(1) == 1 else keep.contiguous()
+
+
 def compact(pool, seq_page_lists: Sequence[Sequence[int]], retained: Sequence[torch.Tensor],
             seq_lens: Sequence[int], *, free_sources: bool = False) -> CompactionResult:
     """Gather each sequence's retained pages into freshly allocated pages of the same pool.
@@ -220,10 +230,7 @@ def compact(pool, seq_page_lists: Sequence[Sequence[int]], retained: Sequence[to
         if keep.dim() != 2 or int(keep.shape[0]) != L:
             raise ValueError("compact: retained index rows must match the pool's layers")
         page_arrays.append(_check_pool_ids(pool, pages, f"compact: sequence {s}"))
-        if keep.dtype != torch.int32:  # checked at its own width before it is narrowed
-            _check_keep(keep, len(pages), f"compact: sequence {s}")
-        keep = keep.to(device=dev, dtype=torch.int32)
-        keeps.append(keep if keep.stride(1) == 1 else keep.contiguous())
+        keeps.append(_keep_ids(keep, len(pages), dev, f"compact: sequence {s}"))
     src = _source_ids(pool, page_arrays, keeps)
     at = 0
     if free_sources:
