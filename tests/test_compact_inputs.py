@@ -17,3 +17,13 @@ def test_indices_are_checked_wider_than_their_type(dtype, n_pages):
 def test_wide_indices_are_refused_before_they_are_narrowed(value):
     with pytest.raises(ValueError, match=r"outside \[0, 300\)"):
         compaction._keep_ids(torch.tensor([[0, value]]), 300, torch.device("cpu"), "t")
+
+
+@pytest.mark.parametrize("bad", [-1, 10, 2 ** 31, 2 ** 40, 2 ** 63, 2 ** 70, -2 ** 70])
+def test_page_ids_of_any_size_are_refused_alike(bad):
+    class Pool:
+        N_total = 10
+
+    with pytest.raises(ValueError, match="outside the pool"):
+        compaction._check_pool_ids(Pool, [1, bad, 2], "t")
+    assert [int(x) for x in compaction._check_pool_ids(Pool, [1.0, 9], "t")] == [1, 9]

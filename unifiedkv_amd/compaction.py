@@ -146,11 +146,11 @@ def _host_ids(ids, dev) -> torch.Tensor:
 
 
 def _id_array(ids) -> np.ndarray:
-    """A list of ids as an integer array (int32 where they fit)."""
+    """A list of ids as an integer array (int32 where they fit; Python ints of any size otherwise)."""
     try:
         return np.frombuffer(array.array("i", ids), dtype=np.int32) if len(ids) else np.zeros(0, np.int32)
     except (TypeError, OverflowError):  # not plain ints, or beyond 32 bits
-        return np.array([int(x) for x in ids], dtype=np.int64)
+        return np.array([int(x) for x in ids], dtype=object)
 
 
 def _check_pool_ids(pool, ids, what) -> np.ndarray:
