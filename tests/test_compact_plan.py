@@ -28,6 +28,26 @@ def test_retained_pages(cuda, k, sink, obs):
                 compaction.retained_pages(L, bad, sink_len=sink, obs_len=obs)
 
 
+def test_retained_pages_with_nothing_selected_can_be_captured(cuda):
+    sel = torch.empty((3, 0), dtype=torch.int32, device=cuda)
+    want = compaction.retained_pages(16 * 8, sel, sink_len=32, obs_len=16)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = compaction.retained_pages(16 * 8, sel, sink_len=32, obs_len=16)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert got.tolist() == want.tolist() == [[0, 1, 7]] * 3
+
+
+def test_retained_pages_of_more_rows_than_a_grid_takes(cuda):
+    sel = torch.arange(65600, dtype=torch.int32, device=cuda).remainder_(5).unsqueeze(1)
+    got = compaction.retained_pages(16 * 8, sel, sink_len=32, obs_len=16)
+    assert torch.equal(got[:, 1:3].cpu(), torch.stack([torch.ones(65600, dtype=torch.int32), sel[:, 0].cpu() + 2], 1))
+
+
 def _pool(cuda, layers, n):
     pool = PagedKVPool(16, layers, 2, 64, torch.float16, num_blocks=n, device=cuda)
     g = torch.Generator(device=cuda).manual_seed(0)

@@ -102,7 +102,10 @@ def retained_pages(L: int, selected_mid: torch.Tensor, *, block_size: int = 16, 
     if L % B or sink_len % B or obs_len % B:
         raise ValueError("retained_pages: the page-granular path needs block-aligned L, sink and window")
     n_mid = (L - sink_len - obs_len) // B
+    # The kernel's flag costs a synchronisation: with nothing selected there is nothing to check, and the
+    # expressions below stay capturable. One grid row per layer bounds its layers.
     if (selected_mid.is_cuda and selected_mid.dtype == torch.int32 and selected_mid.dim() == 2
+            and selected_mid.numel() and int(selected_mid.shape[0]) <= 65535
             and selected_mid.stride(1) == 1 and n_mid >= 0):
         return _retained_pages_gpu(selected_mid, n_mid, sink_len // B, (L - obs_len) // B, obs_len // B)
     if selected_mid.numel() and bool(((selected_mid < 0) | (selected_mid >= n_mid)).any()):
