@@ -9,6 +9,7 @@ error 2^-12 each) get 2^-11 of the largest |V|.
 """
 import numpy as np
 import pytest
+import torch
 
 from oracle import oracle
 from test_prefill import check, expected, make_case, run_gpu, to_dev
@@ -65,6 +66,28 @@ def test_key_parts_match_the_closed_form(cuda, n_rep, Hkv, D, prefix, chunk, dty
     fine = D != 128 or 16 % n_rep
     _close(out.float().cpu().numpy(), expected(case), _v_max(case), dtype, 2.0 ** -15 if fine else 2.0 ** -11,
            f"parts n_rep={n_rep} Hkv={Hkv} D={D} prefix={prefix} chunk={chunk} {dtype}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_rep,Hkv,D,prefix,chunk", [PARTS[0], PARTS[3], PARTS[5]])
+def test_a_launch_without_room_for_its_parts_runs_in_one(cuda, n_rep, Hkv, D, prefix, chunk, monkeypatch):
+    case = make_case(n_rep * 10 + D + sum(prefix), prefix, chunk, Hq=n_rep * Hkv, Hkv=Hkv, D=D, dtype="bf16")
+    assert _parts_bytes(case) > 0
+    empty, refused = torch.empty, []
+
+    def no_scratch(*args, **kw):
+        if kw.get("dtype") is torch.uint8:
+            refused.append(args)
+            raise torch.OutOfMemoryError("no room")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_scratch)
+    out, _ = run_gpu(case, cuda)
+    monkeypatch.undo()
+    assert refused
+    fine = D != 128 or 16 % n_rep
+    _close(out.float().cpu().numpy(), expected(case), _v_max(case), "bf16", 2.0 ** -15 if fine else 2.0 ** -11,
+           f"one part n_rep={n_rep} Hkv={Hkv} D={D}")
 
 
 @pytest.mark.gpu

@@ -162,7 +162,12 @@ def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     lib = _ext.load()
     # The parts' scratch comes from the caching allocator, which keeps it for this stream's kernels.
     need = lib.ukv_paged_prefill_workspace_bytes(B, total_q, mc, Hq, Hkv, D, int(n_rep), int(bt.shape[1]))
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    ws = None
+    if need:
+        try:
+            ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        except torch.OutOfMemoryError:  # without scratch the keys stay in one part
+            need = 0
     stats_args = (0, 0, None, 0) if stats_view is None else (obs_stats.sink_len, obs_stats.obs_len, *stats_view)
     code = lib.ukv_paged_prefill_parts(*args, *stats_args, ws.data_ptr() if ws is not None else None, need,
                                        _current_stream(dev))
