@@ -48,13 +48,15 @@ struct DecodeArgs {
   uint16_t* out;
   float* part_o;     // [slots][Hq][D], slots = grid_wgs + B
   float2* part_ml;   // [slots][Hq]: (running max in log2 units, sum of exp2)
-  int32_t* seq_start;  // [B] first global page of each sequence (written by workgroup 0)
+  int32_t* seq_start;  // [B] first global page of each sequence (written by workgroup 0); entry 0, whose
+                       // page is 0, holds the shares the pages were cut into
   int32_t* seq_pages;  // [B] pages of each sequence
   int64_t q_sb, q_sh;
   int64_t k_sp, k_st, k_sh;
   int64_t v_sp, v_st, v_sh;
   int B, Hq, n_rep, n_groups, D, max_blocks, num_pages;
-  int grid_wgs;      // G: workgroups sharing the batch's pages
+  int grid_wgs;      // workgroups sharing the batch's pages (the most shares they are cut into)
+  int fixed_shares;  // cut them into exactly grid_wgs shares (launch-shape sweeps)
   int subs;          // waves of a workgroup that share each KV head's pages (split kernel, SHARED)
   // Decode-token append (fused variant): k_new/v_new [B][n_groups][D] rows with
   // strides n_sb, n_sh; the token of sequence b goes to position lens[b] - 1.
@@ -90,6 +92,28 @@ __device__ __forceinline__ int mul_div(int x, int y, int z) {
   const uint64_t p = (uint64_t)(uint32_t)x * (uint32_t)y;
   if ((p >> 32) == 0) return (int)((uint32_t)p / (uint32_t)z);
   return (int)(p / (uint32_t)z);
+}
+
+// Largest of the wave's 64 values (>= 0), in every lane.
+__device__ __forceinline__ int wave_max_i32(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Shares the batch's P pages are cut into, at most G. The host sees the table's width alone; here the
+// lengths say how much there is to share: a page more in a share costs ~0.85 us, a share more of the
+// longest sequence ~0.05 us in the merge, so a share takes about sqrt(longest) / 4 pages. One sequence
+// of 4096 tokens beside three of 17: 16.8 us with 72 shares, 23.9 with 256, 21.2 with 32; four of 128
+// pages keep their 128 shares. A multiple of 8 (G too, or it is taken whole) for the XCDs' equal runs.
+__device__ __forceinline__ int shares_for(const DecodeArgs& a, int P, int longest) {
+  if (a.fixed_shares) return a.grid_wgs;
+  const int per = max(1, (int)(0.25f * __builtin_sqrtf((float)longest) + 0.5f));
+  return min(a.grid_wgs, max(8, ((P + per - 1) / per + 7) & ~7));
 }
 
 // Splits fp32 softmax weights into two 16-bit parts (p ~= hi + lo, relative
@@ -234,16 +258,22 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   const int subs = DIRECT ? UKV_PAGE16_WAVES : SHARED ? a.subs : 1;
   const int g = DIRECT ? (int)blockIdx.y : SHARED ? wv - sub * a.n_groups : blockIdx.z * (blockDim.x >> 6) + wv;
   if (!SHARED && g >= a.n_groups) return;  // whole wave leaves; only SHARED has barriers below
-  const int G = a.grid_wgs;
-  // Share w of the page list runs on workgroup blockIdx.x = 8 * (w % (G/8)) + w / (G/8): dispatch
+  // Share w of the page list's G runs on workgroup blockIdx.x = 8 * (w % (G/8)) + w / (G/8): dispatch
   // puts workgroup i on XCD i % 8, so XCD x runs the contiguous shares x*G/8 .. (x+1)*G/8 - 1 and
   // the shares that carry one page more than the average (their positions follow P/G) spread evenly
   // over the XCDs instead of gathering on a few of them. Which workgroup runs a share does not
-  // change its pages, slot or result.
-  const int w = (G & 7) == 0 ? (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  // change its pages, slot or result. Workgroups past the shares have nothing to do.
+  int w = 0;
   const bool writer = blockIdx.x == 0 && blockIdx.z == 0 && wv == 0;
+  auto share = [&](int G, int P, int& x0, int& x1) {
+    w = (G & 7) == 0 ? (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    x0 = x1 = 0;
+    if ((int)blockIdx.x >= G) return;
+    x0 = mul_div(w, P, G);
+    x1 = mul_div(w + 1, P, G);
+  };
 
-  // The batch's pages in sequence order form one list of P pages; workgroup w
+  // The batch's pages in sequence order form one list of P pages; share w
   // takes pages [w*P/G, (w+1)*P/G), crossing sequence boundaries as needed. Exclusive
   // prefix sums of pages per sequence give P and the sequence holding page x0. A batch of up
   // to 64 sequences is scanned once and its lengths stay in the lanes' registers.
@@ -261,22 +291,25 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
     const int incl = wave_inclusive_scan_i32(n);
     P = __builtin_amdgcn_readlane(incl, 63);
     nonempty = __ballot(n > 0);
+    const int G = shares_for(a, P, wave_max_i32(n));
     if (writer && lane < a.B) {
-      a.seq_start[lane] = incl - n;
+      a.seq_start[lane] = lane == 0 ? G : incl - n;
       a.seq_pages[lane] = n;
     }
-    x0 = mul_div(w, P, G);
-    x1 = mul_div(w + 1, P, G);
+    share(G, P, x0, x1);
     if (x0 >= x1) return;
     b_first = __builtin_ctzll(__ballot(n > 0 && incl > x0));
     s_first = __builtin_amdgcn_readlane(incl - n, b_first);
   } else {
+    int longest = 0;
     for (int c0 = 0; c0 < a.B; c0 += 64) {
       const int bb = c0 + lane;
-      P += __builtin_amdgcn_readlane(wave_inclusive_scan_i32(bb < a.B ? pages_of(a.lens[bb], a.max_blocks) : 0), 63);
+      const int n = bb < a.B ? pages_of(a.lens[bb], a.max_blocks) : 0;
+      P += __builtin_amdgcn_readlane(wave_inclusive_scan_i32(n), 63);
+      longest = max(longest, wave_max_i32(n));
     }
-    x0 = mul_div(w, P, G);
-    x1 = mul_div(w + 1, P, G);
+    const int G = shares_for(a, P, longest);
+    share(G, P, x0, x1);
     if (x0 >= x1 && !writer) return;
     int carry = 0;
     for (int c0 = 0; c0 < a.B; c0 += 64) {
@@ -285,7 +318,7 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
       const int incl = wave_inclusive_scan_i32(n);
       const int start = carry + incl - n;
       if (writer && bb < a.B) {
-        a.seq_start[bb] = start;
+        a.seq_start[bb] = bb == 0 ? G : start;
         a.seq_pages[bb] = n;
       }
       if (b_first < 0) {
@@ -614,7 +647,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 
 // Merges the partials of one (sequence, q head): log-sum-exp in log2 units.
 // The sequence's pages [S, S+n) of the batch's P pages were split over
-// workgroups w = floor(((S+1)G - 1)/P) .. floor(((S+n)G - 1)/P), whose partials
+// shares w = floor(((S+1)G - 1)/P) .. floor(((S+n)G - 1)/P), whose partials
 // sit in slots w + b. 256 threads: thread (cs, dq) owns float4 dims 4*dq.. of
 // partials cs, cs+CS, ...; it issues the loads of its first kPre rows together
 // with the (m, l) loads, so that one memory round trip serves both. Every wave computes
@@ -631,9 +664,9 @@ __global__ void __launch_bounds__(256) page16_combine_kernel(const DecodeArgs a)
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int n_pages = a.seq_pages[b];
-  const int P = a.seq_start[a.B - 1] + a.seq_pages[a.B - 1];
-  const int S = a.seq_start[b];
-  const int G = a.grid_wgs;
+  const int P = (a.B > 1 ? a.seq_start[a.B - 1] : 0) + a.seq_pages[a.B - 1];
+  const int S = b > 0 ? a.seq_start[b] : 0;
+  const int G = a.seq_start[0];
   auto share_of = [&](int x) -> int {  // floor(((x + 1) G - 1) / P): the share holding page x
     const uint64_t p = (uint64_t)(uint32_t)(x + 1) * (uint32_t)G - 1;
     return (p >> 32) == 0 ? (int)((uint32_t)p / (uint32_t)P) : (int)(p / (uint32_t)P);
@@ -798,8 +831,8 @@ int env_wgs() {
 // Workgroups G sharing the batch's pages: one per CU (a single round of equal
 // workgroups measured fastest), fewer when even the largest possible batch
 // (batch * max_blocks pages) gives each fewer than kMinPagesPerWg pages, but one per sequence (a
-// workgroup takes its segments one after another); a multiple of 8 for the XCDs' equal runs. Four
-// sequences of 256-2048 tokens: 12.7 us with 4 pages, 16.1 with 8, 15.4 with 2. Partials
+// workgroup takes its segments one after another); a multiple of 8 for the XCDs' equal runs. The lengths
+// may lower it on the device (shares_for). Partials
 // beyond kMaxPartials bytes keep the coarser rule. UKV_PAGE16_WGS overrides it for launch-shape sweeps.
 constexpr size_t kMaxPartials = size_t(16) << 20;
 int split_wgs_for(int batch, int hq, int d, int max_blocks) {
@@ -996,6 +1029,7 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
     a.seq_start = reinterpret_cast<int32_t*>(ws + w.seq_off);
     a.seq_pages = a.seq_start + batch;
     a.grid_wgs = w.wgs;
+    a.fixed_shares = env_wgs() > 0;
     if (fused) {
       a.k_new = static_cast<const uint16_t*>(tok->k);
       a.v_new = static_cast<const uint16_t*>(tok->v);
