@@ -35,6 +35,7 @@ CUTS = [
     (32, 8, [4096, 17, 17, 17], 256, 76, 32), (4, 1, [4096, 17, 17, 17], 256, 76, 32),
     (32, 8, [1040] + [17] * 15, 65, 80, 40), (32, 8, [4096] + [17] * 69, 256, 176, 96),
     (32, 8, [100, 200, 250, 300], 256, 60, 48), (32, 8, [2048] * 4, 128, 132, 128),
+    (16, 16, [4090] * 4, 256, 132, 128),  # two workgroups a share: one round of them
 ]
 
 

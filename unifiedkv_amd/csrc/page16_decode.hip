@@ -835,15 +835,28 @@ int env_wgs() {
 // may lower it on the device (shares_for). Partials
 // beyond kMaxPartials bytes keep the coarser rule. UKV_PAGE16_WGS overrides it for launch-shape sweeps.
 constexpr size_t kMaxPartials = size_t(16) << 20;
+long long coarse_wgs(int batch, int max_blocks) {  // one per eight pages the table holds
+  const long long bound = (long long)batch * (long long)std::max(max_blocks, 1);
+  return std::max<long long>(1, std::min<long long>(device_cu_count(), (bound + 7) / 8));
+}
 int split_wgs_for(int batch, int hq, int d, int max_blocks) {
   if (const int v = env_wgs()) return v;
   const long long bound = (long long)batch * (long long)std::max(max_blocks, 1);
-  const long long cus = device_cu_count();
-  const long long coarse = std::max<long long>(1, std::min(cus, (bound + 7) / 8));
+  const long long cus = device_cu_count(), coarse = coarse_wgs(batch, max_blocks);
   const long long want = std::max<long long>((bound + kMinPagesPerWg - 1) / kMinPagesPerWg, batch);
   const long long g = std::max(coarse, std::min(cus, (want + 7) / 8 * 8));
   const bool fits = (size_t)(g + batch) * hq * (d + 2) * sizeof(float) <= kMaxPartials;
   return (int)(fits ? g : coarse);
+}
+
+// More KV heads than a workgroup's waves take several workgroups a share: the finer split stops where these
+// fill the CUs, as a second round costs more than it spreads (4 x 4096 tokens on 16 heads of 128 dims, one
+// workgroup to a CU: 26.4 us with 128 shares, 37 with 256).
+int launch_wgs(int wgs, int batch, int max_blocks, int n_groups) {
+  const int per_share = (n_groups + UKV_PAGE16_WAVES - 1) / UKV_PAGE16_WAVES;
+  if (per_share == 1 || env_wgs()) return wgs;
+  const int one_round = std::max(8, (device_cu_count() / per_share) & ~7);
+  return (int)std::max<long long>(coarse_wgs(batch, max_blocks), std::min(wgs, one_round));
 }
 
 // kDirect: a CU streams at most ~47 GB/s (32 KB in flight against ~0.7 us), so a sequence on one
@@ -1028,7 +1041,7 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
     a.part_ml = reinterpret_cast<float2*>(ws + w.part_ml_off);
     a.seq_start = reinterpret_cast<int32_t*>(ws + w.seq_off);
     a.seq_pages = a.seq_start + batch;
-    a.grid_wgs = w.wgs;
+    a.grid_wgs = launch_wgs(w.wgs, batch, max_blocks, n_groups);
     a.fixed_shares = env_wgs() > 0;
     if (fused) {
       a.k_new = static_cast<const uint16_t*>(tok->k);
