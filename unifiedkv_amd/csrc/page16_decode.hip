@@ -112,7 +112,9 @@ __device__ __forceinline__ int wave_max_i32(int x) {
 // pages keep their 128 shares. A multiple of 8 (G too, or it is taken whole) for the XCDs' equal runs.
 __device__ __forceinline__ int shares_for(const DecodeArgs& a, int P, int longest) {
   if (a.fixed_shares) return a.grid_wgs;
-  const int per = max(1, (int)(0.25f * __builtin_sqrtf((float)longest) + 0.5f));
+  // (the square root is vector code: its result back to a scalar register, with all that follows from it; three
+  // more vector registers would leave the 64-dim split one workgroup to a CU)
+  const int per = max(1, __builtin_amdgcn_readfirstlane((int)(0.25f * __builtin_sqrtf((float)longest) + 0.5f)));
   return min(a.grid_wgs, max(8, ((P + per - 1) / per + 7) & ~7));
 }
 
@@ -263,14 +265,10 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
   // the shares that carry one page more than the average (their positions follow P/G) spread evenly
   // over the XCDs instead of gathering on a few of them. Which workgroup runs a share does not
   // change its pages, slot or result. Workgroups past the shares have nothing to do.
-  int w = 0;
+  int w = 0, G = 0;
   const bool writer = blockIdx.x == 0 && blockIdx.z == 0 && wv == 0;
-  auto share = [&](int G, int P, int& x0, int& x1) {
-    w = (G & 7) == 0 ? (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-    x0 = x1 = 0;
-    if ((int)blockIdx.x >= G) return;
-    x0 = mul_div(w, P, G);
-    x1 = mul_div(w + 1, P, G);
+  auto share_of_workgroup = [&]() -> int {
+    return (G & 7) == 0 ? (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
   };
 
   // The batch's pages in sequence order form one list of P pages; share w
@@ -291,12 +289,15 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
     const int incl = wave_inclusive_scan_i32(n);
     P = __builtin_amdgcn_readlane(incl, 63);
     nonempty = __ballot(n > 0);
-    const int G = shares_for(a, P, wave_max_i32(n));
+    G = shares_for(a, P, wave_max_i32(n));
     if (writer && lane < a.B) {
       a.seq_start[lane] = lane == 0 ? G : incl - n;
       a.seq_pages[lane] = n;
     }
-    share(G, P, x0, x1);
+    if ((int)blockIdx.x >= G) return;
+    w = share_of_workgroup();
+    x0 = mul_div(w, P, G);
+    x1 = mul_div(w + 1, P, G);
     if (x0 >= x1) return;
     b_first = __builtin_ctzll(__ballot(n > 0 && incl > x0));
     s_first = __builtin_amdgcn_readlane(incl - n, b_first);
@@ -308,8 +309,11 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
       P += __builtin_amdgcn_readlane(wave_inclusive_scan_i32(n), 63);
       longest = max(longest, wave_max_i32(n));
     }
-    const int G = shares_for(a, P, longest);
-    share(G, P, x0, x1);
+    G = shares_for(a, P, longest);
+    if ((int)blockIdx.x >= G) return;
+    w = share_of_workgroup();
+    x0 = mul_div(w, P, G);
+    x1 = mul_div(w + 1, P, G);
     if (x0 >= x1 && !writer) return;
     int carry = 0;
     for (int c0 = 0; c0 < a.B; c0 += 64) {
