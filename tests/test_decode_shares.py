@@ -55,3 +55,17 @@ def test_cuts_around_the_rule_s_steps(cuda, Hkv, lens):
     case = custom_case(len(lens), len(lens), 2 * Hkv, Hkv, 64, lens, max_blocks=90)
     slots, out = _slots_written(case, cuda)
     assert_close(out, expected_dense(case), f"lens {lens[-3:]} Hkv={Hkv}")
+
+
+@pytest.mark.parametrize("B,Hkv,n_rep,D,max_blocks,direct", [
+    (64, 8, 4, 128, 64, False), (64, 8, 4, 128, 33, False), (64, 8, 4, 128, 32, True),  # 512 pairs on 256 CUs
+    (32, 8, 4, 128, 64, True), (16, 8, 4, 128, 65, False), (15, 8, 4, 128, 33, False),
+    (64, 16, 1, 128, 16, False), (64, 16, 1, 128, 8, True), (32, 16, 1, 128, 24, False), (128, 8, 2, 128, 32, False),
+    (64, 16, 1, 64, 32, False), (64, 8, 1, 64, 48, False), (256, 8, 1, 64, 32, True),
+])
+def test_short_tables_leave_what_does_not_fit_at_once_to_the_split(cuda, B, Hkv, n_rep, D, max_blocks, direct):
+    """The one-kernel form of short tables writes no partials. One long sequence among short ones."""
+    case = custom_case(B + D, B, Hkv * n_rep, Hkv, D, [17] * (B - 1) + [16 * max_blocks], max_blocks=max_blocks)
+    slots, out = _slots_written(case, cuda)
+    assert_close(out, expected_dense(case), f"B={B} Hkv={Hkv} n_rep={n_rep} D={D} table {max_blocks}")
+    assert (slots == 0) == direct, slots

@@ -865,13 +865,23 @@ int launch_wgs(int wgs, int batch, int max_blocks, int n_groups) {
 
 // kDirect: a CU streams at most ~47 GB/s (32 KB in flight against ~0.7 us), so a sequence on one
 // workgroup per KV head pays only while its pages are few: per layer of a step at 512 tokens 7-10 us
-// against 9-13 (1-8 sequences) and 14.5 / 24.7 against 19.4 / 29.3 us (32 / 64 sequences, 8 KV heads); at
-// 1024 it wins where the (sequence, head) pairs fill half of the CUs (24.9 / 44.0 against 28.7 / 48.8 us)
-// and loses below (15.7 against 14.3 us at 8 x 8, 11.4 against 9.4 at 8 x 1).
+// against 9-13 (1-8 sequences) and 14.5 / 24.7 against 19.4 / 29.3 us (32 / 64 sequences, 8 KV heads). At
+// 1024 it wins where the (sequence, head) pairs fill half of the CUs (17 against 21 us at 128 pairs, 24
+// against 29 at 256) and loses below (15.7 against 14.3 us at 8 x 8, 11.4 against 9.4 at 8 x 1). Pairs
+// beyond the workgroups the device holds (one to a CU at 128 dims, two at 64) wait ~2.9 us a round behind
+// the short sequences before a long one starts: 64 sequences on 8 heads, one of 1024 tokens among 17s, took
+// 20.2 us against 15.3 for the split. There the longer tables are left to the split, and with few q heads a KV
+// head, whose merge is cheap, all but the shortest (as many q heads as KV heads, one long sequence: 32 x 16 in
+// 24 pages 12.6 against 11.3 us, 64 x 16 in 16 pages 16.1 against 14.5; 128 x 8 at two q heads a KV head in 32
+// pages 18.4 against 16.1, in 16 pages 15 against 17; 256 x 16 one-page sequences 41 against 35).
 constexpr int kDirectPages = 32, kDirectPagesWide = 64;
-bool direct_shape(int batch, int n_groups, int head_dim, int max_blocks) {
+bool direct_shape(int batch, int n_groups, int n_rep, int head_dim, int max_blocks) {
   if (head_dim > 128 || n_groups > 65535 || env_wgs()) return false;
-  return max_blocks <= ((long long)batch * n_groups >= device_cu_count() / 2 ? kDirectPagesWide : kDirectPages);
+  const long long pairs = (long long)batch * n_groups, cus = device_cu_count();
+  const long long held = head_dim == 64 ? 2 * cus : cus;
+  if (max_blocks > (pairs >= cus / 2 && pairs <= cus ? kDirectPagesWide : kDirectPages)) return false;
+  if (pairs <= held || n_rep >= 4 || (head_dim == 64 && n_groups <= UKV_PAGE16_WAVES)) return true;
+  return pairs <= 8 * held && pairs * max_blocks <= held * (head_dim == 64 ? 48 : n_rep == 1 ? 40 : 80);
 }
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -900,7 +910,7 @@ template <int DT, int D>
 void launch_split(const DecodeArgs& a, hipStream_t stream) {
   // Waves left over by the KV heads share the heads' pages (D = 256 has no LDS for their rows).
   if constexpr (D <= 128) {
-    if (direct_shape(a.B, a.n_groups, a.D, a.max_blocks)) {
+    if (direct_shape(a.B, a.n_groups, a.n_rep, a.D, a.max_blocks)) {
       const dim3 grid(a.B, a.n_groups), block(64 * UKV_PAGE16_WAVES);
       if (a.k_new)
         hipLaunchKernelGGL((page16_split_kernel<DT, D, true, kDirect>), grid, block, 0, stream, a);
@@ -1057,7 +1067,7 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
         dtype == UKV_DTYPE_BF16 ? dispatch_split<UKV_DTYPE_BF16>(a, stream) : dispatch_split<UKV_DTYPE_F16>(a, stream);
     if (!launched) return UKV_ERR_LAUNCH;
     if (hipGetLastError() != hipSuccess) return UKV_ERR_LAUNCH;
-    if (!direct_shape(batch, n_groups, head_dim, max_blocks)) launch_combine(a, dtype, stream);
+    if (!direct_shape(batch, n_groups, n_rep, head_dim, max_blocks)) launch_combine(a, dtype, stream);
   } else {
     const dim3 grid(num_q_heads, batch);
     if (dtype == UKV_DTYPE_BF16)
