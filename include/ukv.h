@@ -82,7 +82,8 @@ int ukv_copy_2d(void* dst, size_t dst_pitch, const void* src, size_t src_pitch, 
 const char* ukv_status_string(int status);
 
 /*
- * Bytes of workspace ukv_page16_decode needs for this shape. The workspace
+ * Bytes of workspace ukv_page16_decode needs for this shape; never fewer for a larger argument, so
+ * a buffer sized for the largest shape serves every smaller one. The workspace
  * holds the split-K partial results (never read before written), so it needs
  * no initialisation and may be reused by consecutive calls on one stream.
  */

@@ -1,0 +1,29 @@
+"""Workspace size queries: a buffer sized for the largest shape of a range serves the smaller ones.
+
+CPU: without a device the library assumes 256 CUs, as the MI355X has.
+"""
+import itertools
+
+import pytest
+
+from unifiedkv_amd import _ext
+
+DECODE = dict(batch=[1, 2, 7, 16, 61, 128, 247, 248, 249, 250, 300, 1000], heads=[1, 8, 28, 32, 64, 96, 128],
+              dim=[64, 128, 256], pages=[1, 2, 4, 8, 16, 33, 64, 128, 512, 2048])
+
+
+@pytest.mark.parametrize("axis", list(DECODE))
+def test_decode_size_never_falls_as_the_shape_grows(axis):
+    size = _ext.load().ukv_page16_workspace_bytes
+    others = [k for k in DECODE if k != axis]
+    for rest in itertools.product(*(DECODE[k] for k in others)):
+        at = dict(zip(others, rest))
+        sizes = [int(size(*({**at, axis: x}[k] for k in DECODE))) for x in DECODE[axis]]
+        assert sizes == sorted(sizes), (axis, at, sizes)
+
+
+def test_decode_size_over_every_batch():
+    size = _ext.load().ukv_page16_workspace_bytes
+    for heads, dim, pages in [(64, 128, 4), (128, 256, 1), (28, 128, 40), (96, 128, 3)]:
+        sizes = [int(size(b, heads, dim, pages)) for b in range(1, 700)]
+        assert sizes == sorted(sizes), (heads, dim, pages)

@@ -843,14 +843,16 @@ long long coarse_wgs(int batch, int max_blocks) {  // one per eight pages the ta
   const long long bound = (long long)batch * (long long)std::max(max_blocks, 1);
   return std::max<long long>(1, std::min<long long>(device_cu_count(), (bound + 7) / 8));
 }
+long long fine_wgs(int batch, int max_blocks) {
+  const long long bound = (long long)batch * (long long)std::max(max_blocks, 1);
+  const long long want = std::max<long long>((bound + kMinPagesPerWg - 1) / kMinPagesPerWg, batch);
+  return std::max(coarse_wgs(batch, max_blocks), std::min<long long>(device_cu_count(), (want + 7) / 8 * 8));
+}
 int split_wgs_for(int batch, int hq, int d, int max_blocks) {
   if (const int v = env_wgs()) return v;
-  const long long bound = (long long)batch * (long long)std::max(max_blocks, 1);
-  const long long cus = device_cu_count(), coarse = coarse_wgs(batch, max_blocks);
-  const long long want = std::max<long long>((bound + kMinPagesPerWg - 1) / kMinPagesPerWg, batch);
-  const long long g = std::max(coarse, std::min(cus, (want + 7) / 8 * 8));
+  const long long g = fine_wgs(batch, max_blocks);
   const bool fits = (size_t)(g + batch) * hq * (d + 2) * sizeof(float) <= kMaxPartials;
-  return (int)(fits ? g : coarse);
+  return (int)(fits ? g : coarse_wgs(batch, max_blocks));
 }
 
 // More KV heads than a workgroup's waves take several workgroups a share: the finer split stops where these
@@ -893,15 +895,29 @@ struct WorkspaceLayout {
 
 // [slots][Hq][D] fp32 partials, [slots][Hq] (m, l), then the per-sequence page
 // starts and counts; slots = G + batch.
-WorkspaceLayout workspace_layout(int batch, int hq, int d, int max_blocks) {
+WorkspaceLayout layout_of(int wgs, int batch, int hq, int d) {
   WorkspaceLayout w{};
-  w.wgs = split_wgs_for(batch, hq, d, max_blocks);
+  w.wgs = wgs;
   const size_t slots = ((size_t)w.wgs + (size_t)batch) * hq;
   w.part_o_off = 0;
   w.part_ml_off = align256(slots * d * sizeof(float));
   w.seq_off = w.part_ml_off + align256(slots * sizeof(float2));
   w.total = w.seq_off + align256(2 * (size_t)batch * sizeof(int32_t));
   return w;
+}
+WorkspaceLayout workspace_layout(int batch, int hq, int d, int max_blocks) {
+  return layout_of(split_wgs_for(batch, hq, d, max_blocks), batch, hq, d);
+}
+
+// What the size query reports: no less than workspace_layout() takes, and never less for a larger batch,
+// table or head shape, so that one buffer sized for the largest serves the smaller ones (the layout itself
+// shrinks where the partials pass kMaxPartials).
+size_t workspace_report(int batch, int hq, int d, int max_blocks) {
+  if (env_wgs()) return workspace_layout(batch, hq, d, max_blocks).total;
+  const size_t fine = layout_of((int)fine_wgs(batch, max_blocks), batch, hq, d).total;
+  const size_t coarse = layout_of((int)coarse_wgs(batch, max_blocks), batch, hq, d).total;
+  const size_t most_fine = kMaxPartials + 2 * 256 + align256(2 * (size_t)batch * sizeof(int32_t));  // where it fits
+  return std::max(coarse, std::min(fine, most_fine));
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -973,7 +989,7 @@ using namespace ukv;
 
 extern "C" size_t ukv_page16_workspace_bytes(int batch, int num_q_heads, int head_dim, int max_blocks) {
   if (batch <= 0 || num_q_heads <= 0 || head_dim <= 0) return 0;
-  return workspace_layout(batch, num_q_heads, head_dim, max_blocks).total;
+  return workspace_report(batch, num_q_heads, head_dim, max_blocks);
 }
 
 namespace {
