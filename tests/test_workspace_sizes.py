@@ -27,3 +27,15 @@ def test_decode_size_over_every_batch():
     for heads, dim, pages in [(64, 128, 4), (128, 256, 1), (28, 128, 40), (96, 128, 3)]:
         sizes = [int(size(b, heads, dim, pages)) for b in range(1, 700)]
         assert sizes == sorted(sizes), (heads, dim, pages)
+
+
+@pytest.mark.parametrize("obs,dim,least,most", [(16, 64, 512, 1024), (64, 64, 512, 1024), (64, 128, 256, 512)])
+def test_scores_of_many_items_fill_what_a_cu_holds(obs, dim, least, most):
+    """Workgroups of 64 items of 8000 tokens, read off the size of their statistics' partials: a CU holds two
+    at 64 dims and one at 128."""
+    items, heads, seq_len = 64, 32, 8000
+    size = int(_ext.load().ukv_snapkv_workspace_bytes(items, 1, seq_len, 16, obs, heads, 8, dim, 4, 16))
+    row = items * heads * obs * 8  # one range's (m, l) of every row
+    blocks = (seq_len - 16 - obs + 15) // 16
+    ranges = (size - row - 4 * items * blocks) // row
+    assert least <= items * ranges <= most, ranges

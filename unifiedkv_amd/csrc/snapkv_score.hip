@@ -656,10 +656,12 @@ struct SnapPlan {
 
 // Key ranges S and unit groups of a call: rounds of one workgroup per CU, each taking units / groups
 // units of Kt / S tiles and a fixed cost per unit, kUnitTiles tile times (queries, statistics and first
-// keys: 64 ranges of 4 tiles over 8 units took 4.2 us a tile against 2.4 in long ranges). Groups cost the
-// finish a read of their running maxima.
-constexpr double kUnitTiles = 4.0;
-void choose_ranges(SnapPlan& p, int items, int units, int cus) {
+// keys: 64 ranges of 4 tiles over 8 units took 4.2 us a tile against 2.4 in long ranges). Where a CU holds two
+// workgroups (64 dims, up to two row tiles a wave: registers), two rounds run beside each other in kPairTime of
+// one: without it 64 items of 8000 tokens on 8 KV heads were planned as 256 long workgroups and took 426 us against
+// 327 as 512. Groups cost the finish a read of their running maxima.
+constexpr double kUnitTiles = 4.0, kPairTime = 1.54;
+void choose_ranges(SnapPlan& p, int items, int units, int cus, bool pairs) {
   const int need = (p.Kt * kSnapTile + kSnapMaxKeys - 1) / kSnapMaxKeys;
   double best = 0.0;
   for (int groups = 1; groups <= units; ++groups) {
@@ -667,8 +669,9 @@ void choose_ranges(SnapPlan& p, int items, int units, int cus) {
     const double finish = groups > 1 ? 1.0 + (double)items * groups * p.aligned * 8.0 / 4e6 / 2.4 : 0.0;
     for (int r = 0; r <= 8; ++r) {  // the most ranges that fill r rounds (0: the fewest allowed)
       const int S = std::min(p.Kt, std::max<int>(need, (int)((int64_t)r * cus / ((int64_t)items * groups))));
-      const int64_t rounds = ((int64_t)S * items * groups + cus - 1) / cus;
-      const double t = finish + (double)rounds * (units / groups) * ((p.Kt + S - 1) / S + kUnitTiles);
+      const int64_t n = ((int64_t)S * items * groups + cus - 1) / cus;
+      const double rounds = pairs ? (double)(n / 2) * kPairTime + (double)(n % 2) : (double)n;
+      const double t = finish + rounds * (units / groups) * ((p.Kt + S - 1) / S + kUnitTiles);
       if (best == 0.0 || t < 0.999 * best) {
         best = t;
         p.S = S;
@@ -710,7 +713,8 @@ SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, i
   p.tiled = (head_dim == 64 || head_dim == 128) && p.hp > 0 && aligned_rows;
   p.parts = p.tiled ? (n_rep + p.hp - 1) / p.hp : 1;
   p.S = p.groups = 1;
-  if (p.tiled) choose_ranges(p, items, num_q_heads / n_rep * p.parts, snap_cu_count());
+  if (p.tiled)
+    choose_ranges(p, items, num_q_heads / n_rep * p.parts, snap_cu_count(), head_dim == 64 && p.tw <= 2);
   const size_t rows_all = (size_t)num_q_heads * obs;
   p.part_off = 0;
   p.stats_off = a256((size_t)items * p.S * rows_all * sizeof(float2));
