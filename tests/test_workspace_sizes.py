@@ -29,13 +29,16 @@ def test_decode_size_over_every_batch():
         assert sizes == sorted(sizes), (heads, dim, pages)
 
 
-@pytest.mark.parametrize("obs,dim,least,most", [(16, 64, 512, 1024), (64, 64, 512, 1024), (64, 128, 256, 512)])
-def test_scores_of_many_items_fill_what_a_cu_holds(obs, dim, least, most):
-    """Workgroups of 64 items of 8000 tokens, read off the size of their statistics' partials: a CU holds two
-    at 64 dims and one at 128."""
-    items, heads, seq_len = 64, 32, 8000
-    size = int(_ext.load().ukv_snapkv_workspace_bytes(items, 1, seq_len, 16, obs, heads, 8, dim, 4, 16))
-    row = items * heads * obs * 8  # one range's (m, l) of every row
+@pytest.mark.parametrize("kv_heads,n_rep", [(8, 4), (2, 3)])
+@pytest.mark.parametrize("obs,dim,workgroups", [(16, 64, 512), (32, 64, 512), (64, 64, 512), (128, 64, 256), (64, 128, 256)])
+def test_scores_of_many_items_fill_what_a_cu_holds(obs, dim, workgroups, kv_heads, n_rep):
+    """The plan of 64 items of 8000 tokens (S key ranges and G unit groups an item), read off the size of its
+    scratch: S rows of statistics' partials, one of statistics, G running maxima a key (one sum a block where
+    G is 1). A CU holds two workgroups at 64 dims with up to two row tiles a wave, one otherwise."""
+    items, heads, seq_len = 64, kv_heads * n_rep, 8000
+    size = int(_ext.load().ukv_snapkv_workspace_bytes(items, 1, seq_len, 16, obs, heads, kv_heads, dim, n_rep, 16))
+    row = items * heads * obs * 8
     blocks = (seq_len - 16 - obs + 15) // 16
-    ranges = (size - row - 4 * items * blocks) // row
-    assert least <= items * ranges <= most, ranges
+    plans = [s * g for g in range(1, kv_heads * n_rep + 1) for s in range(1, 126)
+             if 0 <= size - ((s + 1) * row + items * blocks * (4 if g == 1 else 64 * g) + 4 * items) < 4 * 256]
+    assert plans and min(plans) * items == workgroups, plans
