@@ -421,7 +421,9 @@ int ukv_paged_prefill_parts(const void* q, const void* k_cache, const void* v_ca
  *                outside [0, num_pages) read as zero rows
  * num_q_heads must equal num_kv_heads * n_rep (q head h reads KV head h / n_rep); block_size must
  * be 16 (the page size; the reference's SnapKV block); layers * seqs <= 65535; otherwise
- * UKV_ERR_INVALID_ARGUMENT. The workspace (ukv_snapkv_workspace_bytes) needs no initialisation.
+ * UKV_ERR_INVALID_ARGUMENT. The workspace (ukv_snapkv_workspace_bytes) needs no initialisation. The
+ * size does not grow evenly with seq_len, but a buffer sized for a longer sequence serves every
+ * shorter one (with fewer key ranges or unit groups where it is short of the size for it).
  * Replaces core/scheduler.py:565-592 and the scoring steps of core/compress.py:116-130.
  */
 int ukv_snapkv_block_count(int seq_len, int sink_len, int obs_len, int block_size);

@@ -10,7 +10,7 @@ import torch
 
 from oracle import snapkv_oracle as so
 from test_random_shapes import _bits, _down, _f, _up
-from unifiedkv_amd import snapkv
+from unifiedkv_amd import _ext, snapkv
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +48,32 @@ def test_many_items_equal_the_same_items_alone(cuda):
     for b, l in ((0, 0), (2, 11), (3, 23)):
         one = snapkv.score_blocks(q[b:b + 1, l:l + 1].contiguous(), pool[l:l + 1], table[b:b + 1], **kw)
         torch.testing.assert_close(one[0], many[b * layers + l], rtol=2e-4, atol=1e-6)
+
+
+def _score_call(lib, q, k, out, L, obs, n_rep, size):
+    """ukv_snapkv_scores of dense K [layers][H][L][D] with a workspace of `size` bytes; returns the status."""
+    layers, H, _, D = k.shape
+    ws = torch.empty(max(size, 1), dtype=torch.uint8, device=k.device)
+    return lib.ukv_snapkv_scores(
+        q.data_ptr(), _ext.i64_array(q.stride()[:3]), k.data_ptr(),
+        _ext.i64_array((k.stride(0), 0, k.stride(2), k.stride(1))), None, 0, 0, layers, 1, L, 16, obs, H * n_rep, H, D,
+        n_rep, 16, D ** -0.5, _ext.UKV_DTYPE_F16, out.data_ptr(), out.stride(0), ws.data_ptr(), size,
+        torch.cuda.current_stream().cuda_stream)
+
+
+def test_a_workspace_sized_for_the_longest_sequence_serves_the_shorter_ones(cuda):
+    """Where a shorter sequence's own plan takes more scratch it runs with fewer ranges or groups; below the
+    least any plan takes it is refused."""
+    lib, layers, H, R, D, obs = _ext.load(), 12, 2, 2, 64, 32
+    size = lambda L: int(lib.ukv_snapkv_workspace_bytes(layers, 1, L, 16, obs, H * R, H, D, R, 16))
+    assert size(4100) < size(4050)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q = torch.randn((layers, H * R, obs, D), generator=g, device="cuda").half()
+    for L in (4050, 4100, 3000, 200):
+        k = torch.randn((layers, H, L, D), generator=g, device="cuda").half()
+        n = int(lib.ukv_snapkv_block_count(L, 16, obs, 16))
+        want, got = (torch.empty((layers, n), device="cuda") for _ in range(2))
+        assert _score_call(lib, q, k, want, L, obs, R, size(L)) == _ext.UKV_OK
+        assert _score_call(lib, q, k, got, L, obs, R, size(4100)) == _ext.UKV_OK, L
+        torch.testing.assert_close(got, want, rtol=2e-4, atol=1e-6)
+    assert _score_call(lib, q, k, got, 200, obs, R, 1024) == _ext.UKV_ERR_WORKSPACE

@@ -654,16 +654,26 @@ struct SnapPlan {
   size_t part_off, stats_off, raw_off, redo_off, total;  // raw_off: raw, or colbuf with several groups
 };
 
+void lay_out(SnapPlan& p, int items, int rows_all) {
+  p.part_off = 0;
+  p.stats_off = a256((size_t)items * p.S * rows_all * sizeof(float2));
+  p.raw_off = p.stats_off + a256((size_t)items * rows_all * sizeof(float2));
+  p.redo_off = p.raw_off + a256((size_t)items * (p.groups > 1 ? (size_t)p.groups * p.aligned : p.n_blocks) * sizeof(float));
+  p.total = p.redo_off + a256((size_t)items * sizeof(int32_t));
+}
+
 // Key ranges S and unit groups of a call: rounds of one workgroup per CU, each taking units / groups
 // units of Kt / S tiles and a fixed cost per unit, kUnitTiles tile times (queries, statistics and first
 // keys: 64 ranges of 4 tiles over 8 units took 4.2 us a tile against 2.4 in long ranges). Where a CU holds two
 // workgroups (64 dims, up to two row tiles a wave: registers), two rounds run beside each other in kPairTime of
 // one: without it 64 items of 8000 tokens on 8 KV heads were planned as 256 long workgroups and took 426 us against
-// 327 as 512. Groups cost the finish a read of their running maxima.
+// 327 as 512. Groups cost the finish a read of their running maxima. Only plans that fit `budget` bytes of
+// scratch are taken; the fewest ranges in one group where none does, which takes least.
 constexpr double kUnitTiles = 4.0, kPairTime = 1.54;
-void choose_ranges(SnapPlan& p, int items, int units, int cus, bool pairs) {
+void choose_ranges(SnapPlan& p, int items, int rows_all, int units, int cus, bool pairs, size_t budget) {
   const int need = (p.Kt * kSnapTile + kSnapMaxKeys - 1) / kSnapMaxKeys;
   double best = 0.0;
+  p.S = std::min(p.Kt, std::max(1, need));
   for (int groups = 1; groups <= units; ++groups) {
     if (units % groups != 0) continue;
     const double finish = groups > 1 ? 1.0 + (double)items * groups * p.aligned * 8.0 / 4e6 / 2.4 : 0.0;
@@ -673,16 +683,20 @@ void choose_ranges(SnapPlan& p, int items, int units, int cus, bool pairs) {
       const double rounds = pairs ? (double)(n / 2) * kPairTime + (double)(n % 2) : (double)n;
       const double t = finish + rounds * (units / groups) * ((p.Kt + S - 1) / S + kUnitTiles);
       if (best == 0.0 || t < 0.999 * best) {
+        SnapPlan at = p;
+        at.S = S;
+        at.groups = groups;
+        lay_out(at, items, rows_all);
+        if (at.total > budget) continue;
         best = t;
-        p.S = S;
-        p.groups = groups;
+        p = at;
       }
     }
   }
 }
 
 SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, int n_rep, int head_dim,
-                   int block_size, bool aligned_rows) {
+                   int block_size, bool aligned_rows, size_t budget = SIZE_MAX) {
   SnapPlan p{};
   p.L_mid = seq_len - sink - obs;
   p.aligned = ((std::max(1, p.L_mid) + block_size - 1) / block_size) * block_size;
@@ -713,14 +727,10 @@ SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, i
   p.tiled = (head_dim == 64 || head_dim == 128) && p.hp > 0 && aligned_rows;
   p.parts = p.tiled ? (n_rep + p.hp - 1) / p.hp : 1;
   p.S = p.groups = 1;
+  const int rows_all = num_q_heads * obs;
   if (p.tiled)
-    choose_ranges(p, items, num_q_heads / n_rep * p.parts, snap_cu_count(), head_dim == 64 && p.tw <= 2);
-  const size_t rows_all = (size_t)num_q_heads * obs;
-  p.part_off = 0;
-  p.stats_off = a256((size_t)items * p.S * rows_all * sizeof(float2));
-  p.raw_off = p.stats_off + a256((size_t)items * rows_all * sizeof(float2));
-  p.redo_off = p.raw_off + a256((size_t)items * (p.groups > 1 ? (size_t)p.groups * p.aligned : p.n_blocks) * sizeof(float));
-  p.total = p.redo_off + a256((size_t)items * sizeof(int32_t));
+    choose_ranges(p, items, rows_all, num_q_heads / n_rep * p.parts, snap_cu_count(), head_dim == 64 && p.tw <= 2, budget);
+  lay_out(p, items, rows_all);
   return p;
 }
 
@@ -818,8 +828,11 @@ int snapkv_scores_impl(const void* q_obs, const int64_t* q_strides, const void* 
   if (block_table && (max_blocks <= 0 || num_pages <= 0)) return UKV_ERR_INVALID_ARGUMENT;
   if ((int64_t)layers * seqs > 65535) return UKV_ERR_INVALID_ARGUMENT;
   const int items = layers * seqs;
-  const SnapPlan p = snap_plan(items, seq_len, sink_len, obs_len, num_q_heads, n_rep, head_dim, block_size,
-                               snap_aligned(q_obs, k, q_strides, k_strides));
+  const bool aligned_rows = snap_aligned(q_obs, k, q_strides, k_strides);
+  SnapPlan p = snap_plan(items, seq_len, sink_len, obs_len, num_q_heads, n_rep, head_dim, block_size, aligned_rows);
+  if (p.total > workspace_bytes)  // fewer ranges or unit groups, if that fits (a buffer sized for longer sequences does)
+    p = snap_plan(items, seq_len, sink_len, obs_len, num_q_heads, n_rep, head_dim, block_size, aligned_rows,
+                  workspace_bytes);
   if (!workspace || workspace_bytes < p.total || (reinterpret_cast<uintptr_t>(workspace) & 15u)) return UKV_ERR_WORKSPACE;
 
   SnapArgs a{};
