@@ -188,3 +188,68 @@ def test_fine_statistics_match_the_oracle(cuda, dtype, Hq, Hkv, sink, obs, chunk
         if ok.any():
             assert np.abs(got - want)[ok].max() <= 2.0 ** -14, (b, np.abs(got - want)[ok].max())
     assert kept > 0
+
+
+def _wide(case, width):
+    """The same case in a table of `width` pages a row (zero padded)."""
+    table = np.zeros((len(case["block_table"]), width), np.int32)
+    table[:, :case["block_table"].shape[1]] = case["block_table"]
+    return dict(case, block_table=table)
+
+
+def _parts_call(case, dev, poison):
+    """ukv_paged_prefill_parts over the written pool; returns (output, workspace filled with 0xFF before)."""
+    from unifiedkv_amd import prefill
+
+    t, lib = to_dev(case, dev), _ext.load()
+    mc, n_rep = max(case["chunk"]), case["n_rep"]
+    prefill.write_chunk_kv(t["k_cache"], t["v_cache"], t["k_new"], t["v_new"], t["block_table"], t["cu"], t["kv_lens"], mc)
+    (total, Hq, D), Hkv = t["q"].shape, t["k_cache"].shape[2]
+    size = _parts_bytes(case)
+    ws = torch.full((max(size, 1),), 0xFF, dtype=torch.uint8, device=dev)
+    out = torch.full_like(t["q"], poison)
+    code = lib.ukv_paged_prefill_parts(
+        t["q"].data_ptr(), t["k_cache"].data_ptr(), t["v_cache"].data_ptr(), t["block_table"].data_ptr(), t["cu"].data_ptr(),
+        t["kv_lens"].data_ptr(), out.data_ptr(), len(case["chunk"]), total, mc, Hq, Hkv, D, n_rep,
+        t["block_table"].shape[1], t["k_cache"].shape[0], _ext.i64_array(t["q"].stride()[:2]),
+        _ext.i64_array(t["k_cache"].stride()[:3]), _ext.i64_array(t["v_cache"].stride()[:3]), case["scale"],
+        {"bf16": _ext.UKV_DTYPE_BF16, "fp16": _ext.UKV_DTYPE_F16}[case["dtype"]], 0, 0, None, 0, ws.data_ptr(), size,
+        torch.cuda.current_stream().cuda_stream)
+    assert code == _ext.UKV_OK and size > 0
+    return out, ws
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("n_rep,Hkv,D,prefix,chunk", [
+    (4, 8, 128, [0, 0, 0, 0], [512, 512, 300, 512]), (4, 2, 128, [90, 0], [37, 64]), (7, 4, 128, [0, 17], [100, 129]),
+    (4, 2, 64, [0, 0, 5], [64, 1, 33]), (1, 3, 128, [700], [129]),
+])
+def test_a_table_wider_than_its_sequences_takes_no_partials(cuda, n_rep, Hkv, D, prefix, chunk, dtype):
+    """The plan knows the table's width alone and cuts such a launch; sequences that fill one part are written by
+    their blocks, as in an exact table, and leave the scratch as it was."""
+    case = _wide(make_case(n_rep + Hkv + D + sum(chunk), prefix, chunk, Hq=n_rep * Hkv, Hkv=Hkv, D=D, dtype=dtype), 2048)
+    out, ws = _parts_call(case, cuda, 7.0)
+    fine = D != 128 or 16 % n_rep
+    _close(out.float().cpu().numpy(), expected(case), _v_max(case), dtype, 2.0 ** -15 if fine else 2.0 ** -11,
+           f"wide table n_rep={n_rep} Hkv={Hkv} D={D} {prefix} {chunk}")
+    assert int((ws != 0xFF).sum()) == 0  # bytes written
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_rep,Hkv,D", [(4, 2, 128), (7, 1, 128), (4, 1, 64)])
+def test_sequences_in_one_part_beside_sequences_in_many(cuda, n_rep, Hkv, D):
+    """One long sequence is merged from its parts, short ones beside it are written whole, and a sequence
+    shorter than its chunk (its first queries before key 0) or empty gives NaN rows, as without parts."""
+    case = _wide(make_case(21 + D, [3000, 0, 0, 40], [70, 300, 6, 9], Hq=n_rep * Hkv, Hkv=Hkv, D=D, dtype="bf16"), 256)
+    want = expected(case)
+    lens = np.asarray(case["kv_lens"]).copy()
+    out, _ = _parts_call(case, cuda, 7.0)
+    fine = D != 128 or 16 % n_rep
+    tol = 2.0 ** -15 if fine else 2.0 ** -11
+    _close(out.float().cpu().numpy(), want, _v_max(case), "bf16", tol, "one long, three short")
+    lens[2], lens[3] = 0, 4  # no keys at all; nine queries of which five lie before the first key
+    out, _ = _parts_call(dict(case, kv_lens=lens), cuda, 7.0)
+    got = out.float().cpu().numpy()
+    _close(got[:370], want[:370], _v_max(case), "bf16", tol, "the others")
+    assert np.isnan(got[370:381]).all() and np.isfinite(got[381:]).all()

@@ -89,8 +89,9 @@ struct PrefillArgs {
   // Key split (n_parts > 1): the key tiles of a sequence are cut into part_count() <= n_parts equal
   // parts of about part_tiles tiles, each (query block, part) is a work item of its own, and
   // prefill_combine_kernel merges the parts' (m, l, O) from part_o / part_ml, rows
-  // [part][query row][q head] of D floats / one float2.
-  int n_parts, part_tiles;
+  // [part][query row][q head] of D floats / one float2. A sequence whose keys fill one part takes
+  // whole3 + whole2 blocks, the mix of a launch without parts, and writes its rows itself.
+  int n_parts, part_tiles, whole3, whole2;
   // Work items in block order (block j of every pair, then block j + 1) instead of pair after pair: for
   // launches whose blocks see very different key counts, longest first.
   int by_block;
@@ -284,8 +285,9 @@ template <> struct PrefillSplit<UKV_DTYPE_F16> {
 //   FINE   the weights keep fp32-grade precision (PrefillSplit) and V its own type: shapes whose
 //          n_rep does not divide 16 or whose D is 64. Otherwise n_rep divides 16 (a query's heads
 //          lie in one column block) and P and V are fp16.
-//   PARTS  part `part` of the sequence's keys (part_count() of them), left for
-//          prefill_combine_kernel. The running max moves to whole powers of two, so that the
+//   PARTS  part `part` of the sequence's keys (of np = part_count()), left for
+//          prefill_combine_kernel; a sequence in one part is written like an undivided one (every row
+//          through the partials cost 4 x 512-token prompts in a 2048-page table 53 us against 29). The running max moves to whole powers of two, so that the
 //          parts' rounded weights are the ones an undivided pass would have summed.
 // With statistics (obs > 0) it also writes, for each of the sequence's last obs queries in the
 // block and each q head h, the pair (m, l) of the column's running max m (log2 units) and its
@@ -294,7 +296,7 @@ template <> struct PrefillSplit<UKV_DTYPE_F16> {
 // for obs_rows_finish_kernel.
 template <int DT, int D, int WAVES, int CB, bool FINE, bool PARTS>
 __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, const int g, const int c0,
-                                             const int part, PrefillLds<D>& lds) {
+                                             const int part, const int np, PrefillLds<D>& lds) {
   constexpr int STEPS = D / 32;
   constexpr int NE = D / 16;  // output tiles of 16 dims
   constexpr int NT = 64 * WAVES;
@@ -333,11 +335,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   int P0 = Lk - C;  // keys before the chunk
   int kend = max(0, min(Lk, P0 + min(C, q1)));
   int key_a = 0;  // PARTS: first key of this part; Lk, P0 and kend count from it below
+  bool in_parts = false;  // the sequence's keys are in more parts than one (uniform)
   if constexpr (PARTS) {
-    const int nt = (Lk + TK - 1) / TK, np = part_count(a, nt);
+    const int nt = (Lk + TK - 1) / TK;
     if (part >= np) return;  // whole workgroup
+    in_parts = np > 1;
     key_a = (int)((int64_t)part * nt / np) * TK;
-    if (key_a >= kend) return;  // no row of the block sees this part (prefill_combine_kernel skips it)
+    if (in_parts && key_a >= kend) return;  // no row of the block sees this part (prefill_combine_kernel skips it)
     kend = min(kend, (int)((int64_t)(part + 1) * nt / np) * TK) - key_a;
     Lk -= key_a;
     P0 -= key_a;
@@ -715,9 +719,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   }
   if constexpr (kConvert || FINE) {
     if (__syncthreads_or(redo_mine)) {
-      if (!PARTS) flag_obs_rows<WAVES>(a, b, g, C, max(q0, 0), min(C, q1));  // (none without statistics)
+      if (!in_parts) flag_obs_rows<WAVES>(a, b, g, C, max(q0, 0), min(C, q1));  // (none without statistics)
       prefill_cols_fp32<DT, D>(a, b, g, q_begin, C, P0 + key_a, Lk + key_a, c0, WAVES * CB * 16, wv, WAVES, lane,
-                               PARTS ? part : -1, key_a, key_a + kend);
+                               in_parts ? part : -1, key_a, key_a + kend);
       return;
     }
   }
@@ -735,7 +739,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
       // the column's running max, held by lane col (column i16 = col)
       const float m_col = __shfl(m_ref[cb], col);
       if (qi >= 0 && qi < C && hh < a.Hq) {
-        if constexpr (PARTS) {
+        if (PARTS && in_parts) {
           // (FINE's lift by 2^kLift is in o and l alike: taken off the max)
           const int64_t row = ((int64_t)part * a.total_q + q_begin + qi) * a.Hq + hh;
           float* prow = a.part_o + row * D + i16;
@@ -756,16 +760,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
   }
 }
 
-// Merges the parts of each (query, q head) row: with M the largest of the parts' m, out = sum(2^(m - M) O) / sum(2^(m - M) l). A group of D / 4 lanes takes
-// a row, float4 dims 4 * lane ..; its parts' rows are read four at a time. Part s holds a row's
-// keys iff it starts at or below the row's position; the others were not written.
+// Merges the parts of each (query, q head) row of the sequences in more parts than one: with M the largest
+// of the parts' m, out = sum(2^(m - M) O) / sum(2^(m - M) l). A group of D / 4 lanes takes a row, float4 dims
+// 4 * lane ..; its parts' rows are read four at a time. Part s holds a row's keys iff it starts at or below
+// the row's position; the others were not written.
 template <int DT, int D>
-__global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs a) {
-  constexpr int LANES = D / 4, ROWS = 256 / LANES;
+__device__ __forceinline__ void prefill_combine_row(const PrefillArgs& a, const int64_t idx, const int dq) {
   constexpr int TK = kTileKeys;
-  const int64_t idx = (int64_t)blockIdx.x * ROWS + threadIdx.x / LANES;
-  if (idx >= (int64_t)a.total_q * a.Hq) return;
-  const int dq = threadIdx.x % LANES;
   const int row = (int)(idx / a.Hq), h = (int)(idx % a.Hq);
   int b = 0, hi = a.B;  // the last sequence starting at or before the row
   while (hi - b > 1) {
@@ -777,6 +778,7 @@ __global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs 
   if (qi < 0 || qi >= C || C > a.max_chunk) return;
   const int Lk = kv_len_of(a, b);
   const int nt = (Lk + TK - 1) / TK, np = part_count(a, nt);
+  if (np == 1) return;  // written whole by its block
   const int pos = Lk - C + qi;
   // Parts that start at or below the row's tile p: s * nt / np <= p iff s < ceil((p + 1) np / nt).
   const int n = pos < 0 ? 0 : min(np, (int)(((uint32_t)(pos / TK + 1) * np + nt - 1) / (uint32_t)nt));
@@ -816,6 +818,26 @@ __global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs 
   if (dq == 0 && qi >= C - a.obs)  // (never without statistics: obs = 0)
     a.obs_stats[(int64_t)b * a.stats_seq_stride + (int64_t)h * a.obs + (qi - (C - a.obs))] =
         flagged ? make_float2(NAN, 1.f) : make_float2(M, l);
+}
+
+template <int DT, int D>
+__global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs a) {
+  constexpr int LANES = D / 4, ROWS = 256 / LANES;
+  constexpr int TK = kTileKeys;
+  const int64_t rows = (int64_t)a.total_q * a.Hq, step = (int64_t)gridDim.x * ROWS;
+  if (step < rows) {
+    // Several rows a group: a table wider than its sequences may leave nothing to merge, which is then found
+    // once, by every wave.
+    bool any = false;
+    for (int b0 = 0; b0 < a.B && !any; b0 += 64) {
+      const int b = b0 + (threadIdx.x & 63);
+      any = __any(b < a.B && part_count(a, (kv_len_of(a, min(b, a.B - 1)) + TK - 1) / TK) > 1);
+    }
+    if (!any) return;
+  }
+  const int dq = threadIdx.x % LANES;
+  for (int64_t idx = (int64_t)blockIdx.x * ROWS + threadIdx.x / LANES; idx < rows; idx += step)
+    prefill_combine_row<DT, D>(a, idx, dq);
 }
 
 // Rows lo .. hi - 1 of sequence b's chunk, the q heads of KV group g, set to NaN (0x7FFF is a
@@ -889,52 +911,69 @@ __device__ __forceinline__ void xcd_range(int total, int xcd, int& start, int& e
 // statistics run the same instance: compiled with that epilogue, the tile loop's schedule is 0.7 %
 // faster at config 4 than without it.)
 //
-// With PARTS each block comes n_parts times, the blocks of one part next to each other.
+// With PARTS every XCD runs a range of the items for each part, part 0 first: the blocks of one part stay next
+// to each other, and where the table is wider than the sequences the workgroups without keys come last.
+// (Workgroups that exit at once among those that work, for the larger of two block counts, doubled launches
+// of one round: an XCD's shader engines take workgroups in turn, whatever they hold. So did the same four of 28
+// items a part on an XCD of 32 slots, nine times.)
 template <int DT, int D, int WAVES, bool FINE, bool PARTS>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 paged_prefill_kernel(const PrefillArgs a) {
   __shared__ PrefillLds<D> lds;
   constexpr int CB3 = wide_blocks(FINE, D), CB2 = CB3 - 1;
-  const int n_items = a.n3 + a.n2, parts = PARTS ? a.n_parts : 1;
-  int start, end, pair, j;
+  int n3 = a.n3, n2 = a.n2;
+  int start, end, pair, j, part = 0, np = 1;
   if (!PARTS && a.by_block) {
     const int pairs = a.n_groups * a.B;
     j = blockIdx.x / pairs;
     pair = blockIdx.x - j * pairs;
   } else {
-    xcd_range(n_items * parts * a.n_groups * a.B, blockIdx.x & 7, start, end);
-  if (!locate_item(start, end, n_items * parts, a.n3 * parts, blockIdx.x >> 3, pair, j)) return;  // (never: the grid holds total)
-  }
-  int part = 0;
-  if constexpr (PARTS) {
-    if (j < a.n3 * parts) {
-      part = j / a.n3;
-      j -= part * a.n3;
-    } else {
-      j -= a.n3 * parts;
-      part = j / a.n2;
-      j += a.n3 - part * a.n2;
+    const int n = n3 + n2;
+    const int total = n * a.n_groups * a.B, xcd = blockIdx.x & 7;
+    int s = blockIdx.x >> 3, range = xcd;
+    if constexpr (PARTS) {
+      // One range for every part; the total & 7 ranges with an item more go round the XCDs. An XCD had
+      // floor((xcd + (p - 1) rem) / 8) + (xcd < rem) of those in parts 0 .. p - 1.
+      const int per = total >> 3, rem = total & 7, first = xcd < rem ? 1 : 0;
+      auto before = [&](int p) -> int { return p == 0 ? 0 : p * per + ((xcd + (p - 1) * rem) >> 3) + first; };
+      part = s / (per + 1);  // at least
+      while (part < a.n_parts && s >= before(part + 1)) ++part;
+      if (part >= a.n_parts) return;
+      s -= before(part);
+      range = (xcd + part * rem) & 7;
     }
+    xcd_range(total, range, start, end);
+    if (!locate_item(start, end, n, n3, s, pair, j)) return;  // (never)
   }
   const int g = pair % a.n_groups, b = pair / a.n_groups;
   const int C = a.cu_q[b + 1] - a.cu_q[b];
+  if constexpr (PARTS) {
+    np = part_count(a, (kv_len_of(a, b) + kTileKeys - 1) / kTileKeys);
+    if (np == 1) {
+      j += part * (n3 + n2);  // its blocks in the items of every part
+      part = 0;
+      n3 = a.whole3;
+      n2 = a.whole2;
+      if (j >= n3 + n2) return;
+    }
+  }
   constexpr int w2 = WAVES * CB2 * 16, w3 = WAVES * CB3 * 16;
   if (C > a.max_chunk) {
     if (part > 0) return;
     const int cols = a.max_chunk * a.n_rep;  // the plan's columns, counted from the end of the chunk
-    const int c1 = cols - (j < a.n3 ? w3 * j : w3 * a.n3 + w2 * (j - a.n3)), c0 = c1 - (j < a.n3 ? w3 : w2);
+    const int c1 = cols - (j < n3 ? w3 * j : w3 * n3 + w2 * (j - n3)), c0 = c1 - (j < n3 ? w3 : w2);
     const int skip = C - a.max_chunk;
-    const int lo = j == n_items - 1 ? 0 : max(0, skip + (max(c0, 0) / a.n_rep));
+    const int lo = j == n3 + n2 - 1 ? 0 : max(0, skip + (max(c0, 0) / a.n_rep));
     const int hi = min(C, skip + (max(c1, 0) + a.n_rep - 1) / a.n_rep);
     prefill_nan_rows<WAVES>(a, b, g, lo, hi);
     flag_obs_rows<WAVES>(a, b, g, C, lo, hi);  // (none without statistics)
     return;
   }
   const int cols = C * a.n_rep;
-  if (j < a.n3)
-    prefill_tile<DT, D, WAVES, CB3, FINE, PARTS>(a, b, g, cols - w3 * (j + 1), part, lds);
+  if (j < n3)
+    prefill_tile<DT, D, WAVES, CB3, FINE, PARTS>(a, b, g, cols - w3 * (j + 1), part, np, lds);
   else
-    prefill_tile<DT, D, WAVES, CB2, FINE, PARTS>(a, b, g, cols - w3 * a.n3 - w2 * (j - a.n3 + 1), part, lds);
+    prefill_tile<DT, D, WAVES, CB2, FINE, PARTS>(a, b, g, cols - w3 * n3 - w2 * (j - n3 + 1), part, np, lds);
 }
 
 // SnapKV row statistics from the (m, l) pairs paged_prefill_kernel left in obs_stats.
@@ -1292,6 +1331,7 @@ namespace {
 struct BlockPlan {
   int n3, n2;
   int parts, part_tiles;
+  int whole3, whole2;  // the blocks of a pair whose keys fill one part (the table may be wider than they)
 };
 
 // The launch's predicted time when the blocks of every pair cost cost[0 .. n_items - 1], the first nl
@@ -1342,7 +1382,7 @@ struct PlanShape {
 
 BlockPlan choose_plan(const PlanShape& f) {
   const int n3_max = (int)((f.max_cols + f.w3 - 1) / f.w3);
-  BlockPlan best{n3_max, 0, 1, std::max(1, f.tiles)};
+  BlockPlan best{n3_max, 0, 1, std::max(1, f.tiles), n3_max, 0};
   // Large launches run many rounds, where the last one matters little: keep wide blocks.
   if (f.pairs * n3_max > (1 << 16) || f.slots_per_xcd <= 0 || n3_max == 0) return best;
   // Parts are considered for launches of few blocks: there whole blocks leave CUs idle.
@@ -1373,6 +1413,8 @@ BlockPlan choose_plan(const PlanShape& f) {
       best.n2 = n2;
     }
   }
+  best.whole3 = best.n3;
+  best.whole2 = best.n2;
   if (parts_ok) {
     // In tile times, each block as streaming the keys up to its last query's own.
     auto causal = [&](int n3, int n2, int parts) {
@@ -1397,7 +1439,7 @@ BlockPlan choose_plan(const PlanShape& f) {
         const double t = merge + causal(n3, n2, parts);
         if (t < 0.97 * best_t) {
           best_t = t;
-          best = BlockPlan{n3, n2, parts, (f.tiles + parts - 1) / parts};
+          best = BlockPlan{n3, n2, parts, (f.tiles + parts - 1) / parts, best.whole3, best.whole2};
         }
       }
     }
@@ -1460,15 +1502,18 @@ size_t part_bytes(int parts, int64_t rows, int head_dim) {
 // Partials above this are not worth their traffic: the launch is large enough without parts.
 constexpr size_t kMaxPartBytes = size_t(512) << 20;
 
+constexpr int kMergeWgs = 2048;
+
 template <int DT, int D, bool FINE, bool PARTS>
-void launch_tiled(const PrefillArgs& a, unsigned wgs, hipStream_t stream) {
+void launch_tiled(const PrefillArgs& a, unsigned tile_wgs, hipStream_t stream) {
   constexpr int W = UKV_PREFILL_WAVES;
-  hipLaunchKernelGGL((paged_prefill_kernel<DT, D, W, FINE, PARTS>), dim3(wgs), dim3(64 * W), 0, stream, a);
+  hipLaunchKernelGGL((paged_prefill_kernel<DT, D, W, FINE, PARTS>), dim3(tile_wgs), dim3(64 * W), 0, stream, a);
   if constexpr (PARTS) {
     constexpr int ROWS = 256 / (D / 4);
     const int64_t rows = (int64_t)a.total_q * a.Hq;
-    hipLaunchKernelGGL((prefill_combine_kernel<DT, D>), dim3((unsigned)((rows + ROWS - 1) / ROWS)), dim3(256), 0,
-                       stream, a);
+    // (eight workgroups a CU at once; rows beyond them are taken in turn)
+    const int64_t wgs = std::min<int64_t>((rows + ROWS - 1) / ROWS, kMergeWgs);
+    hipLaunchKernelGGL((prefill_combine_kernel<DT, D>), dim3((unsigned)wgs), dim3(256), 0, stream, a);
   }
 }
 
@@ -1572,6 +1617,8 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
     a.n2 = plan.n2;
     a.n_parts = plan.parts;
     a.part_tiles = plan.part_tiles;
+    a.whole3 = plan.whole3;
+    a.whole2 = plan.whole2;
     // No more keys than twice the chunk's: the blocks' key counts differ by a factor of two or more, and
     // every pair's longest blocks go first. (With a long prefix they are alike, and the blocks of one
     // pair stay together for their XCD's L2.)
@@ -1581,7 +1628,10 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
       a.part_o = static_cast<float*>(workspace);
       a.part_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + part_o_bytes(plan.parts, rows, head_dim));
     }
-    const int64_t wgs = (int64_t)(a.n3 + a.n2) * plan.parts * pairs;
+    // Parts: eight times what an XCD runs at most. (Two parts' items hold a pair's whole blocks: narrow ones are
+    // at least half as wide as wide ones.)
+    const int64_t items = pairs * (a.n3 + a.n2);
+    const int64_t wgs = plan.parts > 1 ? 8 * ((items * plan.parts + 7) / 8) : items;
     // The 64-dim instances write no statistics: every row is flagged, and the scoring pass recomputes
     // them from the keys.
     const int obs_rows = obs && head_dim == 64 ? a.obs : 0;
