@@ -57,14 +57,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <functional>
-#include <map>
-#include <mutex>
-#include <queue>
-#include <tuple>
 #include <type_traits>
-#include <vector>
 
+#include "prefill_plan.h"
 #include "ukv_common.h"
 
 namespace ukv {
@@ -154,7 +149,6 @@ __device__ __forceinline__ u32x2 ds_read_tr16(const uint16_t* p) {
 #define UKV_PREFILL_WAVES 8
 #endif
 
-constexpr int kTileKeys = 32;
 // LDS row pitches in 16-bit elements: K and V rows sit 288 B apart, the pitch
 // at which SQ_LDS_BANK_CONFLICT reads 0 for the 16-row x 16-byte K reads, the
 // 4-row x 32-byte V transpose reads and the 16-byte row stores (272 B leaves
@@ -1322,132 +1316,6 @@ extern "C" int ukv_kv_write_varlen(void* k_pool_layer, void* v_pool_layer, const
 }
 
 namespace {
-
-// Block plan of the tiled prefill: the numbers n3 and n2 of wide and narrow query blocks per
-// (sequence, KV group) that cover its chunk's max_chunk queries, and the parts its keys are cut
-// into. A launch runs in rounds of one block per slot (CU, or half a CU where two workgroups share
-// one); the plan with the shortest predicted launch is taken, modelling each XCD's slots as taking
-// the XCD's blocks in the kernel's order, each slot the next block once free.
-struct BlockPlan {
-  int n3, n2;
-  int parts, part_tiles;
-  int whole3, whole2;  // the blocks of a pair whose keys fill one part (the table may be wider than they)
-};
-
-// The launch's predicted time when the blocks of every pair cost cost[0 .. n_items - 1], the first nl
-// of them dispatched before the others.
-double plan_makespan(int64_t pairs, const std::vector<double>& cost, int nl, int slots_per_xcd) {
-  const int n_items = (int)cost.size();
-  const int64_t total = pairs * n_items;
-  const int64_t per = total / 8, rem = total % 8;
-  double worst = 0.0;
-  for (int x = 0; x < 8; ++x) {
-    const int64_t start = x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per;
-    const int64_t end = start + per + (x < rem ? 1 : 0);
-    std::priority_queue<double, std::vector<double>, std::greater<double>> slot;
-    for (int c = 0; c < slots_per_xcd; ++c) slot.push(0.0);
-    if (end > start)
-      for (int pass = 0; pass < 2; ++pass)
-        for (int64_t p = start / n_items; p <= (end - 1) / n_items; ++p) {
-          const int64_t j0 = std::max<int64_t>(pass ? nl : 0, start - p * n_items);
-          const int64_t j1 = std::min<int64_t>(pass ? n_items : nl, end - p * n_items);
-          for (int64_t j = j0; j < j1; ++j) {
-            const double t = slot.top() + cost[j];
-            slot.pop();
-            slot.push(t);
-            worst = std::max(worst, t);
-          }
-        }
-  }
-  return worst;
-}
-
-// Cost of a narrow block relative to a wide one: single blocks timed over the same 32768 keys (3 and
-// 2 column blocks), and estimated from the instruction counts (2 and 1).
-constexpr double kNarrowCost = 0.79, kNarrowCostFine = 0.62;
-// Key parts: a block's fixed cost (first loads, page ids, the output) and the merge launch, in tile
-// times of a wide block (1.16 us), the bytes of partials merged per tile time (read at 4 TB/s and
-// half of them again for the blocks' stores), and the fewest tiles a part is worth a block for.
-constexpr double kStartTiles = 5.0, kMergeTiles = 4.0, kMergeBytesPerTile = 3.1e6;
-constexpr int kMinPartTiles = 12, kMaxParts = 16;
-
-// A launch: pairs of (sequence, KV group) whose longest chunk has max_cols columns (query, head), blocks
-// of w2 / w3 columns, tables of `tiles` key tiles.
-struct PlanShape {
-  int64_t max_cols, pairs, part_row_bytes;  // part_row_bytes: one part's partials of the whole call
-  int w2, w3, n_rep, slots_per_xcd, tiles;
-  double narrow;
-  bool allow_parts;
-};
-
-BlockPlan choose_plan(const PlanShape& f) {
-  const int n3_max = (int)((f.max_cols + f.w3 - 1) / f.w3);
-  BlockPlan best{n3_max, 0, 1, std::max(1, f.tiles), n3_max, 0};
-  // Large launches run many rounds, where the last one matters little: keep wide blocks.
-  if (f.pairs * n3_max > (1 << 16) || f.slots_per_xcd <= 0 || n3_max == 0) return best;
-  // Parts are considered for launches of few blocks: there whole blocks leave CUs idle.
-  const bool parts_ok = f.allow_parts && f.tiles >= 2 * kMinPartTiles && f.pairs * n3_max < 16 * f.slots_per_xcd;
-  static std::mutex mu;
-  static std::map<std::tuple<int64_t, int64_t, int64_t, int, int, int, int>, BlockPlan> cache;
-  const auto key = std::make_tuple(f.max_cols, f.pairs, parts_ok ? f.part_row_bytes : 0, f.w2, f.n_rep, f.slots_per_xcd,
-                                   parts_ok ? f.tiles : 0);
-  std::lock_guard<std::mutex> lock(mu);
-  const auto hit = cache.find(key);
-  if (hit != cache.end()) return hit->second;
-  auto narrow_blocks = [&](int n3) { return (int)((f.max_cols - (int64_t)n3 * f.w3 + f.w2 - 1) / f.w2); };
-  std::vector<double> cost;
-  // Every block as streaming equally many keys (a long prefix).
-  auto flat = [&](int n3, int n2) {
-    cost.assign(n3, 1.0);
-    cost.insert(cost.end(), n2, f.narrow);
-    return plan_makespan(f.pairs, cost, n3, f.slots_per_xcd);
-  };
-  double best_t = flat(n3_max, 0);
-  // Each wide block traded for narrow ones adds work: a dozen trades fill any last round.
-  for (int n3 = n3_max - 1; n3 >= std::max(0, n3_max - 12); --n3) {
-    const int n2 = narrow_blocks(n3);
-    const double t = flat(n3, n2);
-    if (t < best_t - 1e-9) {
-      best_t = t;
-      best.n3 = n3;
-      best.n2 = n2;
-    }
-  }
-  best.whole3 = best.n3;
-  best.whole2 = best.n2;
-  if (parts_ok) {
-    // In tile times, each block as streaming the keys up to its last query's own.
-    auto causal = [&](int n3, int n2, int parts) {
-      cost.assign((size_t)(n3 + n2) * parts, 0.0);
-      for (int j = 0; j < n3 + n2; ++j) {
-        const int64_t after = j < n3 ? (int64_t)f.w3 * j : (int64_t)f.w3 * n3 + (int64_t)f.w2 * (j - n3);
-        const int seen = std::max<int64_t>(1, f.tiles - after / f.n_rep / kTileKeys);
-        for (int s = 0; s < parts; ++s) {
-          const int t0 = (int)((int64_t)s * f.tiles / parts), t1 = (int)((int64_t)(s + 1) * f.tiles / parts);
-          const double c = seen > t0 ? kStartTiles + (std::min(seen, t1) - t0) * (j < n3 ? 1.0 : f.narrow) : 0.3;
-          cost[j < n3 ? (size_t)s * n3 + j : (size_t)parts * n3 + (size_t)s * n2 + (j - n3)] = c;
-        }
-      }
-      return plan_makespan(f.pairs, cost, n3 * parts, f.slots_per_xcd);
-    };
-    best_t = causal(best.n3, best.n2, 1);
-    const int max_parts = std::min(kMaxParts, f.tiles / kMinPartTiles);
-    for (int parts = 2; parts <= max_parts; ++parts) {
-      const double merge = kMergeTiles + parts * (double)f.part_row_bytes / kMergeBytesPerTile;
-      for (int n3 = n3_max; n3 >= std::max(0, n3_max - 2); --n3) {
-        const int n2 = n3 == n3_max ? 0 : narrow_blocks(n3);
-        const double t = merge + causal(n3, n2, parts);
-        if (t < 0.97 * best_t) {
-          best_t = t;
-          best = BlockPlan{n3, n2, parts, (f.tiles + parts - 1) / parts, best.whole3, best.whole2};
-        }
-      }
-    }
-  }
-  if (cache.size() >= 4096) cache.clear();  // a caller cycling through many shapes recomputes
-  cache.emplace(key, best);
-  return best;
-}
 
 // CUs per XCD of the current device (8 XCDs), 0 when unknown.
 int cus_per_xcd() {
