@@ -156,12 +156,26 @@ def test_parts_replay_from_a_captured_graph(cuda):
         prefill.paged_prefill_attention(*args, **kw)
 
 
-def test_parts_are_taken_only_by_launches_short_of_blocks():
-    """The plan on the CPU (no device: 256 CUs are not known, so nothing is cut)."""
+def test_no_scratch_for_shapes_without_a_tiled_instance():
     lib = _ext.load()
     assert lib.ukv_paged_prefill_workspace_bytes(0, 1, 1, 8, 2, 128, 4, 100) == 0
-    assert lib.ukv_paged_prefill_workspace_bytes(1, 64, 64, 8, 2, 96, 4, 1000) == 0  # no tiled instance
-    assert lib.ukv_paged_prefill_workspace_bytes(64, 64 * 2048, 2048, 32, 8, 128, 4, 1000) == 0
+    assert lib.ukv_paged_prefill_workspace_bytes(1, 64, 64, 8, 2, 96, 4, 1000) == 0
+
+
+@pytest.mark.gpu
+def test_parts_are_taken_only_by_launches_short_of_blocks(cuda):
+    """Without a device no shape is cut, so the rule is asked here: 16 blocks a slot (256 CUs, one slot each) and
+    more stay whole whatever their keys, launches of few blocks are cut."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    size = _ext.load().ukv_paged_prefill_workspace_bytes
+
+    def cut(batch, queries, pages):  # 32/8 heads of 128 dims: blocks of 96 queries
+        return size(batch, batch * queries, queries, 32, 8, 128, 4, pages) > 0
+
+    assert not cut(64, 2048, 1000)
+    assert not cut(8, 768, 2048)  # 64 pairs of 8 blocks: 512, an XCD's 16 * 32
+    assert cut(1, 512, 2048) and cut(1, 96, 100)
+    assert not cut(1, 512, 46)  # 23 key tiles: no two parts of 12
 
 
 @pytest.mark.gpu
