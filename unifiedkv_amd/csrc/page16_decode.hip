@@ -74,19 +74,6 @@ __device__ __forceinline__ int clamp_len(int L, int max_blocks) {
 
 __device__ __forceinline__ int pages_of(int len, int max_blocks) { return (clamp_len(len, max_blocks) + 15) >> 4; }
 
-// Inclusive prefix sum over the wave's 64 lanes, in registers: DPP row shifts inside each 16-lane
-// row, then the rows' totals broadcast onwards (0x111 + n - 1 = row_shr:n, 0x142 / 0x143 =
-// row_bcast:15 / :31). Six dependent VALU adds; six cross-lane LDS permutes took ~0.3 us here.
-__device__ __forceinline__ int wave_inclusive_scan_i32(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
-  return x;
-}
-
 // floor(x * y / z) for 0 <= x, y and 0 < z: one 32-bit division where the product fits.
 __device__ __forceinline__ int mul_div(int x, int y, int z) {
   const uint64_t p = (uint64_t)(uint32_t)x * (uint32_t)y;
@@ -110,8 +97,13 @@ __device__ __forceinline__ int wave_max_i32(int x) {
 // longest sequence ~0.05 us in the merge, so a share takes about sqrt(longest) / 4 pages. One sequence
 // of 4096 tokens beside three of 17: 16.8 us with 72 shares, 23.9 with 256, 21.2 with 32; four of 128
 // pages keep their 128 shares. A multiple of 8 (G too, or it is taken whole) for the XCDs' equal runs.
-__device__ __forceinline__ int shares_for(const DecodeArgs& a, int P, int longest) {
-  if (a.fixed_shares) return a.grid_wgs;
+// With P >= G^2 / 16 + 2 G the rule gives G whatever the longest (a share takes at most
+// sqrt(P) / 4 + 1/2 pages), and neither it nor the square root is waited for.
+template <class F>
+__device__ __forceinline__ int shares_for(const DecodeArgs& a, int P, F longest_pages) {
+  const int many = (int)min((int64_t)INT32_MAX, (int64_t)a.grid_wgs * (a.grid_wgs + 32) / 16 + 1);
+  if (a.fixed_shares || P >= many) return a.grid_wgs;
+  const int longest = longest_pages();
   // (the square root is vector code: its result back to a scalar register, with all that follows from it; three
   // more vector registers would leave the 64-dim split one workgroup to a CU)
   const int per = max(1, __builtin_amdgcn_readfirstlane((int)(0.25f * __builtin_sqrtf((float)longest) + 0.5f)));
@@ -289,7 +281,7 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
     const int incl = wave_inclusive_scan_i32(n);
     P = __builtin_amdgcn_readlane(incl, 63);
     nonempty = __ballot(n > 0);
-    G = shares_for(a, P, wave_max_i32(n));
+    G = shares_for(a, P, [&]() { return wave_max_i32(n); });
     if (writer && lane < a.B) {
       a.seq_start[lane] = lane == 0 ? G : incl - n;
       a.seq_pages[lane] = n;
@@ -309,7 +301,7 @@ __global__ void __launch_bounds__(64 * UKV_PAGE16_WAVES, UKV_PAGE16_MIN_WAVES_PE
       P += __builtin_amdgcn_readlane(wave_inclusive_scan_i32(n), 63);
       longest = max(longest, wave_max_i32(n));
     }
-    G = shares_for(a, P, longest);
+    G = shares_for(a, P, [&]() { return longest; });
     if ((int)blockIdx.x >= G) return;
     w = share_of_workgroup();
     x0 = mul_div(w, P, G);
