@@ -281,8 +281,9 @@ template <> struct PrefillSplit<UKV_DTYPE_F16> {
 //          lie in one column block) and P and V are fp16.
 //   PARTS  part `part` of the sequence's keys (of np = part_count()), left for
 //          prefill_combine_kernel; a sequence in one part is written like an undivided one (every row
-//          through the partials cost 4 x 512-token prompts in a 2048-page table 53 us against 29). The running max moves to whole powers of two, so that the
-//          parts' rounded weights are the ones an undivided pass would have summed.
+//          through the partials cost 4 x 512-token prompts in a 2048-page table 53 us against 29). The
+//          running max moves to whole powers of two, so that the parts' rounded weights are the ones an
+//          undivided pass would have summed.
 // With statistics (obs > 0) it also writes, for each of the sequence's last obs queries in the
 // block and each q head h, the pair (m, l) of the column's running max m (log2 units) and its
 // softmax denominator l (the sum of the rounded weights 2^(s * scale * log2e - m) over every key the
@@ -890,9 +891,10 @@ __device__ __forceinline__ bool locate_item(int start, int end, int n, int nl, i
 }
 
 // Column blocks per wave of the wide query blocks (the narrow ones have one fewer): the widest whose
-// accumulators, queries and weights stay in 256 VGPRs, and in 128 at D = 64, where two workgroups
+// accumulators, queries and weights (in two parts for FINE) stay in 256 VGPRs. 64-dim heads are FINE, and
+// two blocks of theirs fit the 128 VGPRs that paged_prefill_kernel asks for at D = 64: two workgroups
 // then share a CU and cover each other's first loads (one 96-token prompt 7.5 us against 11.6).
-constexpr int wide_blocks(bool fine, int d) { return fine ? 2 : 3; }
+constexpr int wide_blocks(bool fine) { return fine ? 2 : 3; }
 
 // The range of work items [start, end) of a launch's n_items items that XCD xcd runs: dispatch
 // is round-robin over the 8 XCDs, so the workgroups with blockIdx.x % 8 == xcd run there, and
@@ -921,7 +923,7 @@ template <int DT, int D, int WAVES, bool FINE, bool PARTS>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 paged_prefill_kernel(const PrefillArgs a) {
   __shared__ PrefillLds<D> lds;
-  constexpr int CB3 = wide_blocks(FINE, D), CB2 = CB3 - 1;
+  constexpr int CB3 = wide_blocks(FINE), CB2 = CB3 - 1;
   int n3 = a.n3, n2 = a.n2;
   int start, end, pair, j, part = 0, np = 1;
   if (!PARTS && a.by_block) {
@@ -1354,7 +1356,7 @@ bool fine_shape(int head_dim, int n_rep) { return head_dim != 128 || 16 % n_rep 
 BlockPlan plan_for(int batch, int64_t rows, int max_chunk, int n_groups, int head_dim, int n_rep, int max_blocks,
                    bool parts) {
   constexpr int W = UKV_PREFILL_WAVES, tile_pages = kTileKeys / 16;
-  const int cb3 = wide_blocks(fine_shape(head_dim, n_rep), head_dim);
+  const int cb3 = wide_blocks(fine_shape(head_dim, n_rep));
   PlanShape f{};
   f.max_cols = (int64_t)max_chunk * n_rep;
   f.pairs = (int64_t)n_groups * batch;
@@ -1370,7 +1372,9 @@ BlockPlan plan_for(int batch, int64_t rows, int max_chunk, int n_groups, int hea
 }
 
 size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
-size_t part_o_bytes(int parts, int64_t rows, int head_dim) { return up256((size_t)parts * rows * head_dim * sizeof(float)); }
+size_t part_o_bytes(int parts, int64_t rows, int head_dim) {
+  return up256((size_t)parts * rows * head_dim * sizeof(float));
+}
 size_t part_bytes(int parts, int64_t rows, int head_dim) {
   return part_o_bytes(parts, rows, head_dim) + up256((size_t)parts * rows * sizeof(float2));
 }
@@ -1473,7 +1477,8 @@ int prefill_impl(const void* q, const void* k_cache, const void* v_cache, const 
   const bool strides_ok = mul8(a.q_st) && mul8(a.q_sh) && mul8(a.k_sp) && mul8(a.k_st) && mul8(a.k_sh) &&
                           mul8(a.v_sp) && mul8(a.v_st) && mul8(a.v_sh) && in_page_ok(a.k_st, a.k_sh) &&
                           in_page_ok(a.v_st, a.v_sh) && page_stride_ok(a.k_sp) && page_stride_ok(a.v_sp);
-  const bool fast = tiled_shape(head_dim, n_rep) && softmax_scale > 0.f && std::isfinite(softmax_scale) && strides_ok && al16(q) && al16(out) && al16(k_cache) && al16(v_cache) && max_blocks > 0;
+  const bool fast = tiled_shape(head_dim, n_rep) && softmax_scale > 0.f && std::isfinite(softmax_scale) && strides_ok &&
+                    al16(q) && al16(out) && al16(k_cache) && al16(v_cache) && max_blocks > 0;
   if (obs) {
     a.obs_stats = static_cast<float2*>(obs->stats);
     a.stats_seq_stride = obs->seq_stride;

@@ -26,17 +26,6 @@ __device__ __forceinline__ uint32_t select_key(float s) {
   return ~ord;
 }
 
-// Inclusive prefix sum over the wave (DPP row shifts, then the rows' totals broadcast onwards).
-__device__ __forceinline__ int wave_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
-  return x;
-}
-
 __device__ __forceinline__ int lanes_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
 }
@@ -117,7 +106,7 @@ __global__ void __launch_bounds__(NT) select_topk_kernel(const float* __restrict
       hist[tid * PER + j] = 0;
       sum += c[j];
     }
-    const int incl = wave_scan(sum);
+    const int incl = wave_inclusive_scan_i32(sum);
     if (lane == 63) wave_sum[wv] = incl;
     __syncthreads();
     int before = incl - sum;

@@ -658,7 +658,8 @@ void lay_out(SnapPlan& p, int items, int rows_all) {
   p.part_off = 0;
   p.stats_off = a256((size_t)items * p.S * rows_all * sizeof(float2));
   p.raw_off = p.stats_off + a256((size_t)items * rows_all * sizeof(float2));
-  p.redo_off = p.raw_off + a256((size_t)items * (p.groups > 1 ? (size_t)p.groups * p.aligned : p.n_blocks) * sizeof(float));
+  const size_t raw_item = p.groups > 1 ? (size_t)p.groups * p.aligned : p.n_blocks;
+  p.redo_off = p.raw_off + a256((size_t)items * raw_item * sizeof(float));
   p.total = p.redo_off + a256((size_t)items * sizeof(int32_t));
 }
 
@@ -729,7 +730,8 @@ SnapPlan snap_plan(int items, int seq_len, int sink, int obs, int num_q_heads, i
   p.S = p.groups = 1;
   const int rows_all = num_q_heads * obs;
   if (p.tiled)
-    choose_ranges(p, items, rows_all, num_q_heads / n_rep * p.parts, snap_cu_count(), head_dim == 64 && p.tw <= 2, budget);
+    choose_ranges(p, items, rows_all, num_q_heads / n_rep * p.parts, snap_cu_count(), head_dim == 64 && p.tw <= 2,
+                  budget);
   lay_out(p, items, rows_all);
   return p;
 }
@@ -833,7 +835,8 @@ int snapkv_scores_impl(const void* q_obs, const int64_t* q_strides, const void* 
   if (p.total > workspace_bytes)  // fewer ranges or unit groups, if that fits (a buffer sized for longer sequences does)
     p = snap_plan(items, seq_len, sink_len, obs_len, num_q_heads, n_rep, head_dim, block_size, aligned_rows,
                   workspace_bytes);
-  if (!workspace || workspace_bytes < p.total || (reinterpret_cast<uintptr_t>(workspace) & 15u)) return UKV_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < p.total || (reinterpret_cast<uintptr_t>(workspace) & 15u))
+    return UKV_ERR_WORKSPACE;
 
   SnapArgs a{};
   a.q = static_cast<const uint16_t*>(q_obs);

@@ -103,6 +103,19 @@ __device__ __forceinline__ float row_sum16(float x) {
   return x;
 }
 
+// Inclusive prefix sum over the wave's 64 lanes, in registers: DPP row shifts inside each 16-lane
+// row, then the rows' totals broadcast onwards (0x111 + n - 1 = row_shr:n, 0x142 / 0x143 =
+// row_bcast:15 / :31). Six dependent VALU adds; six cross-lane LDS permutes took ~0.3 us in the decode.
+__device__ __forceinline__ int wave_inclusive_scan_i32(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *reinterpret_cast<const u32x4*>(p); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
