@@ -267,3 +267,42 @@ def test_sequences_in_one_part_beside_sequences_in_many(cuda, n_rep, Hkv, D):
     got = out.float().cpu().numpy()
     _close(got[:370], want[:370], _v_max(case), "bf16", tol, "the others")
     assert np.isnan(got[370:381]).all() and np.isfinite(got[381:]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("long_at", [0, 63, 64, 69, None])
+def test_many_sequences_of_which_one_or_none_is_in_parts(cuda, long_at):
+    """Seventy sequences in a wide table: each workgroup looks through all lengths, 64 at a time, for one in parts."""
+    prefix = [3 * (i % 5) for i in range(70)]
+    if long_at is not None:
+        prefix[long_at] = 3000
+    chunk = [1 + i % 4 for i in range(70)]
+    case = _wide(make_case(70, prefix, chunk, Hq=4, Hkv=1, D=128, dtype="bf16"), 256)
+    out, ws = _parts_call(case, cuda, 7.0)
+    _close(out.float().cpu().numpy(), expected(case), _v_max(case), "bf16", 2.0 ** -11, f"long at {long_at}")
+    assert bool((ws != 0xFF).any()) == (long_at is not None)
+
+
+@pytest.mark.gpu
+def test_lengths_the_host_knows_leave_a_wide_table_uncut(cuda):
+    """The call in a table of 2048 pages is the one in a table of the sequences' own pages, bit for bit."""
+    from unifiedkv_amd import prefill
+
+    case = make_case(5, [0, 40], [300, 257], Hq=16, Hkv=4, D=128, dtype="bf16")
+    wide = _wide(case, 2048)
+    assert _parts_bytes(wide) > 0 and _parts_bytes(case) == 0
+    t, w = to_dev(case, cuda), to_dev(wide, cuda)
+    prefill.write_chunk_kv(t["k_cache"], t["v_cache"], t["k_new"], t["v_new"], t["block_table"], t["cu"], t["kv_lens"],
+                           300)
+    kw = dict(softmax_scale=case["scale"], n_rep=4, max_chunk=300)
+    args = (t["q"], t["k_cache"], t["v_cache"])
+    want = prefill.paged_prefill_attention(*args, t["block_table"], t["cu"], t["kv_lens"], **kw)
+    lens = [int(x) for x in case["kv_lens"]]
+    for got in (prefill.paged_prefill_attention(*args, w["block_table"], t["cu"], lens, **kw),
+                prefill.paged_prefill_attention(*args, w["block_table"], t["cu"], t["kv_lens"].cpu(), **kw),
+                prefill.paged_prefill_attention(*args, w["block_table"], t["cu"], t["kv_lens"],
+                                                host_lens=([300, 257], lens), **kw)):
+        assert torch.equal(got, want)
+    got = prefill.paged_prefill_attention(*args, w["block_table"], t["cu"], t["kv_lens"], host_lens=([300, 257], None),
+                                          **kw)  # (not known after all)
+    torch.testing.assert_close(got.float(), want.float(), atol=2e-2, rtol=2e-2)

@@ -108,6 +108,16 @@ struct PrefillArgs {
   int sink, obs;
 };
 
+// paged_prefill_kernel's argument (its only one, at the start of the kernel's argument segment), read again
+// behind a barrier to the compiler: the fields that only a block's rows need at the end would otherwise be loaded
+// at the start and held through the tiles, where the scalar registers they spill cost a v_readlane each (16 a tile in
+// the parts' instance for three column blocks, 150 instructions of it against 128).
+__device__ __forceinline__ const PrefillArgs& args_again() {
+  auto* p = (const __attribute__((address_space(4))) PrefillArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const PrefillArgs*)p;
+}
+
 __device__ __forceinline__ int kv_len_of(const PrefillArgs& a, int b) {
   const int cap = a.max_blocks * 16;
   const int L = a.kv_lens[b];
@@ -167,6 +177,18 @@ constexpr int kStages = 4;  // K/V ring slots: tiles are written two ahead, a ba
 // [s * n_tiles / n, (s + 1) * n_tiles / n).
 __device__ __forceinline__ int part_count(const PrefillArgs& a, int n_tiles) {
   return max(1, min(a.n_parts, (n_tiles + a.part_tiles - 1) / a.part_tiles));
+}
+
+// Whether any sequence is in more parts than one: the plan knows the table's width alone. (Wave-uniform. The first
+// rows are loaded beside the lengths for the reads that follow: first rows are not negative.)
+__device__ __forceinline__ bool any_in_parts(const PrefillArgs& a) {
+  const int most = a.part_tiles * kTileKeys;  // keys of a sequence in one part
+  bool any = false;
+  for (int b0 = 0; b0 < a.B && !any; b0 += 64) {
+    const int b = min(b0 + (int)(threadIdx.x & 63), a.B - 1);
+    any = __any(kv_len_of(a, b) > most || a.cu_q[b + 1] < 0);
+  }
+  return any;
 }
 
 // Fallback for a workgroup whose keys hold a V the matrix cores' P.V would get wrong (a bf16 V of
@@ -335,9 +357,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     const int nt = (Lk + TK - 1) / TK;
     if (part >= np) return;  // whole workgroup
     in_parts = np > 1;
-    key_a = (int)((int64_t)part * nt / np) * TK;
+    key_a = (int)((uint32_t)(part * nt) / (uint32_t)np) * TK;  // (at most kMaxParts * 2^26: 32 bits)
     if (in_parts && key_a >= kend) return;  // no row of the block sees this part (prefill_combine_kernel skips it)
-    kend = min(kend, (int)((int64_t)(part + 1) * nt / np) * TK) - key_a;
+    kend = min(kend, (int)((uint32_t)((part + 1) * nt) / (uint32_t)np) * TK) - key_a;
     Lk -= key_a;
     P0 -= key_a;
   }
@@ -692,6 +714,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
     vm_wait<0>(rv1);
   }
 
+  const PrefillArgs& e = PARTS ? args_again() : a;
   // A V the matrix cores got wrong anywhere in this workgroup's keys: its columns again on the fp32
   // fallback.
   bool redo_mine = false;
@@ -707,55 +730,48 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, const int b, 
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-      for (int e = 0; e < NE; ++e)
+      for (int d = 0; d < NE; ++d)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z = __builtin_fmaf(o[cb][e][r], 0.f, z);
+        for (int r = 0; r < 4; ++r) z = __builtin_fmaf(o[cb][d][r], 0.f, z);
     redo_mine = z != 0.f;
   }
   if constexpr (kConvert || FINE) {
     if (__syncthreads_or(redo_mine)) {
-      if (!in_parts) flag_obs_rows<WAVES>(a, b, g, C, max(q0, 0), min(C, q1));  // (none without statistics)
-      prefill_cols_fp32<DT, D>(a, b, g, q_begin, C, P0 + key_a, Lk + key_a, c0, WAVES * CB * 16, wv, WAVES, lane,
+      if (!in_parts) flag_obs_rows<WAVES>(e, b, g, C, max(q0, 0), min(C, q1));  // (none without statistics)
+      prefill_cols_fp32<DT, D>(e, b, g, q_begin, C, P0 + key_a, Lk + key_a, c0, WAVES * CB * 16, wv, WAVES, lane,
                                in_parts ? part : -1, key_a, key_a + kend);
       return;
     }
   }
 
-  // out[column] = o / l: lane (i16, kg) holds dims 16e + i16 of columns 4*kg + r,
+  // out[column] = o / l: lane (i16, kg) holds dims 16d + i16 of columns 4*kg + r,
   // and lacc[cb][r] is the denominator of column 4*kg + r (the same in its 16 lanes).
   if (!wave_live) return;
-  if constexpr (PARTS) {
-    // Found again, behind a barrier to the compiler, so that nothing of it is held through the tiles: a launch of
-    // one round 209.4 us against 210.4 (207.7 with every sequence in parts).
-    int seq = b;
-    asm volatile("" : "+s"(seq));
-    in_parts = part_count(a, (kv_len_of(a, seq) + TK - 1) / TK) > 1;
-  }
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int col = 4 * kg + r;
-      const int qi = FINE ? col_query(cb * 16 + col) : wq0 + cb * qpb + col / a.n_rep;
-      const int hh = FINE ? col_head(cb * 16 + col) : g * a.n_rep + col % a.n_rep;
+      const int qi = FINE ? col_query(cb * 16 + col) : wq0 + cb * qpb + col / e.n_rep;
+      const int hh = FINE ? col_head(cb * 16 + col) : g * e.n_rep + col % e.n_rep;
       // the column's running max, held by lane col (column i16 = col)
       const float m_col = __shfl(m_ref[cb], col);
-      if (qi >= 0 && qi < C && hh < a.Hq) {
+      if (qi >= 0 && qi < C && hh < e.Hq) {
         if (PARTS && in_parts) {
           // (FINE's lift by 2^kLift is in o and l alike: taken off the max)
-          const int64_t row = ((int64_t)part * a.total_q + q_begin + qi) * a.Hq + hh;
-          float* prow = a.part_o + row * D + i16;
+          const int64_t row = ((int64_t)part * e.total_q + q_begin + qi) * e.Hq + hh;
+          float* prow = e.part_o + row * D + i16;
 #pragma unroll
-          for (int e = 0; e < NE; ++e) prow[16 * e] = o[cb][e][r];
-          if (i16 == 0) a.part_ml[row] = make_float2(m_col - kLift, lacc[cb][r]);
+          for (int d = 0; d < NE; ++d) prow[16 * d] = o[cb][d][r];
+          if (i16 == 0) e.part_ml[row] = make_float2(m_col - kLift, lacc[cb][r]);
           continue;
         }
         const float inv = 1.f / lacc[cb][r];
-        uint16_t* orow = a.out + ((int64_t)(q_begin + qi) * a.Hq + hh) * D + i16;
+        uint16_t* orow = e.out + ((int64_t)(q_begin + qi) * e.Hq + hh) * D + i16;
 #pragma unroll
-        for (int e = 0; e < NE; ++e) orow[16 * e] = Elem<DT>::from_float(o[cb][e][r] * inv);
-        if (i16 == 0 && qi >= C - a.obs)  // (never without statistics: obs = 0)
-          a.obs_stats[(int64_t)b * a.stats_seq_stride + (int64_t)hh * a.obs + (qi - (C - a.obs))] =
+        for (int d = 0; d < NE; ++d) orow[16 * d] = Elem<DT>::from_float(o[cb][d][r] * inv);
+        if (i16 == 0 && qi >= C - e.obs)  // (never without statistics: obs = 0)
+          e.obs_stats[(int64_t)b * e.stats_seq_stride + (int64_t)hh * e.obs + (qi - (C - e.obs))] =
               make_float2(m_col - kLift, lacc[cb][r]);
       }
     }
@@ -825,17 +841,11 @@ __device__ __forceinline__ void prefill_combine_row(const PrefillArgs& a, const 
 template <int DT, int D>
 __global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillArgs a) {
   constexpr int LANES = D / 4, ROWS = 256 / LANES;
-  constexpr int TK = kTileKeys;
   const int64_t rows = (int64_t)a.total_q * a.Hq, step = (int64_t)gridDim.x * ROWS;
   if (step < rows) {
     // Several rows a group: a table wider than its sequences may leave nothing to merge, which is then found
     // once, by every wave.
-    bool any = false;
-    for (int b0 = 0; b0 < a.B && !any; b0 += 64) {
-      const int b = b0 + (threadIdx.x & 63);
-      any = __any(b < a.B && part_count(a, (kv_len_of(a, min(b, a.B - 1)) + TK - 1) / TK) > 1);
-    }
-    if (!any) return;
+    if (!any_in_parts(a)) return;
   }
   const int dq = threadIdx.x % LANES;
   for (int64_t idx = (int64_t)blockIdx.x * ROWS + threadIdx.x / LANES; idx < rows; idx += step)
@@ -918,7 +928,10 @@ __device__ __forceinline__ void xcd_range(int total, int xcd, int& start, int& e
 // to each other, and where the table is wider than the sequences the workgroups without keys come last.
 // (Workgroups that exit at once among those that work, for the larger of two block counts, doubled launches
 // of one round: an XCD's shader engines take workgroups in turn, whatever they hold. So did the same four of 28
-// items a part on an XCD of 32 slots, nine times.)
+// items a part on an XCD of 32 slots, nine times.) Where no sequence is in parts the launch runs as one without
+// parts, its workgroups past the items exiting at the end: 8 x 512 queries behind 4000 tokens in a 2048-page
+// table 292 us, 380 in the order of parts, 284 in a launch without parts. Looking for one costs a launch
+// in parts a round of loads, ~1.3 us.
 template <int DT, int D, int WAVES, bool FINE, bool PARTS>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 paged_prefill_kernel(const PrefillArgs a) {
@@ -926,6 +939,11 @@ paged_prefill_kernel(const PrefillArgs a) {
   constexpr int CB3 = wide_blocks(FINE), CB2 = CB3 - 1;
   int n3 = a.n3, n2 = a.n2;
   int start, end, pair, j, part = 0, np = 1;
+  const bool parts = PARTS && any_in_parts(a);
+  if (PARTS && !parts) {
+    n3 = a.whole3;
+    n2 = a.whole2;
+  }
   if (!PARTS && a.by_block) {
     const int pairs = a.n_groups * a.B;
     j = blockIdx.x / pairs;
@@ -934,7 +952,7 @@ paged_prefill_kernel(const PrefillArgs a) {
     const int n = n3 + n2;
     const int total = n * a.n_groups * a.B, xcd = blockIdx.x & 7;
     int s = blockIdx.x >> 3, range = xcd;
-    if constexpr (PARTS) {
+    if (parts) {
       // One range for every part; the total & 7 ranges with an item more go round the XCDs. An XCD had
       // floor((xcd + (p - 1) rem) / 8) + (xcd < rem) of those in parts 0 .. p - 1.
       const int per = total >> 3, rem = total & 7, first = xcd < rem ? 1 : 0;
@@ -946,11 +964,11 @@ paged_prefill_kernel(const PrefillArgs a) {
       range = (xcd + part * rem) & 7;
     }
     xcd_range(total, range, start, end);
-    if (!locate_item(start, end, n, n3, s, pair, j)) return;  // (never)
+    if (!locate_item(start, end, n, n3, s, pair, j)) return;  // (only where no sequence is in parts)
   }
   const int g = pair % a.n_groups, b = pair / a.n_groups;
   const int C = a.cu_q[b + 1] - a.cu_q[b];
-  if constexpr (PARTS) {
+  if (parts) {
     np = part_count(a, (kv_len_of(a, b) + kTileKeys - 1) / kTileKeys);
     if (np == 1) {
       j += part * (n3 + n2);  // its blocks in the items of every part
