@@ -98,6 +98,14 @@ def _host_ints(x):
     return [int(v) for v in (x.tolist() if torch.is_tensor(x) else x)]
 
 
+def _longest_pages(kv_lens, host_lens):
+    """Pages of the longest sequence where the host knows the lengths, else None."""
+    lens = kv_lens if host_lens is None else host_lens[1]
+    if lens is None or (torch.is_tensor(lens) and lens.device.type != "cpu"):
+        return None
+    return -(-max(_host_ints(lens), default=0) // 16)
+
+
 def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                             block_table: torch.Tensor, cu_seqlens_q, kv_lens, *, softmax_scale: float, n_rep: int,
                             max_chunk: Optional[int] = None, obs_stats: Optional[ObsStats] = None,
@@ -161,7 +169,15 @@ def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
             _DTYPE_CODES[q.dtype]]
     lib = _ext.load()
     # The parts' scratch comes from the caching allocator, which keeps it for this stream's kernels.
-    need = lib.ukv_paged_prefill_workspace_bytes(B, total_q, mc, Hq, Hkv, D, int(n_rep), int(bt.shape[1]))
+    width = int(bt.shape[1])
+    need = lib.ukv_paged_prefill_workspace_bytes(B, total_q, mc, Hq, Hkv, D, int(n_rep), width)
+    if need:
+        # The plan knows the table's width alone; where the host knows the lengths and they would not be cut in a
+        # table of their own, a call without scratch saves the merge's launch.
+        pages = _longest_pages(kv_lens, host_lens)
+        if pages is not None and pages < width and not lib.ukv_paged_prefill_workspace_bytes(
+                B, total_q, mc, Hq, Hkv, D, int(n_rep), pages):
+            need = 0
     ws = None
     if need:
         try:
