@@ -235,7 +235,11 @@ inline BlockPlan compute_plan(const PlanShape& f, bool parts_ok) {
     }
   };
   for (int n3 = n3_max; n3 >= std::max(0, n3_max - 2); --n3) add(n3, n3 == n3_max ? 0 : narrow_blocks(n3));
-  if (best.n3 < n3_max - 2) add(best.n3, best.n2);
+  // (Not where the chunk holds half of the keys or more: its later blocks see the first parts alone, and the
+  // workgroups that exit in their place leave shader engines idle, which take workgroups in turn. One 2048-token
+  // prompt on 16 heads without GQA in three parts: 54 us with wide blocks, 65 with eight narrow ones.)
+  const int64_t chunk_tiles = f.max_cols / f.n_rep / kTileKeys;
+  if (best.n3 < n3_max - 2 && 2 * chunk_tiles <= f.tiles) add(best.n3, best.n2);
   std::sort(c.begin(), c.begin() + n, [](const Candidate& a, const Candidate& b) { return a.bound < b.bound; });
   best_t = 0.97 * whole;
   int64_t steps = kMaxPlanSteps;
