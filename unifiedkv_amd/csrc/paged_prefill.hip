@@ -183,6 +183,7 @@ __device__ __forceinline__ int part_count(const PrefillArgs& a, int n_tiles) {
 // rows are loaded beside the lengths for the reads that follow: first rows are not negative.)
 __device__ __forceinline__ bool any_in_parts(const PrefillArgs& a) {
   const int most = a.part_tiles * kTileKeys;  // keys of a sequence in one part
+  if (a.B == 1) return kv_len_of(a, 0) > most;  // (scalar loads)
   bool any = false;
   for (int b0 = 0; b0 < a.B && !any; b0 += 64) {
     const int b = min(b0 + (int)(threadIdx.x & 63), a.B - 1);
@@ -931,7 +932,7 @@ __device__ __forceinline__ void xcd_range(int total, int xcd, int& start, int& e
 // items a part on an XCD of 32 slots, nine times.) Where no sequence is in parts the launch runs as one without
 // parts, its workgroups past the items exiting at the end: 8 x 512 queries behind 4000 tokens in a 2048-page
 // table 292 us, 380 in the order of parts, 284 in a launch without parts. Looking for one costs a launch
-// in parts a round of loads, ~1.3 us.
+// in parts of several sequences a round of loads, ~1.3 us.
 template <int DT, int D, int WAVES, bool FINE, bool PARTS>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 paged_prefill_kernel(const PrefillArgs a) {
