@@ -196,3 +196,12 @@ def test_closed_form_of_whole_blocks(lib):
         n3, n2 = rng.randint(0, 9), rng.randint(0, 14)
         if n3 + n2:
             assert abs(lib.flat_error(rng.randint(1, 200), n3, n2, rng.choice([0.79, 0.62]), rng.choice([32, 64]))) < 1e-9
+
+
+def test_whole_mix_is_cut_only_behind_a_prefix(lib):
+    """Narrow blocks alone, the mix of whole blocks here, are a candidate for parts where the chunk holds at most half
+    of the keys; a prompt without a prefix keeps wide blocks."""
+    n3, n2, parts, _, whole3, whole2 = _plan(lib, _shape(2, 2 * 512 * 32, 512, 8, 128, 4, 1024))
+    assert parts > 1 and (n3, n2) == (whole3, whole2) == (0, 8)
+    n3, _, parts, _, whole3, _ = _plan(lib, _shape(1, 2048 * 16, 2048, 16, 128, 1, 128))
+    assert parts > 1 and whole3 == 0 and n3 >= 4  # of six
